@@ -214,6 +214,15 @@ struct cpg_handle {
   DevBuf<int2> devinfo, lift;
   DevBuf<SfxtCtl> sctl;
   DevBuf<unsigned long long> dfw;  // dataflow loop: one progress word per block
+  // The resident graph's level-order schedule: laid out by the second SFXT
+  // on the graph from the first one's level order (queue, level, lvlp), kept
+  // until the graph or its relabelling changes.
+  DevBuf<int2> sc_mem;  // one allocation: edge, then pos, ofs, pad, tiles
+  SfxtSched sched{};
+  bool sched_ready = false;
+  bool order_ready = false;    // queue, level and lvlp hold a finished level loop of the resident graph
+  bool order_pending = false;  // the queued SFXT will leave them so
+  bool budgeted = false;       // the query has a device-byte budget: no schedule
   bool sfxt_valid = false;
   std::vector<uint8_t> sfxt_sinks;  // endpoint subset of the current SFXT, per sink (empty = all)
   DevBuf<uint8_t> emask;
@@ -375,6 +384,7 @@ struct cpg_handle {
     graph_on_device = true;
     sfxt_valid = false;
     relabelled = false;
+    order_ready = sched_ready = false;
     if (csr_reorder == 1) relabel_graph();
   }
 
@@ -435,6 +445,7 @@ struct cpg_handle {
     oadjp.swap(nadjp); oadj.swap(nadj); owgt.swap(nw); iadjp.swap(niadjp_d); iedge.swap(nie);
     relabelled = true;
     sfxt_valid = false;
+    order_ready = sched_ready = false;
     h_succ.clear();
     hb.valid = false;
     reorder_ms = now_ms() - t0;
@@ -454,6 +465,14 @@ struct cpg_handle {
     const int64_t per_level = g.n / last_diameter;
     return static_cast<int>(std::min<int64_t>(128, std::max<int64_t>(16, (per_level + 255) / 256)));
   }
+
+  // Scheduled-loop grid: one block per CU, over all XCDs.  The loop has no
+  // barrier to pay for more blocks, and a CU's scattered-load rate bounds
+  // wide levels: on the 1.5M-vertex DAG 0.74 ms with 256 blocks, 0.87 with
+  // 128, 1.6 with 32; narrow levels measure the same from 32 up (50K-vertex
+  // DAG 0.14 ms).  Keeping the blocks on one XCD was slower on every graph
+  // wider than that one (1.6 ms and 0.74; 3.4 and 1.9 at 1.1M vertices).
+  int sched_blocks() const { return sfxt_blocks > 0 ? sfxt_blocks : std::max(1, grid / 8); }
 
   // The endpoint subset of an n-byte mask as one flag per sink (in sink
   // order); empty when the mask is null or chooses every sink.
@@ -480,6 +499,72 @@ struct cpg_handle {
     CPG_HIP(hipStreamSynchronize(stream));
     sfxt_finish(c, count_cache, mask);
     return now_ms() - t0;
+  }
+
+  // Lays out the schedule of the resident graph from the level order the
+  // last level loop left (a relabelled graph's ids are in level order
+  // already).
+  void build_schedule(SfxtArgs& a) {
+    const size_t n = static_cast<size_t>(g.n), m = static_cast<size_t>(g.m);
+    const int L = last_diameter;
+    std::vector<int> first(static_cast<size_t>(L) + 1);
+    d2h(first.data(), lvlp.p, first.size(), stream);
+    CPG_HIP(hipStreamSynchronize(stream));
+    const int nl = first[static_cast<size_t>(L)];
+    // Lanes per vertex: the power of two that takes twice a mean row in one
+    // load (most rows whole, out-degrees being skewed), at most 32.  Level
+    // loop on the 1.5M-vertex DAG (mean 2.7) with 4 / 8 / 16 lanes: 0.96 /
+    // 0.74 / 0.88 ms; 1.1M vertices (5.3) with 8 / 16 / 32: 2.34 / 1.93 /
+    // 2.40; 400K (20) with 16 / 32: 0.66 / 0.55; 250K (27): 2.24 / 1.76.
+    // More lanes where levels are narrower than a wave's vertices, so that
+    // padding every level to whole waves at most doubles the positions.
+    int lanes = 1;
+    const double mean = static_cast<double>(g.m) / static_cast<double>(std::max(1, g.n));
+    while (lanes < 32 && lanes < 2.0 * mean) lanes *= 2;
+    while (lanes < 64 && static_cast<int64_t>(L) * (64 / lanes) > nl) lanes *= 2;
+    const int per = 64 / lanes;
+    std::vector<int> pad(static_cast<size_t>(L) + 1);
+    int64_t np = 0;
+    for (int d = 0; d < L; ++d) {
+      pad[static_cast<size_t>(d)] = static_cast<int>(np);
+      np += (static_cast<int64_t>(first[static_cast<size_t>(d) + 1] - first[static_cast<size_t>(d)]) + per - 1) / per * per;
+      if (np > 0x7fffff00ll) {  // positions are 32-bit: such a graph keeps the level loop
+        order_ready = false;
+        return;
+      }
+    }
+    pad[static_cast<size_t>(L)] = static_cast<int>(np);
+    const size_t ints = n + (static_cast<size_t>(np) + 1) + pad.size() + sfxt_sched_tiles(static_cast<int>(np));
+    sc_mem.reserve(std::max<size_t>(m, 1) + (ints + 1) / 2);
+    int2* edge_d = sc_mem.p;
+    int* pos_d = reinterpret_cast<int*>(edge_d + std::max<size_t>(m, 1));
+    unsigned* ofs_d = reinterpret_cast<unsigned*>(pos_d + n);
+    int* pad_d = reinterpret_cast<int*>(ofs_d + np + 1);
+    unsigned* tiles_d = reinterpret_cast<unsigned*>(pad_d + pad.size());
+    best.reserve(static_cast<size_t>(std::max<int64_t>(np, g.n)) + kSfxtPad);
+    a.best = best.p;
+    h2d(pad_d, pad.data(), pad.size(), stream);
+    launch_sfxt_sched_build(a, relabelled ? nullptr : queue.p, pad_d, nl, static_cast<int>(np), pos_d, ofs_d, edge_d,
+                            tiles_d, stream);
+    CPG_HIP(hipStreamSynchronize(stream));  // pad goes out of scope
+    sched = SfxtSched{};
+    sched.np = static_cast<int>(np);
+    sched.first = L > 1 ? pad[1] : static_cast<int>(np);
+    sched.nl = nl;
+    sched.lanes = lanes;
+    sched.pos = pos_d;
+    sched.ofs = reinterpret_cast<const int*>(ofs_d);
+    sched.edge = edge_d;
+    sched_ready = true;
+  }
+
+  // Gives the schedule's memory back (a query under a device-byte budget
+  // holds what it held without one; the level order stays).
+  void drop_schedule() {
+    if (!sched_ready) return;
+    sched_ready = false;
+    sc_mem.release();
+    if (best.n > static_cast<size_t>(g.n) + kSfxtPad) best.release();
   }
 
   // The SFXT in two halves, so that a caller can put its own work on the
@@ -531,8 +616,14 @@ struct cpg_handle {
         a.sink_mask = emask.p;
       }
       a.orig = relabelled ? orig_d.p : nullptr;
-      // 0 (automatic) is the edge-parallel fence-free level loop
+      // 0 (automatic): the scheduled loop once an earlier SFXT on this graph
+      // has left its level order, before that the edge-parallel fence-free
+      // level loop
       const int method = sfxt_method == 0 ? 5 : sfxt_method;
+      if (sfxt_method == 0 && !budgeted && !sched_ready && order_ready && last_diameter > 0) build_schedule(a);
+      const bool scheduled = sfxt_method == 0 && sched_ready;
+      if (!scheduled) order_ready = false;
+      order_pending = !scheduled && (method == 1 || method >= 4);
       // Its blocks on one XCD (round-robin dispatch puts every 8th block on
       // the same XCD) while a level holds few fanin records, over all XCDs
       // above that: on the 1.5M-vertex DAG (13.6K records per level) one
@@ -571,17 +662,20 @@ struct cpg_handle {
         ev_levels.create();
         CPG_HIP(hipEventRecord(ev_sfxt.a, stream));
       }
-      if (dataflow || method >= 4) launch_sfxt_dataflow_init(a, stream);
+      if (scheduled) {}  // its own pass over the positions
+      else if (dataflow || method >= 4) launch_sfxt_dataflow_init(a, stream);
       else if (method == 3) launch_sfxt_local_init(a, stream);
       else launch_sfxt_init(a, stream);
       if (kernel_timing) CPG_HIP(hipEventRecord(ev_levels.a, stream));
-      timing.sfxt_blocks = dataflow      ? launch_sfxt_dataflow(a, df_grid, stream)
+      a.find_succ = scheduled ? 1 : 0;
+      timing.sfxt_blocks = scheduled     ? launch_sfxt_scheduled(a, sched, sched_blocks(), stream)
+                           : dataflow    ? launch_sfxt_dataflow(a, df_grid, stream)
                            : method == 3 ? launch_sfxt_local(a, level_loop_blocks(), stream)
                            : method == 4 ? launch_sfxt_levels_nf(a, level_loop_blocks(), stream)
                            : method == 5 ? launch_sfxt_levels_edges(a, level_loop_blocks(), stream)
                                          : launch_sfxt_levels(a, level_loop_blocks(), stream);
       if (kernel_timing) CPG_HIP(hipEventRecord(ev_levels.b, stream));
-      if (relabelled) launch_sfxt_succ_relabel(succ.p, perm_d.p, g.n, stream);
+      if (relabelled && !scheduled) launch_sfxt_succ_relabel(succ.p, perm_d.p, g.n, stream);
       // The lifting table needs the level count.  Levels depend on the
       // graph alone (not on the endpoint subset), so after this graph's
       // first levelization the count is known without waiting for the loop.
@@ -622,6 +716,7 @@ struct cpg_handle {
     if (c.nsv_err) throw std::runtime_error("SFXT next-smaller descent found no answer");
     diameter = c.num_levels;
     last_diameter = diameter;
+    order_ready = order_ready || order_pending;
     uint32_t bits = c.max_abs_distf_bits;
     std::memcpy(&max_abs_distf, &bits, 4);
     sfxt_valid = true;
@@ -640,7 +735,7 @@ struct cpg_handle {
     return b(oadjp) + b(oadj) + b(owgt) + b(iadjp) + b(iedge) + b(srcs) + b(sinks) + b(deps) +
            b(queue) + b(lvlp) + b(level) + b(dist) + b(succ) + b(src_dist) + b(big) + b(best) +
            b(distf) + b(vrec) + b(devs) + b(devs_tmp) + b(devinfo) + b(lift) + b(sctl) + b(dfw) +
-           b(emask) + b(keep);
+           b(emask) + b(keep) + b(sc_mem);
   }
 
   void release_pfxt_buffers() {
@@ -800,7 +895,10 @@ struct cpg_handle {
         d2h(h_src_dist.p, src_dist.p, nsrc, stream);
       }
     };
+    budgeted = o.mem_budget_bytes > 0;
+    if (budgeted) drop_schedule();
     const bool queued = sfxt_enqueue(true, o.endpoint_mask);
+    budgeted = false;
     copy_source_dists();
     if (queued) d2h(h_sctl.p, sctl.p, 1, stream);
     CPG_HIP(hipStreamSynchronize(stream));

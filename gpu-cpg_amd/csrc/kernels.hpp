@@ -63,6 +63,24 @@ struct SfxtArgs {
   int place_stride;
   int wave_entries;  // edge-parallel loop: queue entries a wave takes at a time (1-64; 0 = 64)
   int64_t m;  // edges (the fence-free loop picks its records per step by m / n)
+  // 1: succ[] is not set yet; the deviation pass finds each successor among
+  // the fanouts (largest original id at the smallest candidate)
+  int find_succ;
+};
+
+// Level-order schedule of a graph: what the scheduled loop reads instead of
+// the CSR.  It depends on the edges alone, so it is laid out once per
+// resident graph and serves every endpoint subset.  Vertices have positions
+// in level order, every level starting at a multiple of 64 / lanes (the
+// vertices a wave takes at a time), so a wave never holds two levels.
+struct SfxtSched {
+  int np;            // positions (padding included), a multiple of 64 / lanes
+  int first;         // first position of level 1 (level 0: the sinks, in list order)
+  int nl;            // levelized vertices
+  int lanes;         // lanes per vertex: 1, 2, 4, 8, 16, 32 or 64
+  const int* pos;    // position of each vertex (-1: never levelized), n
+  const int* ofs;    // fanout records of each position, np + 1
+  const int2* edge;  // {position of w, (int)(w_e * 10000.0f)}
 };
 
 // Q endpoint subsets relaxed in one level loop (served queries): the
@@ -121,6 +139,17 @@ int launch_sfxt_dataflow(const SfxtArgs& args, int blocks, hipStream_t stream);
 // barrier; same results as the level loop).  Returns the grid used.
 void launch_sfxt_local_init(const SfxtArgs& args, hipStream_t stream);
 int launch_sfxt_local(const SfxtArgs& args, int blocks, hipStream_t stream);
+// Builds a schedule's arrays (n, np + 1 and m slots) from a finished level
+// loop: order[0..nl) the vertices in level order (null: ascending ids),
+// level and lvlp of that loop, pad the levels' first positions.  tiles needs
+// sfxt_sched_tiles(np) counts.
+uint64_t sfxt_sched_tiles(int np);
+void launch_sfxt_sched_build(const SfxtArgs& args, const int* order, const int* pad, int nl, int np, int* pos,
+                             unsigned* ofs, int2* edge, unsigned* tiles, hipStream_t stream);
+// The SFXT in schedule order: level and dist of every vertex (distf too),
+// succ[] left to the deviation pass (args.find_succ).  args.best holds a
+// state word per position.  Returns the working blocks.
+int launch_sfxt_scheduled(const SfxtArgs& args, const SfxtSched& sched, int blocks, hipStream_t stream);
 // Relabelled graph: succ[] holds original ids after a level loop; map
 // them to the relabelled ids (perm: original -> relabelled).
 void launch_sfxt_succ_relabel(int* succ, const int* perm, int n, hipStream_t stream);

@@ -1126,6 +1126,244 @@ __global__ void __launch_bounds__(kLocBlock) sfxt_local_kernel(SfxtArgs a) {
   if (ok && bid == 0 && t == 0) ctl->num_levels = a.nsinks > 0 ? d + 1 : 0;
 }
 
+// ---------------------------------------------------------------------------
+// Scheduled loop: levelize and relax in a known level order.
+//
+// The level loops above find the level order as they go (deps counters,
+// queue, a grid barrier per level).  The order depends on the edges alone,
+// so once one of them has run, a resident graph keeps it as a schedule
+// (SfxtSched), and later runs settle the vertices in that order pull-style,
+// as relax_bu_step (gpucpg/gpucpg.cu:1167-1187) reads the fanouts: dist =
+// min over reachable fanouts of dist[w] + (int)(w_e * 10000.0f), level = 1 +
+// max level[w] (the peel depth of bfs_td_step_privatized, :2215-2283).  Only
+// the order is kept; both values are computed from the edges on every run.
+//
+// There is no barrier, queue or atomic.  Each position has a write-once
+// 64-bit state word, level << 32 | dist (all ones until settled), stored and
+// loaded at device scope, and a lane polls a fanout's word until it is
+// there.  Wave k of W takes the chunks k, k + W, ... of 64 / lanes
+// consecutive positions; a chunk lies within one level and a vertex's
+// fanouts lie in earlier levels, so the first unsettled chunk never waits
+// and, with every wave resident, the loop always advances.  A wait ends at
+// kSpinLimit polls, or once another wave has raised the error.
+//
+// What bounds it: the latency of one level (a state store becoming visible
+// to a load, one reduction over a vertex's lanes), then the rate of
+// scattered loads (one CU about 1.2 G lanes/s).  The records of the next
+// chunk are loaded while this one waits.
+// ---------------------------------------------------------------------------
+struct SchedArgs {
+  SfxtSched s;
+  unsigned long long* state;
+  SfxtCtl* ctl;
+};
+
+constexpr int kSchedBlock = 256;
+
+template <int kLanes, int kU>
+__global__ void __launch_bounds__(kSchedBlock) sfxt_sched_kernel(SchedArgs a) {
+  constexpr int kV = 64 / kLanes;  // vertices per chunk
+  const unsigned nblk = gridDim.x, bid = blockIdx.x;
+  const int lane = __lane_id();
+  const int sub = lane % kLanes, grp = lane / kLanes;
+  const int nw = static_cast<int>(nblk * (blockDim.x / 64u));
+  const int nchunk = a.s.np / kV;
+  // consecutive chunks go to different blocks (CUs)
+  int c = a.s.first / kV + static_cast<int>((threadIdx.x / 64u) * nblk + bid);
+
+  auto range = [&](int ch, int& b, int& e) {
+    b = e = 0;
+    if (ch < nchunk) {
+      b = a.s.ofs[ch * kV + grp];
+      e = a.s.ofs[ch * kV + grp + 1];
+    }
+  };
+  // this lane's first kU records of a row; past the end {-1, 0}
+  auto fetch = [&](int b, int e, int2* r) {
+#pragma unroll
+    for (int q = 0; q < kU; ++q) {
+      const int j = b + sub + q * kLanes;
+      r[q] = a.s.edge[j < e ? j : 0];
+      if (j >= e) r[q].x = -1;
+    }
+  };
+  int b0, e0, b1, e1;
+  int2 r0[kU];
+  range(c, b0, e0);
+  fetch(b0, e0, r0);
+  range(c + nw, b1, e1);
+  for (; c < nchunk; c += nw) {
+    int bd = kIntMax, lev = 0;
+    unsigned long long st[kU];
+    auto load = [&](const int2* r) {
+#pragma unroll
+      for (int q = 0; q < kU; ++q) st[q] = r[q].x >= 0 ? ld_dev64(a.state + r[q].x) : 0ull;
+    };
+    // polls the words still empty (the wave stays together), then takes all
+    auto settle = [&](const int2* r) {
+      for (unsigned spins = 1;; ++spins) {
+        bool open = false;
+#pragma unroll
+        for (int q = 0; q < kU; ++q) open = open || st[q] == ~0ull;
+        if (__ballot(open) == 0) break;
+        if (spins > kSpinLimit) { atomicExch(&a.ctl->err, 1); break; }
+        if ((spins & 255u) == 0u && __ballot(ld_dev32(&a.ctl->err) != 0) != 0) break;
+        __builtin_amdgcn_s_sleep(1);
+#pragma unroll
+        for (int q = 0; q < kU; ++q)
+          if (st[q] == ~0ull) st[q] = ld_dev64(a.state + r[q].x);
+      }
+#pragma unroll
+      for (int q = 0; q < kU; ++q) {
+        if (r[q].x < 0 || st[q] == ~0ull) continue;  // empty only after an error
+        lev = max(lev, static_cast<int>(st[q] >> 32) + 1);
+        const int d = static_cast<int>(static_cast<uint32_t>(st[q]));
+        if (d != kIntMax) bd = min(bd, static_cast<int>(static_cast<unsigned>(d) + static_cast<unsigned>(r[q].y)));
+      }
+    };
+    load(r0);
+    // the next chunk's records and the range after it travel meanwhile
+    int2 r1[kU];
+    int b2, e2;
+    fetch(b1, e1, r1);
+    range(c + 2 * nw, b2, e2);
+    settle(r0);
+    for (int b = b0 + kU * kLanes; __ballot(b < e0) != 0; b += kU * kLanes) {  // longer rows
+      fetch(b, e0, r0);
+      load(r0);
+      settle(r0);
+    }
+#pragma unroll
+    for (int o = 1; o < kLanes; o <<= 1) {
+      bd = min(bd, __shfl_xor(bd, o));
+      lev = max(lev, __shfl_xor(lev, o));
+    }
+    if (sub == 0 && b0 < e0)  // a padding position has no records and is never read
+      st_dev64(a.state + c * kV + grp,
+               (static_cast<unsigned long long>(static_cast<uint32_t>(lev)) << 32) | static_cast<uint32_t>(bd));
+#pragma unroll
+    for (int q = 0; q < kU; ++q) r0[q] = r1[q];
+    b0 = b1;
+    e0 = e1;
+    b1 = b2;
+    e1 = e2;
+  }
+}
+
+// State words before the loop: the sinks are settled, every other position
+// is empty.
+__global__ void __launch_bounds__(256) sfxt_sched_init_kernel(SfxtArgs a, SfxtSched s) {
+  for (int p = blockIdx.x * blockDim.x + threadIdx.x; p < s.np; p += gridDim.x * blockDim.x) {
+    unsigned long long v = ~0ull;
+    if (p < a.nsinks)
+      v = a.sink_mask && !a.sink_mask[a.sinks[p]] ? static_cast<unsigned long long>(kIntMax) : 0ull;
+    a.best[p] = v;
+  }
+}
+
+// dist, level and distf of every vertex from its position's state, and the
+// control block's level count and largest |distf|.
+__global__ void __launch_bounds__(256) sfxt_sched_finish_kernel(SfxtArgs a, SfxtSched s) {
+  float mx = 0.0f;
+  int top = -1;
+  for (int v = blockIdx.x * blockDim.x + threadIdx.x; v < a.n; v += gridDim.x * blockDim.x) {
+    const int p = s.pos[v];
+    int d = kIntMax, lev = -1;
+    if (p >= 0) {
+      const unsigned long long st = a.best[p];
+      d = static_cast<int>(static_cast<uint32_t>(st));
+      lev = static_cast<int>(st >> 32);
+    }
+    const float df = static_cast<float>(d) / static_cast<float>(kScaleUp);
+    a.dist[v] = d;
+    a.level[v] = lev;
+    a.distf[v] = df;
+    top = max(top, lev);
+    if (d != kIntMax) mx = fmaxf(mx, fabsf(df));
+  }
+  mx = wave_max(mx);
+  top = wave_max_int(top);
+  if (__lane_id() == 0) {
+    atomicMax(&a.ctl->max_abs_distf_bits, __float_as_uint(mx));
+    if (top >= 0) atomicMax(&a.ctl->num_levels, top + 1);
+  }
+  if (blockIdx.x == 0 && threadIdx.x == 0) a.ctl->levelized = static_cast<unsigned>(s.nl);
+}
+
+// Schedule build: positions and fanout counts, ...
+__global__ void __launch_bounds__(256) sfxt_sched_clear_kernel(int n, int np, int* pos, unsigned* ofs) {
+  const int m = max(n, np + 1);
+  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < m; i += gridDim.x * blockDim.x) {
+    if (i < n) pos[i] = -1;
+    if (i <= np) ofs[i] = 0u;
+  }
+}
+__global__ void __launch_bounds__(256) sfxt_sched_place_kernel(SfxtArgs a, const int* order, const int* pad, int nl,
+                                                               int* pos, unsigned* ofs) {
+  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < nl; i += gridDim.x * blockDim.x) {
+    const int u = order ? order[i] : i;
+    const int d = a.level[u];
+    const int p = pad[d] + (i - a.lvlp[d]);
+    pos[u] = p;
+    ofs[p] = static_cast<unsigned>(a.oadjp[u + 1] - a.oadjp[u]);
+  }
+}
+// ... the counts' exclusive scan (tile sums, scanned by one block, then the
+// tiles), ...
+constexpr int kSchedTile = 2048;
+__global__ void __launch_bounds__(256) sfxt_sched_sums_kernel(const unsigned* ofs, int len, unsigned* tiles) {
+  __shared__ unsigned s_sum;
+  if (threadIdx.x == 0) s_sum = 0;
+  __syncthreads();
+  unsigned c = 0;
+  for (int j = threadIdx.x; j < kSchedTile; j += 256) {
+    const int64_t i = static_cast<int64_t>(blockIdx.x) * kSchedTile + j;
+    if (i < len) c += ofs[i];
+  }
+  atomicAdd(&s_sum, c);
+  __syncthreads();
+  if (threadIdx.x == 0) tiles[blockIdx.x] = s_sum;
+}
+__global__ void __launch_bounds__(256) sfxt_sched_scan_kernel(unsigned* ofs, int len, const unsigned* tiles) {
+  constexpr int kPer = kSchedTile / 256;
+  __shared__ unsigned s_wave[4];
+  const int lane = __lane_id(), wave = static_cast<int>(threadIdx.x) >> 6;
+  const int64_t i0 = static_cast<int64_t>(blockIdx.x) * kSchedTile + static_cast<int64_t>(threadIdx.x) * kPer;
+  unsigned v[kPer], mine = 0;
+#pragma unroll
+  for (int q = 0; q < kPer; ++q) {
+    v[q] = i0 + q < len ? ofs[i0 + q] : 0u;
+    mine += v[q];
+  }
+  unsigned incl = mine;
+  for (int o = 1; o < 64; o <<= 1) {
+    const unsigned x = __shfl_up(incl, o);
+    if (lane >= o) incl += x;
+  }
+  if (lane == 63) s_wave[wave] = incl;
+  __syncthreads();
+  unsigned run = tiles[blockIdx.x] + incl - mine;
+  for (int w = 0; w < wave; ++w) run += s_wave[w];
+#pragma unroll
+  for (int q = 0; q < kPer; ++q) {
+    if (i0 + q < len) ofs[i0 + q] = run;
+    run += v[q];
+  }
+}
+// ... and the records, a vertex's in fanout order.
+__global__ void __launch_bounds__(256) sfxt_sched_edges_kernel(SfxtArgs a, const int* pos, const unsigned* ofs,
+                                                               int2* edge) {
+  for (int u = blockIdx.x * blockDim.x + threadIdx.x; u < a.n; u += gridDim.x * blockDim.x) {
+    const int p = pos[u];
+    if (p < 0) continue;
+    const int b = a.oadjp[u], e = a.oadjp[u + 1];
+    const unsigned to = ofs[p];
+    for (int j = b; j < e; ++j)
+      edge[to + static_cast<unsigned>(j - b)] =
+          make_int2(pos[a.oadj[j]], static_cast<int>(a.owgt[j] * static_cast<float>(kScaleUp)));
+  }
+}
+
 // Relabelled graph: the level loops store the successor's original id;
 // this maps it to the relabelled id before the deviation index is built.
 __global__ void __launch_bounds__(256) sfxt_succ_relabel_kernel(int* succ, const int* perm, int n) {
@@ -1329,6 +1567,21 @@ __device__ inline unsigned xcd_block(unsigned b, unsigned nb) {
   return nb % kX == 0 ? (b % kX) * (nb / kX) + b / kX : b;
 }
 
+// One fanout w (distance dw, weight we) against the best so far: candidate bd,
+// original id bt, vertex s.
+__device__ __forceinline__ void succ_candidate(const SfxtArgs& a, int w, int dw, float we, int& bd, int& bt, int& s) {
+  if (dw == kIntMax) return;
+  const int c = static_cast<int>(static_cast<unsigned>(dw) +
+                                 static_cast<unsigned>(static_cast<int>(we * static_cast<float>(kScaleUp))));
+  if (c > bd) return;
+  const int t = a.orig ? a.orig[w] : w;
+  if (c < bd || t > bt) {
+    bd = c;
+    bt = t;
+    s = w;
+  }
+}
+
 // Deviation records of every settled vertex in fanout order, their smallest
 // delta, and the vertex record without its nsv pointer.  Lists of up to
 // kThreadSort records are sorted here (stable insertion sort by delta);
@@ -1353,8 +1606,21 @@ __global__ void __launch_bounds__(256) sfxt_devs_kernel(SfxtArgs a) {
       if (a.level[u] < 0 || a.dist[u] == kIntMax) {  // unsettled or reaches no chosen sink
         a.vrec[u] = default_vrec();
         a.devinfo[u] = make_int2(b, 0);
+        if (a.find_succ) a.succ[u] = -1;
       } else {
-        const int s = a.succ[u];
+        int s = -1;
+        if (a.find_succ) {
+          // update_successors_bu (gpucpg/gpucpg.cu:2606-2628): the largest id
+          // among the fanouts at the minimum
+          int bd = kIntMax, bt = -1;
+          for (int j = b; j < e; ++j) {
+            const int w = a.oadj[j];
+            succ_candidate(a, w, a.dist[w], a.owgt[j], bd, bt, s);
+          }
+          a.succ[u] = s;
+        } else {
+          s = a.succ[u];
+        }
         const float df = a.distf[u];
         float mind = __builtin_huge_valf();
         for (int j = b; j < e; ++j) {
@@ -1437,10 +1703,29 @@ __global__ void __launch_bounds__(256) sfxt_devs_wave_kernel(SfxtArgs a) {
       if (lane == 0) {
         a.vrec[u] = default_vrec();
         a.devinfo[u] = make_int2(b, 0);
+        if (a.find_succ) a.succ[u] = -1;
       }
       continue;
     }
-    const int s = a.succ[u];
+    int s = -1;
+    if (a.find_succ) {
+      int bd = kIntMax, bt = -1;
+      for (int j = b + lane; j < e; j += 64) {
+        const int w = a.oadj[j];
+        succ_candidate(a, w, a.dist[w], a.owgt[j], bd, bt, s);
+      }
+      for (int o = 32; o > 0; o >>= 1) {
+        const int od = __shfl_xor(bd, o), ot = __shfl_xor(bt, o), os = __shfl_xor(s, o);
+        if (od < bd || (od == bd && ot > bt)) {
+          bd = od;
+          bt = ot;
+          s = os;
+        }
+      }
+      if (lane == 0) a.succ[u] = s;
+    } else {
+      s = a.succ[u];
+    }
     const float df = a.distf[u];
     int cnt = 0;
     float mind = __builtin_huge_valf();
@@ -1696,6 +1981,59 @@ int launch_sfxt_levels_edges(const SfxtArgs& args, int blocks, hipStream_t strea
   const int working = loop_grid(blocks, resident_blocks(k, kSfxtBlock) / stride);
   launch_resident(k, working * stride, kSfxtBlock, args, stream);
   return working;
+}
+
+uint64_t sfxt_sched_tiles(int np) { return (static_cast<uint64_t>(np) + 1 + kSchedTile - 1) / kSchedTile; }
+
+void launch_sfxt_sched_build(const SfxtArgs& args, const int* order, const int* pad, int nl, int np, int* pos,
+                             unsigned* ofs, int2* edge, unsigned* tiles, hipStream_t stream) {
+  const int cus = device_cus();
+  const int nt = static_cast<int>(sfxt_sched_tiles(np));
+  hipLaunchKernelGGL(sfxt_sched_clear_kernel, dim3(flat_grid(std::max(args.n, np + 1), cus)), dim3(256), 0, stream,
+                     args.n, np, pos, ofs);
+  CPG_HIP(hipGetLastError());
+  hipLaunchKernelGGL(sfxt_sched_place_kernel, dim3(flat_grid(nl, cus)), dim3(256), 0, stream, args, order, pad, nl,
+                     pos, ofs);
+  CPG_HIP(hipGetLastError());
+  hipLaunchKernelGGL(sfxt_sched_sums_kernel, dim3(nt), dim3(256), 0, stream, ofs, np + 1, tiles);
+  CPG_HIP(hipGetLastError());
+  launch_exclusive_scan_u32(tiles, static_cast<uint64_t>(nt), stream);
+  hipLaunchKernelGGL(sfxt_sched_scan_kernel, dim3(nt), dim3(256), 0, stream, ofs, np + 1, tiles);
+  CPG_HIP(hipGetLastError());
+  hipLaunchKernelGGL(sfxt_sched_edges_kernel, dim3(flat_grid(args.n, cus)), dim3(256), 0, stream, args, pos, ofs,
+                     edge);
+  CPG_HIP(hipGetLastError());
+}
+
+template <int kLanes, int kU>
+static int launch_sched_loop(const SchedArgs& a, int blocks, hipStream_t stream) {
+  auto k = sfxt_sched_kernel<kLanes, kU>;
+  const int working = loop_grid(blocks, resident_blocks(k, kSchedBlock));
+  launch_resident(k, working, kSchedBlock, a, stream);
+  return working;
+}
+
+int launch_sfxt_scheduled(const SfxtArgs& args, const SfxtSched& s, int blocks, hipStream_t stream) {
+  const int cus = device_cus();
+  hipLaunchKernelGGL(sfxt_sched_init_kernel, dim3(flat_grid(s.np, cus)), dim3(256), 0, stream, args, s);
+  CPG_HIP(hipGetLastError());
+  int used = 0;
+  if (s.np > s.first) {
+    const SchedArgs a{s, args.best, args.ctl};
+    switch (s.lanes) {
+      case 1: used = launch_sched_loop<1, 4>(a, blocks, stream); break;
+      case 2: used = launch_sched_loop<2, 4>(a, blocks, stream); break;
+      case 4: used = launch_sched_loop<4, 2>(a, blocks, stream); break;
+      case 8: used = launch_sched_loop<8, 2>(a, blocks, stream); break;
+      case 16: used = launch_sched_loop<16, 2>(a, blocks, stream); break;
+      case 32: used = launch_sched_loop<32, 2>(a, blocks, stream); break;
+      case 64: used = launch_sched_loop<64, 2>(a, blocks, stream); break;
+      default: throw std::runtime_error("scheduled SFXT loop: lanes per vertex must be a power of two up to 64");
+    }
+  }
+  hipLaunchKernelGGL(sfxt_sched_finish_kernel, dim3(flat_grid(args.n, cus)), dim3(256), 0, stream, args, s);
+  CPG_HIP(hipGetLastError());
+  return used;
 }
 
 int sfxt_dataflow_grid(int blocks) {

@@ -1,0 +1,140 @@
+"""The SFXT in schedule order: the second and later runs on a resident graph
+settle its vertices in the level order the first run left.  Every run has
+to give the oracle's dist, succ and level, with and without an endpoint
+subset, as loaded and relabelled, and the query's costs bit for bit.  The
+cases sit at the edges of the schedule: each choice of lanes per vertex,
+rows longer than a wave's step, levels narrower and wider than a wave's
+vertices, vertices on a cycle, one level, no edges, and a graph replaced by
+another in the same handle."""
+import numpy as np
+import pytest
+
+import cpgamd
+import pyoracle
+from test_simt_emulator import bits_equal, emu  # noqa: F401  (fixture)
+
+
+def layered(sizes, deg, seed, hub=0):
+    """Levels of the given sizes (sources first), deg random fanouts per
+    vertex one to three levels ahead, one vertex of hub extra fanouts."""
+    rng = np.random.default_rng(seed)
+    first = np.concatenate([[0], np.cumsum(sizes)])
+    n, L = int(first[-1]), len(sizes)
+    eu, ev = [], []
+    for lv in range(L - 1):
+        for a in range(first[lv], first[lv + 1]):
+            d = rng.integers(1, 2 * deg) if deg > 1 else 1
+            tl = np.minimum(lv + rng.integers(1, 4, size=d), L - 1)
+            heads = {int(rng.integers(first[t], first[t + 1])) for t in tl}
+            heads.add(int(rng.integers(first[lv + 1], first[lv + 2])))
+            eu += [a] * len(heads)
+            ev += sorted(heads)
+    if hub:
+        heads = rng.choice(np.arange(first[1], n), size=min(hub, n - first[1]), replace=False)
+        eu += [0] * len(heads)
+        ev += [int(x) for x in heads]
+    ids = rng.permutation(n)
+    u, v = ids[np.asarray(eu, np.int64)], ids[np.asarray(ev, np.int64)]
+    w = rng.uniform(0.01, 1.0, len(u)).astype(np.float32)
+    w[rng.random(len(w)) < 0.3] = 0.25  # equal candidates: the successor's tie rule
+    return n, u.astype(np.int32), v.astype(np.int32), w
+
+
+SHAPES = {
+    "sparse": lambda: layered([9, 70, 130, 64, 1, 3, 65, 20], 1, 1),
+    "mean3": lambda: layered([40] * 9, 3, 2),
+    "mean6": lambda: layered([33, 100, 31, 32, 17], 6, 3),
+    "mean12": lambda: layered([50, 60, 70, 20], 12, 4),
+    "dense_hub": lambda: layered([20, 90, 90, 40], 24, 5, hub=200),
+    "chain": lambda: (19, np.arange(18, dtype=np.int32), np.arange(1, 19, dtype=np.int32),
+                      np.linspace(0.01, 0.9, 18, dtype=np.float32)),
+    "one_edge": lambda: (2, np.array([1], np.int32), np.array([0], np.int32), np.array([0.5], np.float32)),
+    "cycle": lambda: with_cycle(*layered([12, 30, 30, 9], 3, 6)),
+    "no_edges": lambda: (5, np.zeros(0, np.int32), np.zeros(0, np.int32), np.zeros(0, np.float32)),
+}
+
+
+def with_cycle(n, u, v, w):
+    """Three vertices on a cycle that reaches the graph, and one alone."""
+    more = np.array([[n, n + 1], [n + 1, n + 2], [n + 2, n], [n, int(v[0])]], np.int32)
+    return (n + 4, np.concatenate([u, more[:, 0]]), np.concatenate([v, more[:, 1]]),
+            np.concatenate([w, np.full(4, 0.1, np.float32)]))
+
+
+def check_runs(lib, n, u, v, w, reorder, k):
+    og = pyoracle.OracleGraph.from_edges(n, u, v, w)
+    sinks = np.nonzero(np.bincount(u, minlength=n)[:n] == 0)[0]
+    some = np.zeros(n, np.uint8)
+    some[sinks[::2]] = 1
+    g = lib.CpGen()
+    try:
+        g.load_edges(n, u, v, w)
+        if reorder:
+            g.set_csr_reorder(1)
+        for mask in (None, None, some, None, some):
+            dist, succ, level, levels = og.sfxt(mask)
+            g.reset()
+            g.report_paths(k, endpoint_mask=mask)
+            gd, gs, gl = g.sfxt()
+            np.testing.assert_array_equal(gd, dist)
+            np.testing.assert_array_equal(gs, succ)
+            np.testing.assert_array_equal(gl, level)
+            assert g.graph_diameter == levels
+            want, _ = og.topk(dist, succ, k)
+            assert bits_equal(want, g.get_slacks(k))
+    finally:
+        g.close()
+
+
+@pytest.mark.parametrize("reorder", [False, True])
+@pytest.mark.parametrize("shape", sorted(SHAPES))
+def test_emulated_schedule_equals_oracle(emu, shape, reorder):  # noqa: F811
+    check_runs(emu, *SHAPES[shape](), reorder, 0)
+
+
+def test_emulated_schedule_follows_the_loaded_graph(emu):  # noqa: F811
+    g = emu.CpGen()
+    try:
+        for shape in ("mean6", "chain", "mean3"):
+            n, u, v, w = SHAPES[shape]()
+            og = pyoracle.OracleGraph.from_edges(n, u, v, w)
+            dist, succ, level, _ = og.sfxt()
+            g.load_edges(n, u, v, w)
+            for method in (0, 0, 2, 0, 3, 0):  # loops that leave no level order between
+                g.reset()
+                g.report_paths(0, sfxt_method=method)
+                for got, want in zip(g.sfxt(), (dist, succ, level)):
+                    np.testing.assert_array_equal(got, want)
+    finally:
+        g.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("reorder", [False, True])
+@pytest.mark.parametrize("shape", sorted(SHAPES))
+def test_gpu_schedule_equals_oracle(shape, reorder):
+    check_runs(cpgamd, *SHAPES[shape](), reorder, 40)
+
+
+@pytest.mark.gpu
+def test_gpu_schedule_deep_and_wide():
+    n, u, v, w = layered([300] * 150, 4, 7)
+    check_runs(cpgamd, n, u, v, w, False, 500)
+
+
+@pytest.mark.gpu
+def test_gpu_budget_leaves_the_schedule_out():
+    """A budget of what the first query held is enough for every later one."""
+    n, u, v, w = layered([300] * 150, 4, 8)
+    g = cpgamd.CpGen()
+    try:
+        g.load_edges(n, u, v, w)
+        g.report_paths(100)
+        want, held = g.get_slacks(100), g.timings()["device_bytes"]
+        for budget in (0, held, 0, held):
+            g.reset()
+            g.report_paths(100, mem_budget_bytes=budget)
+            assert bits_equal(want, g.get_slacks(100))
+            assert not budget or g.timings()["device_bytes"] <= budget
+    finally:
+        g.close()

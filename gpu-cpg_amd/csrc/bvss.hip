@@ -60,6 +60,57 @@ __device__ inline unsigned wave_excl_scan(unsigned v, unsigned* total) {
   return incl - v;
 }
 
+// A wave's triples on their way out.  They are staged in LDS and leave with
+// one atomic on the output counter per kBvssStage of them: the counter is
+// one address for the whole grid, about 10 ns an atomic, and one atomic per
+// tile made it the MFMA kernel's bound (239K tiles 0.80 ms).
+constexpr unsigned kBvssStage = 256;
+
+struct BvssOut {
+  uint64_t* stage;   // this wave's kBvssStage slots
+  unsigned staged;   // wave-uniform
+
+  __device__ inline void put(const BvssArgs& a, uint64_t slot, uint64_t key) {
+    if (slot < a.cap) a.keys[slot] = key;
+  }
+  __device__ inline uint64_t reserve(const BvssArgs& a, unsigned n) {
+    unsigned long long base = 0;
+    if (__lane_id() == 0) base = atomicAdd(&a.ctl->count, static_cast<unsigned long long>(n));
+    return __shfl(base, 0);
+  }
+  __device__ inline void flush(const BvssArgs& a) {
+    if (staged == 0) return;
+    __builtin_amdgcn_wave_barrier();
+    const uint64_t base = reserve(a, staged);
+    for (unsigned i = __lane_id(); i < staged; i += 64) put(a, base + i, stage[i]);
+    __builtin_amdgcn_wave_barrier();
+    staged = 0;
+  }
+  // Emits every set bit of each lane's words (frontier f, interval iv, rows).
+  template <int kN>
+  __device__ inline void emit(const BvssArgs& a, int f, int iv, const uint64_t (&hits)[kN], const int (&rows)[kN]) {
+    unsigned cnt = 0, tot = 0;
+#pragma unroll
+    for (int i = 0; i < kN; ++i) cnt += static_cast<unsigned>(__popcll(hits[i]));
+    const unsigned off = wave_excl_scan(cnt, &tot);
+    if (tot == 0) return;
+    if (staged + tot > kBvssStage) flush(a);
+    const bool direct = tot > kBvssStage;  // more than the stage holds
+    uint64_t slot = direct ? reserve(a, tot) + off : staged + off;
+#pragma unroll
+    for (int i = 0; i < kN; ++i)
+      for (uint64_t h = hits[i]; h; h &= h - 1) {
+        const int u = iv * 64 + __ffsll(static_cast<long long>(h)) - 1;
+        const uint64_t key = (((static_cast<uint64_t>(static_cast<uint32_t>(f)) << a.vbits) |
+                               static_cast<uint32_t>(u)) << a.vbits) | static_cast<uint32_t>(rows[i]);
+        if (direct) put(a, slot, key);
+        else stage[slot] = key;
+        ++slot;
+      }
+    if (!direct) staged += tot;
+  }
+};
+
 }  // namespace
 
 __global__ void __launch_bounds__(kBvssBlock) bvss_frontier_kernel(BvssArgs a, const int* fptr,
@@ -90,6 +141,8 @@ __global__ void __launch_bounds__(kBvssBlock) bvss_density_kernel(BvssArgs a, in
 
 // Bitmap path: one lane per (row entry, frontier) of the sparse intervals.
 __global__ void __launch_bounds__(kBvssBlock) bvss_bitmap_kernel(BvssArgs a) {
+  __shared__ uint64_t s_stage[kBvssBlock / 64][kBvssStage];
+  BvssOut out{s_stage[threadIdx.x >> 6], 0u};
   const uint64_t total = static_cast<uint64_t>(a.n_entries) * a.nfront;
   for (uint64_t base = static_cast<uint64_t>(blockIdx.x) * blockDim.x; base < total;
        base += static_cast<uint64_t>(gridDim.x) * blockDim.x) {
@@ -105,19 +158,11 @@ __global__ void __launch_bounds__(kBvssBlock) bvss_bitmap_kernel(BvssArgs a) {
         hits = a.masks[e] & a.front[static_cast<size_t>(f) * a.n_int + iv];
       }
     }
-    unsigned wtot = 0;
-    const unsigned off = wave_excl_scan(static_cast<unsigned>(__popcll(hits)), &wtot);
-    unsigned long long wbase = 0;
-    if (__lane_id() == 0 && wtot) wbase = atomicAdd(&a.ctl->count, static_cast<unsigned long long>(wtot));
-    wbase = __shfl(wbase, 0);
-    uint64_t slot = wbase + off;
-    while (hits) {
-      const int bit = __ffsll(static_cast<long long>(hits)) - 1;
-      if (slot < a.cap) a.out[slot] = make_int4(f, iv * 64 + bit, row, 0);
-      ++slot;
-      hits &= hits - 1;
-    }
+    const uint64_t h1[1] = {hits};
+    const int r1[1] = {row};
+    out.emit(a, f, iv, h1, r1);
   }
+  out.flush(a);
 }
 
 // MFMA path: one wave per (tile of 16 rows of a dense interval, group of 16
@@ -126,6 +171,9 @@ __global__ void __launch_bounds__(kBvssBlock) bvss_bitmap_kernel(BvssArgs a) {
 // holds the shared-source counts of rows 4 (l / 16) + i (i = 0..3) with
 // frontier l % 16.
 __global__ void __launch_bounds__(kBvssBlock) bvss_mfma_kernel(BvssArgs a) {
+  __shared__ uint64_t s_stage[kBvssBlock / 64][kBvssStage];
+  BvssOut out{s_stage[threadIdx.x >> 6], 0u};
+  unsigned long long tiles = 0;
   const int lane = __lane_id();
   const int wave = static_cast<int>((blockIdx.x * blockDim.x + threadIdx.x) >> 6);
   const int nwaves = static_cast<int>((gridDim.x * blockDim.x) >> 6);
@@ -149,7 +197,6 @@ __global__ void __launch_bounds__(kBvssBlock) bvss_mfma_kernel(BvssArgs a) {
     // decode: this lane owns rows 4 kg + i with frontier c
     uint64_t hits[4];
     int rowid[4];
-    unsigned cnt = 0;
     const int counts[4] = {acc.x, acc.y, acc.z, acc.w};
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
@@ -160,27 +207,33 @@ __global__ void __launch_bounds__(kBvssBlock) bvss_mfma_kernel(BvssArgs a) {
         hits[i] = a.masks[er] & fword;
         rowid[i] = a.rows[er];
         if (__popcll(hits[i]) != counts[i]) atomicExch(&a.ctl->mismatch, 1);
-        cnt += static_cast<unsigned>(__popcll(hits[i]));
       }
     }
-    unsigned wtot = 0;
-    const unsigned off = wave_excl_scan(cnt, &wtot);
-    unsigned long long wbase = 0;
-    if (lane == 0 && wtot) wbase = atomicAdd(&a.ctl->count, static_cast<unsigned long long>(wtot));
-    wbase = __shfl(wbase, 0);
-    if (lane == 0) atomicAdd(&a.ctl->tiles, 1ull);
-    uint64_t slot = wbase + off;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      uint64_t h = hits[i];
-      while (h) {
-        const int bit = __ffsll(static_cast<long long>(h)) - 1;
-        if (slot < a.cap) a.out[slot] = make_int4(fc, iv * 64 + bit, rowid[i], 0);
-        ++slot;
-        h &= h - 1;
-      }
-    }
+    ++tiles;
+    out.emit(a, fc, iv, hits, rowid);
   }
+  out.flush(a);
+  if (lane == 0 && tiles) atomicAdd(&a.ctl->tiles, tiles);
+}
+
+// Sorted keys into the caller's three arrays.
+__global__ void __launch_bounds__(kBvssBlock) bvss_unpack_kernel(const uint64_t* key, uint64_t n, int vbits, int* of,
+                                                                 int* ou, int* ov) {
+  const uint64_t mask = (1ull << vbits) - 1;
+  for (uint64_t i = static_cast<uint64_t>(blockIdx.x) * blockDim.x + threadIdx.x; i < n;
+       i += static_cast<uint64_t>(gridDim.x) * blockDim.x) {
+    const uint64_t k = key[i];
+    ov[i] = static_cast<int>(k & mask);
+    ou[i] = static_cast<int>((k >> vbits) & mask);
+    of[i] = static_cast<int>(k >> (2 * vbits));
+  }
+}
+
+void launch_bvss_unpack(const uint64_t* key, uint64_t n, int vbits, int* of, int* ou, int* ov, int grid,
+                        hipStream_t s) {
+  if (n == 0) return;
+  hipLaunchKernelGGL(bvss_unpack_kernel, dim3(grid), dim3(kBvssBlock), 0, s, key, n, vbits, of, ou, ov);
+  CPG_HIP(hipGetLastError());
 }
 
 void launch_bvss_discover(const BvssArgs& a, const int* fptr, const int* fsrc, int mode,

@@ -289,7 +289,7 @@ struct cpg_handle {
   DevBuf<unsigned long long> bv_masks, bv_front;
   DevBuf<int2> bv_tiles;
   DevBuf<uint8_t> bv_dense;
-  DevBuf<int4> bv_out;
+  DevBuf<int> bv_out;  // the sorted triples' three columns
   DevBuf<BvssCtl> bv_ctl;
   EventPair ev_bvss;
 
@@ -1292,7 +1292,15 @@ struct cpg_handle {
     const size_t fw = static_cast<size_t>(nfront) * std::max(1, hb.n_int);
     bv_front.reserve(fw);
     CPG_HIP(hipMemsetAsync(bv_front.p, 0, fw * sizeof(unsigned long long), stream));
-    bv_out.reserve(std::max<int64_t>(1, cap));
+    // A triple is one 64-bit key, so that the device sorts it: two vertex ids
+    // and the frontier.  Ids of up to 2^28 leave 8 bits for 256 frontiers, the
+    // frontiers beyond 2^(64 - 2 vbits) are taken in calls of their own.
+    int vbits = 1;
+    while ((1ll << vbits) < g.n) ++vbits;
+    const int fbits = 64 - 2 * vbits;
+    if (fbits < 31 && nfront > (1 << fbits)) return bvss_in_parts(nfront, 1 << fbits, fptr, fsrc, mode, dense_min, of, ou, ov, cap);
+    const size_t room = std::max<int64_t>(1, cap);
+    skey[0].reserve(room); skey[1].reserve(room);
     bv_ctl.reserve(1);
     CPG_HIP(hipMemsetAsync(bv_ctl.p, 0, sizeof(BvssCtl), stream));
     BvssArgs a{};
@@ -1300,7 +1308,7 @@ struct cpg_handle {
     a.n_tiles = static_cast<int>(hb.tiles.size()); a.nfront = nfront;
     a.int_ptr = bv_int_ptr.p; a.rows = bv_rows.p; a.entry_int = bv_entry_int.p;
     a.masks = bv_masks.p; a.tiles = bv_tiles.p; a.front = bv_front.p; a.dense = bv_dense.p;
-    a.out = bv_out.p; a.cap = static_cast<uint64_t>(cap); a.ctl = bv_ctl.p;
+    a.keys = skey[0].p; a.vbits = vbits; a.cap = static_cast<uint64_t>(cap); a.ctl = bv_ctl.p;
     ev_bvss.create();
     CPG_HIP(hipEventRecord(ev_bvss.a, stream));
     launch_bvss_discover(a, bv_fptr.p, bv_fsrc.p, mode, dense_min, grid, stream);
@@ -1313,20 +1321,48 @@ struct cpg_handle {
     if (c.mismatch) throw std::runtime_error("BVSS MFMA count disagrees with the decoded words");
     const uint64_t cnt = c.count;
     if (cnt > static_cast<uint64_t>(cap)) return -static_cast<int64_t>(cnt) - 1000;
-    std::vector<int4> t(cnt);
-    d2h(t.data(), bv_out.p, cnt, stream);
+    // ordered by (f, u, v): the keys' used bytes
+    int used = 2 * vbits;
+    while (used < 64 && (1ll << (used - 2 * vbits)) < nfront) ++used;
+    int bytes[8];
+    const int nbytes = (used + 7) / 8;
+    for (int b = 0; b < nbytes; ++b) bytes[b] = b;
+    ghist.reserve(sort_ghist_len(cnt));
+    SortBufs sb{{skey[0].p, skey[1].p}, {nullptr, nullptr}, ghist.p, cnt};
+    const int res = radix_sort_pairs(sb, cnt, bytes, nbytes, stream);
+    bv_out.reserve(3 * std::max<uint64_t>(1, cnt));
+    launch_bvss_unpack(skey[res].p, cnt, vbits, bv_out.p, bv_out.p + cnt, bv_out.p + 2 * cnt, grid, stream);
+    if (of) d2h(of, bv_out.p, cnt, stream);
+    if (ou) d2h(ou, bv_out.p + cnt, cnt, stream);
+    if (ov) d2h(ov, bv_out.p + 2 * cnt, cnt, stream);
     CPG_HIP(hipStreamSynchronize(stream));
-    std::sort(t.begin(), t.end(), [](const int4& x, const int4& y) {
-      if (x.x != y.x) return x.x < y.x;
-      if (x.y != y.y) return x.y < y.y;
-      return x.z < y.z;
-    });
-    for (uint64_t i = 0; i < cnt; ++i) {
-      if (of) of[i] = t[i].x;
-      if (ou) ou[i] = t[i].y;
-      if (ov) ov[i] = t[i].z;
-    }
     return static_cast<int64_t>(cnt);
+  }
+
+  // Discovery for more frontiers than one key holds: parts of `per`
+  // frontiers, each part's triples after the last's (f ascends over parts).
+  int64_t bvss_in_parts(int nfront, int per, const int* fptr, const int* fsrc, int mode, int dense_min, int* of,
+                        int* ou, int* ov, int64_t cap) {
+    int64_t total = 0;
+    double ms = 0.0;
+    int64_t tiles = 0;
+    for (int f0 = 0; f0 < nfront; f0 += per) {
+      const int nf = std::min(per, nfront - f0);
+      std::vector<int> ptr(fptr + f0, fptr + f0 + nf + 1);
+      for (int& p : ptr) p -= fptr[f0];
+      const int64_t left = std::max<int64_t>(0, cap - total);
+      const int64_t at = std::min(total, cap);
+      const int64_t got = bvss_discover(nf, ptr.data(), fsrc + fptr[f0], mode, dense_min, of ? of + at : nullptr,
+                                        ou ? ou + at : nullptr, ov ? ov + at : nullptr, left);
+      const int64_t cnt = got < 0 ? -got - 1000 : got;
+      for (int64_t i = 0; got > 0 && of && i < cnt; ++i) of[at + i] += f0;
+      total += cnt;
+      ms += timing.bvss_ms;
+      tiles += timing.bvss_tiles;
+    }
+    timing.bvss_ms = ms;
+    timing.bvss_tiles = tiles;
+    return total > cap ? -total - 1000 : total;
   }
 
   void fetch_succ() {

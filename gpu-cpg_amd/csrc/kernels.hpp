@@ -333,7 +333,8 @@ struct BvssArgs {
   const int2* tiles;          // {interval, first entry}
   unsigned long long* front;  // nfront x n_int frontier words (zeroed by the caller)
   uint8_t* dense;             // n_int: interval takes the MFMA path
-  int4* out;                  // {frontier, u, v, 0} triples
+  uint64_t* keys;             // triples as (frontier << vbits | u) << vbits | v
+  int vbits;                  // bits of a vertex id
   uint64_t cap;
   BvssCtl* ctl;
 };
@@ -343,8 +344,12 @@ struct BvssArgs {
 void launch_bvss_discover(const BvssArgs& a, const int* fptr, const int* fsrc, int mode,
                           int dense_min, int grid, hipStream_t s);
 
+void launch_bvss_unpack(const uint64_t* key, uint64_t n, int vbits, int* of, int* ou, int* ov, int grid,
+                        hipStream_t s);
+
 // ---------------- final selection ----------------
-// Stable LSD radix sort of (key, value) pairs over the given key bytes.
+// Stable LSD radix sort of (key, value) pairs over the given key bytes (keys
+// alone where the value buffers are null).
 struct SortBufs {
   uint64_t* key[2];
   uint32_t* val[2];

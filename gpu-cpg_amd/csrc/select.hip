@@ -154,7 +154,7 @@ __global__ void __launch_bounds__(kSortBlock) sort_scatter_kernel(const uint64_t
     unsigned d = 0;
     if (act) {
       k = kin[i];
-      v = vin[i];
+      if (vin) v = vin[i];
       d = static_cast<unsigned>(k >> shift) & 255u;
     }
     uint64_t peers = __ballot(act);
@@ -170,7 +170,7 @@ __global__ void __launch_bounds__(kSortBlock) sort_scatter_kernel(const uint64_t
       for (int w = 0; w < wave; ++w) off += wcnt[w][d];
       const uint64_t dst = static_cast<uint64_t>(base[d]) + off;
       kout[dst] = k;
-      vout[dst] = v;
+      if (vin) vout[dst] = v;
     }
     __syncthreads();
     unsigned tot = 0;

@@ -161,6 +161,28 @@ void pick_roots(const std::vector<int>& sd, bool quirk, float perc, std::vector<
     if (kp[i]) minc = std::min(minc, static_cast<float>(sd[i]) / static_cast<float>(kScaleUp));
 }
 
+// Distance of the first trial bound from the cheapest root: the roots' 10th
+// percentile cost (of an evenly strided sample of about 2048), which only
+// sets the width, and at least a 256th of the costs' magnitude.
+double first_gap(const std::vector<float>& rc, float cmin, float max_abs_distf) {
+  const size_t step = std::max<size_t>(1, rc.size() / 2048);
+  std::vector<float> sample;
+  sample.reserve(rc.size() / step + 1);
+  for (size_t i = 0; i < rc.size(); i += step) sample.push_back(rc[i]);
+  std::nth_element(sample.begin(), sample.begin() + static_cast<std::ptrdiff_t>(sample.size() / 10), sample.end());
+  const float p10 = sample[sample.size() / 10];
+  return std::max({static_cast<double>(p10) - static_cast<double>(cmin),
+                   std::fabs(static_cast<double>(cmin)) * 0x1p-8, static_cast<double>(max_abs_distf) * 0x1p-8, 1e-6});
+}
+
+// A multi-query slot's first trial bound (see mq.hip).
+void start_trial(MqQuery& m, const std::vector<float>& rc, float cmin, float max_abs_distf) {
+  m.trial = 1;
+  m.cmin = cmin;
+  m.gap = first_gap(rc, cmin, max_abs_distf);
+  m.ukey = float_key(static_cast<float>(static_cast<double>(cmin) + m.gap));
+}
+
 // A pair of HIP events bracketing work on one stream.
 struct EventPair {
   hipEvent_t a = nullptr, b = nullptr;
@@ -794,18 +816,8 @@ struct cpg_handle {
     const double tb0 = now_ms();
     const uint64_t nb = rc.size();
     launch_iota(batch.p, nb, grid, stream);
-    // the roots' 10th-percentile cost, which only sets the first trial's
-    // width: from an evenly strided sample of about 2048 roots
-    const size_t step = std::max<size_t>(1, rc.size() / 2048);
-    std::vector<float> sample;
-    sample.reserve(rc.size() / step + 1);
-    for (size_t i = 0; i < rc.size(); i += step) sample.push_back(rc[i]);
-    std::nth_element(sample.begin(), sample.begin() + static_cast<std::ptrdiff_t>(sample.size() / 10), sample.end());
-    const float p10 = sample[sample.size() / 10];
+    double gap = first_gap(rc, cmin, max_abs_distf);
     if (trace) std::fprintf(stderr, "probe: host preparation %.3f ms\n", now_ms() - tb0);
-    double gap = static_cast<double>(p10) - static_cast<double>(cmin);
-    gap = std::max({gap, std::fabs(static_cast<double>(cmin)) * 0x1p-8,
-                    static_cast<double>(max_abs_distf) * 0x1p-8, 1e-6});
     uint64_t prev_total = 0;
     double prev_gap = gap;
     wa.strict = 0;  // a trial keeps the children at the trial bound itself
@@ -1576,7 +1588,13 @@ struct cpg_batch {
       m = MqQuery{};
       m.ukey = kKeyInf;
       m.klo = cnt ? float_key(minc) : 0u;
-      m.shift = window_shift_bins(m.klo, kKeyInf, kMqBins);
+      if (cnt) {
+        std::vector<float> rc;
+        for (size_t i = 0; i < nr; ++i)
+          if (keep[i]) rc.push_back(rcost[q][i]);
+        start_trial(m, rc, minc, uh.max_abs_distf);
+      }
+      m.shift = window_shift_bins(m.klo, m.ukey, kMqBins);
       m.k = static_cast<unsigned long long>(std::max<int64_t>(0, designs[q].k));
       m.batch_target = std::max<unsigned long long>(
           256, m.k / static_cast<unsigned long long>(std::max(1, tune.target_div[k_class(m.k)])));
@@ -1606,11 +1624,11 @@ struct cpg_batch {
       for (int r = 0;; ++r) {
         if (r > 100000) throw std::runtime_error("batched PFXT round limit exceeded");
         if (now_ms() - t0 > CPG_QUERY_LIMIT_MS) throw std::runtime_error("batched query exceeded its time limit");
-        // round 0 expands every root; later rounds replay the captured round
+        // round 0 runs as it is; later rounds replay the captured round
         const int group = r == 0 ? 1 : std::max(1, tune.group);
         const int rgrid = std::max(1, uh.grid / 8 * std::max(1, tune.grid_mult));
         if (r == 0) {
-          launch_mq_round(a, true, rgrid, stream);
+          launch_mq_round(a, false, rgrid, stream);
         } else {
           // the captured round holds buffer addresses and sizes: capture
           // again whenever any of them changed (node store growth, designs
@@ -1959,9 +1977,9 @@ struct cpg_server {
     // where the roots' chains are short (the single query's rule for
     // skipping its probe); otherwise the probe finds a tight bound.
     const bool short_chains = nkept * (static_cast<int64_t>(h.diameter) + 1) <= (int64_t(1) << 20);
-    const bool roots_bound = q.k > 0 && static_cast<int64_t>(rc.size()) >= q.k && short_chains;
-    if (roots_bound) {
-      std::nth_element(rc.begin(), rc.begin() + (q.k - 1), rc.end());
+    bool trial = false;
+    // the roots in the graph handle's node store, for admission to copy
+    auto seed_roots = [&]() {
       const uint64_t cap = std::max<uint64_t>(uint64_t(1) << 16, static_cast<uint64_t>(nkept));
       h.ensure_pfxt_buffers(std::max<uint64_t>(cap, h.node_cap));
       PfxtCtl init{};
@@ -1971,55 +1989,30 @@ struct cpg_server {
       h.keep.reserve(std::max(1, nsrc));
       h2d(h.keep.p, kp.data(), nsrc, h.stream);
       launch_roots(h.srcs.p, h.keep.p, nsrc, aq.dist, aq.distf, h.node_store(), h.pctl.p, h.stream);
-      PfxtCtl pc = h.read_pctl();
+      q.seed_n = h.read_pctl().node_n;
+    };
+    const bool roots_bound = q.k > 0 && static_cast<int64_t>(rc.size()) >= q.k && short_chains;
+    if (roots_bound) {
+      std::nth_element(rc.begin(), rc.begin() + (q.k - 1), rc.end());
+      seed_roots();
       u0 = float_key(rc[q.k - 1]);
-      q.seed_n = pc.node_n;
       std::lock_guard<std::mutex> lk(stats_mu);
       stats.root_bounds++;
     } else if (nkept > 0 && q.k > 0) {
-      uint64_t cap = std::min<uint64_t>(
-          std::max<uint64_t>(uint64_t(1) << 22, 16ull * static_cast<uint64_t>(q.k) + nkept + (1u << 20)),
-          0x7fffffffull);
-      // a probe whose trial bound's children fill the handle's store runs
-      // again in a larger one: without a bound the first round would expand
-      // every root under a coarse bound and store far more
-      for (int attempt = 0;; ++attempt) {
-        h.ensure_pfxt_buffers(cap);
-        PfxtCtl init{};
-        init.ukey = kKeyInf;
-        init.klo = klo;
-        init.shift = window_shift(klo, kKeyInf);
-        init.node_cap = cap;
-        h2d(h.pctl.p, &init, 1, h.stream);
-        h.keep.reserve(std::max(1, nsrc));
-        h2d(h.keep.p, kp.data(), nsrc, h.stream);
-        launch_roots(h.srcs.p, h.keep.p, nsrc, aq.dist, aq.distf, h.node_store(), h.pctl.p, h.stream);
-        WalkArgs wa{};
-        wa.vrec = aq.vrec; wa.devinfo = aq.devinfo; wa.devs = aq.devs; wa.batch = h.batch.p;
-        wa.nodes = h.node_store(); wa.ckeys = h.ckeys.p; wa.ckeys_cap = cap; wa.ctl = h.pctl.p;
-        wa.max_abs_distf = max_abs_distf; wa.max_abs_wgt = h.g.max_abs_wgt;
-        wa.step_limit = h.step_limit();
-        const double tp = now_ms();
-        u0 = h.probe_bound(wa, q.k, kp, sd, minc, klo, false);
-        {
-          std::lock_guard<std::mutex> lk(stats_mu);
-          stats.probe_ms += now_ms() - tp;
-          if (trace_on())
-            std::fprintf(stderr, "served t %.2f probe query %lld graph %d k %lld trials %d ms %.2f\n", now_ms(),
-                         static_cast<long long>(q.id), q.graph, static_cast<long long>(q.k), h.timing.probes,
-                         now_ms() - tp);
-        }
-        PfxtCtl pc = h.read_pctl();
-        if (pc.err) throw std::runtime_error("PFXT walk exceeded its step bound");
-        q.seed_n = std::min<uint64_t>(pc.node_n, cap);
-        if (!(u0 == kKeyInf && h.probe_overflowed) || attempt >= 4 || cap >= 0x7fffffffull) break;
-        cap = std::min<uint64_t>(cap * 2, 0x7fffffffull);
-      }
+      // roots alone, with a trial bound: the shared rounds find the first one
+      trial = true;
+      seed_roots();
     }
     MqQuery m{};
     m.ukey = u0;
     m.klo = klo;
-    m.shift = window_shift_bins(m.klo, u0, kMqBins);
+    if (trial) {
+      std::vector<float> roots;  // zero-cost ones too
+      for (int i = 0; i < nsrc; ++i)
+        if (kp[i]) roots.push_back(static_cast<float>(sd[i]) / static_cast<float>(kScaleUp));
+      start_trial(m, roots, minc, max_abs_distf);
+    }
+    m.shift = window_shift_bins(m.klo, m.ukey, kMqBins);
     m.k = static_cast<unsigned long long>(q.k);
     m.batch_target = std::max<unsigned long long>(256, m.k / 8);
     m.done = (nkept == 0 || q.k == 0) ? 1 : 0;
@@ -2028,7 +2021,6 @@ struct cpg_server {
     m.devs = aq.devs;
     m.mag = 2.0f * max_abs_distf + h.g.max_abs_wgt + 1.0f;
     m.step_limit = h.step_limit();
-    m.all = u0 == kKeyInf ? 1 : 0;
     q.init = m;
   }
 

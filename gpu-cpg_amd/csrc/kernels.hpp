@@ -259,7 +259,15 @@ struct MqQuery {
   float mag;                      // 2 max|distf| + max|w| + 1 (walk slack)
   int step_limit;                 // bound on one walk's steps
   int all;                        // the next round expands every unexpanded path
-  int pad;
+  // Trial of a first bound (see mq.hip): its number (0: the bound stands),
+  // the smallest root cost, the bound's distance from it, and the last
+  // trial's distance and path count
+  int trial;
+  int retry;                      // this round's trial fell short: nothing is stored
+  float cmin;
+  double gap;
+  double prev_gap;
+  unsigned long long prev_total;
   unsigned long long stored;      // children the fill passes stored for this query
 };
 

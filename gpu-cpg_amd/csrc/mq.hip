@@ -18,6 +18,13 @@
 //      at memory),
 //   5. a fill pass storing its children <= U_q (inclusive: the counted
 //      children at U_q are needed).
+// A query starts with its roots and a trial bound a little above the
+// cheapest (the single query's probe, without its host round trips): a round
+// counts the children of the roots under the trial bound, and if the roots
+// and they are fewer than K_q it stores nothing, puts the roots back and
+// widens the bound for the next round.  Without a first bound round 0 walks
+// every root's whole chain: on a batch of 48 designs the first two rounds
+// took 49 ms counting and 11 ms storing of a 67-76 ms run.
 // The per-query semantics equal the single-query rounds' (see pfxt.hip);
 // the final selection sorts (query, cost, level) so each query's K_q
 // results are contiguous.
@@ -130,7 +137,7 @@ __global__ void __launch_bounds__(kMqSelBlock) mq_select_batch_kernel(MqArgs a, 
   if (qs->done) return;
   const unsigned* h = a.hist + static_cast<size_t>(q) * kMqHistStride;
   unsigned long long total = 0;
-  const bool take_all = all || qs->all;
+  const bool take_all = all || qs->all || qs->trial;
   const uint32_t b = mq_crossing(h + kMqBins, take_all ? ~0ull : qs->batch_target, &total);
   if (threadIdx.x == 0) {
     qs->all = 0;
@@ -147,21 +154,34 @@ __global__ void __launch_bounds__(kMqSelBlock) mq_select_batch_kernel(MqArgs a, 
   }
 }
 
+// A block takes tiles of eight slots per thread and reserves a tile's batch
+// entries with one atomic (one address for the whole grid).
 __global__ void __launch_bounds__(kMqBlock) mq_make_batch_kernel(MqArgs a) {
   const uint64_t n = a.ctl->node_n < a.nodes.cap ? a.ctl->node_n : a.nodes.cap;
-  for (uint64_t base = static_cast<uint64_t>(blockIdx.x) * blockDim.x; base < n;
-       base += static_cast<uint64_t>(gridDim.x) * blockDim.x) {
-    const uint64_t i = base + threadIdx.x;
-    bool take = false;
-    if (i < n && a.nodes.flag[i] == 0) {
-      const MqQuery qs = a.qs[a.nq[i]];
+  constexpr int kPer = 8;
+  constexpr uint64_t kTile = static_cast<uint64_t>(kMqBlock) * kPer;
+  for (uint64_t base = static_cast<uint64_t>(blockIdx.x) * kTile; base < n;
+       base += static_cast<uint64_t>(gridDim.x) * kTile) {
+    const uint64_t i0 = base + threadIdx.x;
+    unsigned mask = 0, cnt = 0;
+#pragma unroll
+    for (int j = 0; j < kPer; ++j) {
+      const uint64_t i = i0 + static_cast<uint64_t>(j) * kMqBlock;
+      if (i >= n || a.nodes.flag[i] != 0) continue;
+      const MqQuery& qs = a.qs[a.nq[i]];
       const uint32_t k = a.nodes.key[i];
-      take = !qs.done && k <= qs.thkey && k < qs.ukey;
+      if (!qs.done && k <= qs.thkey && k < qs.ukey) {
+        mask |= 1u << j;
+        ++cnt;
+      }
     }
-    const uint64_t slot = wave_reserve(&a.ctl->batch_n, take);
-    if (take) {
+    uint64_t slot = block_reserve<kMqBlock>(&a.ctl->batch_n, cnt);
+#pragma unroll
+    for (int j = 0; j < kPer; ++j) {
+      if (!(mask & (1u << j))) continue;
+      const uint64_t i = i0 + static_cast<uint64_t>(j) * kMqBlock;
       a.nodes.flag[i] = 1;
-      a.batch[slot] = static_cast<uint32_t>(i);
+      a.batch[slot++] = static_cast<uint32_t>(i);
     }
   }
 }
@@ -174,13 +194,47 @@ __global__ void __launch_bounds__(kMqBlock) mq_make_batch_kernel(MqArgs a) {
 // consecutive batch entries mostly belong to one query (a parent's
 // children are stored together), and every global atomic is performed at
 // memory.  Parents of other queries count with global atomics.
+// In the fill pass a wave stages its children in LDS and stores them with
+// one atomic on node_n per kMqStage of them (one address for the whole grid:
+// an atomic per wave step bound the pass).
+constexpr int kMqStage = 256;
 template <bool kFill>
 __global__ void __launch_bounds__(kMqBlock) mq_walk_kernel(MqArgs a) {
-  __shared__ unsigned s_h[kMqBins];
+  __shared__ unsigned s_h[kFill ? 1 : kMqBins];
   __shared__ int s_q;
+  constexpr int kW = kMqBlock / 64, kS = kFill ? kMqStage : 1;
+  __shared__ float s_cost[kW][kS];
+  __shared__ int s_to[kW][kS], s_from[kW][kS], s_parent[kW][kS], s_level[kW][kS], s_nq[kW][kS];
+  const int wave = static_cast<int>(threadIdx.x) >> 6, lane = __lane_id();
+  int staged = 0;  // wave-uniform
   MqCtl* ctl = a.ctl;
   const uint64_t nb = ctl->batch_n;
   unsigned long long hops = 0, devv = 0, nonmono = 0;
+  auto flush = [&]() {
+    if (staged == 0) return;
+    __builtin_amdgcn_wave_barrier();
+    unsigned long long base = 0;
+    if (lane == 0) base = atomicAdd(&ctl->node_n, static_cast<unsigned long long>(staged));
+    base = __shfl(base, 0);
+    for (int j = lane; j < staged; j += 64) {
+      const uint64_t slot = base + static_cast<uint64_t>(j);
+      if (slot >= a.nodes.cap) {
+        atomicExch(&ctl->overflow, 1);
+        continue;
+      }
+      const float cost = s_cost[wave][j];
+      a.nodes.cost[slot] = cost;
+      a.nodes.to[slot] = s_to[wave][j];
+      a.nodes.from[slot] = s_from[wave][j];
+      a.nodes.parent[slot] = s_parent[wave][j];
+      a.nodes.level[slot] = s_level[wave][j];
+      a.nodes.key[slot] = float_key(cost);
+      a.nodes.flag[slot] = 0;
+      a.nq[slot] = s_nq[wave][j];
+    }
+    __builtin_amdgcn_wave_barrier();
+    staged = 0;
+  };
   for (uint64_t base = static_cast<uint64_t>(blockIdx.x) * blockDim.x; base < nb;
        base += static_cast<uint64_t>(gridDim.x) * blockDim.x) {  // block-uniform
     if (!kFill) {
@@ -201,9 +255,11 @@ __global__ void __launch_bounds__(kMqBlock) mq_walk_kernel(MqArgs a) {
       q = a.nq[p];
       qs = a.qs[q];
     }
+    const bool back = kFill && i < nb && qs.retry;  // a trial that fell short
+    if (back) a.nodes.flag[p] = 0;
     const float U = key_float(qs.ukey);
     ChainWalk w;
-    w.start(i < nb, c, to, U, qs.ukey != kKeyInf, qs.mag);
+    w.start(i < nb && !back, c, to, U, qs.ukey != kKeyInf, qs.mag);
     unsigned* h = a.hist + static_cast<size_t>(q) * kMqHistStride;
     const bool local = !kFill && q == s_q;  // count in the block's LDS histogram
     unsigned stored = 0;  // fill: children this lane stored for its parent
@@ -223,21 +279,21 @@ __global__ void __launch_bounds__(kMqBlock) mq_walk_kernel(MqArgs a) {
         }
         continue;
       }
-      const uint64_t slot = wave_reserve(&ctl->node_n, emit);
-      if (emit) {
-        if (slot < a.nodes.cap) {
-          a.nodes.cost[slot] = cc;
-          a.nodes.to[slot] = cw;
-          a.nodes.from[slot] = from;
-          a.nodes.parent[slot] = p;
-          a.nodes.level[slot] = lvl + 1;
-          a.nodes.key[slot] = float_key(cc);
-          a.nodes.flag[slot] = 0;
-          a.nq[slot] = q;
+      const uint64_t m = __ballot(emit);
+      if (m) {
+        const int add = static_cast<int>(__popcll(m));
+        if (staged + add > kS) flush();
+        if (emit) {
+          const int j = staged + static_cast<int>(__popcll(m & lanemask_lt()));
+          s_cost[wave][j] = cc;
+          s_to[wave][j] = cw;
+          s_from[wave][j] = from;
+          s_parent[wave][j] = p;
+          s_level[wave][j] = lvl + 1;
+          s_nq[wave][j] = q;
           ++stored;
-        } else {
-          atomicExch(&ctl->overflow, 1);
         }
+        staged += add;
       }
     }
     if (kFill) {
@@ -264,10 +320,39 @@ __global__ void __launch_bounds__(kMqBlock) mq_walk_kernel(MqArgs a) {
       __syncthreads();  // s_h and s_q are set again for the next step
     }
   }
+  if (kFill) flush();
   (void)hops;
   (void)devv;
   for (int o = 32; o > 0; o >>= 1) nonmono += __shfl_xor(nonmono, o);
   if (kFill && __lane_id() == 0 && nonmono) atomicAdd(&ctl->nonmono, nonmono);  // once per expansion
+}
+
+// Next bound of a query whose trial found too few paths (total < K_q).
+// Counts grow steeply with the bound: model total ~ gap^alpha, alpha fitted
+// to the last two trials (4 at first), aim 10% past K_q and widen by at most
+// 4x (a trial that is too wide stores nothing more, it only counts more).
+// Past every distance without a new path, or after kMqTrials, the query
+// goes on unbounded, all its roots at once.
+constexpr int kMqTrials = 16;
+__device__ inline void mq_widen(MqQuery* qs, unsigned long long total) {
+  const double gap = qs->gap;
+  qs->retry = 1;
+  if (qs->trial >= kMqTrials || (gap > static_cast<double>(qs->mag) && total == qs->prev_total)) {
+    qs->trial = 0;
+    qs->all = 1;
+    qs->ukey = kKeyInf;
+    return;
+  }
+  double alpha = 4.0;
+  if (qs->trial > 1 && qs->prev_total > 0 && total > qs->prev_total)
+    alpha = fmin(8.0, fmax(1.0, log(static_cast<double>(total) / static_cast<double>(qs->prev_total)) /
+                                    log(gap / qs->prev_gap)));
+  const double f = pow(static_cast<double>(qs->k) / static_cast<double>(total > 0 ? total : 1ull), 1.0 / alpha) * 1.1;
+  qs->prev_total = total;
+  qs->prev_gap = gap;
+  qs->gap = gap * fmin(4.0, fmax(1.25, f));
+  qs->trial += 1;
+  qs->ukey = float_key(static_cast<float>(static_cast<double>(qs->cmin) + qs->gap));
 }
 
 // One block per query: U_q = the upper edge of the bin where the running
@@ -280,13 +365,17 @@ __global__ void __launch_bounds__(kMqSelBlock) mq_select_bound_kernel(MqArgs a) 
   unsigned long long total = 0;
   const uint32_t b = mq_crossing(h, qs->k, &total);
   if (threadIdx.x == 0) {
+    qs->retry = 0;
     uint32_t uk = qs->ukey;
     if (b < static_cast<uint32_t>(kMqBins)) {
       const uint64_t up = static_cast<uint64_t>(qs->klo) + ((static_cast<uint64_t>(b) + 1) << qs->shift) - 1;
       if (up < uk) uk = static_cast<uint32_t>(up);
+      qs->ukey = uk;
+      qs->trial = 0;
+    } else if (qs->trial) {
+      mq_widen(qs, total);
     }
-    qs->ukey = uk;
-    qs->shift = mq_shift(qs->klo, uk);
+    qs->shift = mq_shift(qs->klo, qs->ukey);
     qs->rounds += 1;
   }
 }
@@ -294,39 +383,69 @@ __global__ void __launch_bounds__(kMqSelBlock) mq_select_bound_kernel(MqArgs a) 
 // Sort input: each stored path with a nonzero key <= its query's bound as
 // (query << 48 | key << 16 | level) -> node, for the queries sel marks
 // (every query when sel is null).
+// Blocks take tiles of eight slots per thread, one atomic per tile on the
+// path count; the queries' counts gather in LDS while there are at most
+// kMqLdsQ of them (a wave's taken nodes of one query add together).
+constexpr int kMqLdsQ = 1024;
 __global__ void __launch_bounds__(kMqBlock) mq_build_keys_kernel(MqArgs a, const uint8_t* sel,
                                                                  uint64_t* key, uint32_t* val,
                                                                  unsigned long long* count,
                                                                  unsigned long long* per_q) {
+  __shared__ unsigned s_cnt[kMqLdsQ];
+  const bool lds = a.nq_count <= kMqLdsQ;
+  for (int j = threadIdx.x; j < kMqLdsQ; j += blockDim.x) s_cnt[j] = 0;
+  __syncthreads();
   const uint64_t n = a.ctl->node_n < a.nodes.cap ? a.ctl->node_n : a.nodes.cap;
-  for (uint64_t base = static_cast<uint64_t>(blockIdx.x) * blockDim.x; base < n;
-       base += static_cast<uint64_t>(gridDim.x) * blockDim.x) {
-    const uint64_t i = base + threadIdx.x;
-    bool take = false;
-    uint32_t k = 0;
-    int q = 0;
-    if (i < n) {
-      q = a.nq[i];
-      k = a.nodes.key[i];
-      take = (!sel || sel[q]) && k <= a.qs[q].ukey && !key_is_zero(k);
+  constexpr int kPer = 8;
+  constexpr uint64_t kTile = static_cast<uint64_t>(kMqBlock) * kPer;
+  for (uint64_t base = static_cast<uint64_t>(blockIdx.x) * kTile; base < n;
+       base += static_cast<uint64_t>(gridDim.x) * kTile) {
+    const uint64_t i0 = base + threadIdx.x;
+    unsigned mask = 0, cnt = 0;
+    uint32_t ks[kPer];
+    int qv[kPer];
+#pragma unroll
+    for (int j = 0; j < kPer; ++j) {
+      const uint64_t i = i0 + static_cast<uint64_t>(j) * kMqBlock;
+      ks[j] = 0;
+      qv[j] = 0;
+      bool take = false;
+      if (i < n) {
+        qv[j] = a.nq[i];
+        ks[j] = a.nodes.key[i];
+        take = (!sel || sel[qv[j]]) && ks[j] <= a.qs[qv[j]].ukey && !key_is_zero(ks[j]);
+      }
+      if (take) {
+        mask |= 1u << j;
+        ++cnt;
+      }
+      uint64_t pend = __ballot(take);
+      while (pend) {
+        const int leader = __ffsll(static_cast<long long>(pend)) - 1;
+        const int lq = __shfl(qv[j], leader);
+        const uint64_t peers = __ballot(take && qv[j] == lq);
+        if (__lane_id() == leader) {
+          if (lds) atomicAdd(&s_cnt[lq], static_cast<unsigned>(__popcll(peers)));
+          else atomicAdd(&per_q[lq], static_cast<unsigned long long>(__popcll(peers)));
+        }
+        pend &= ~peers;
+      }
     }
-    const uint64_t slot = wave_reserve(count, take);
-    if (take) {
-      key[slot] = (static_cast<uint64_t>(q) << 48) | (static_cast<uint64_t>(k) << 16) |
+    uint64_t slot = block_reserve<kMqBlock>(count, cnt);
+#pragma unroll
+    for (int j = 0; j < kPer; ++j) {
+      if (!(mask & (1u << j))) continue;
+      const uint64_t i = i0 + static_cast<uint64_t>(j) * kMqBlock;
+      key[slot] = (static_cast<uint64_t>(qv[j]) << 48) | (static_cast<uint64_t>(ks[j]) << 16) |
                   static_cast<uint32_t>(a.nodes.level[i] & 0xffff);
       val[slot] = static_cast<uint32_t>(i);
-    }
-    // per-query counts: one atomic per distinct query among the wave's
-    // taken lanes (consecutive nodes mostly share a query)
-    uint64_t pend = __ballot(take);
-    while (pend) {
-      const int leader = __ffsll(static_cast<long long>(pend)) - 1;
-      const int lq = __shfl(q, leader);
-      const uint64_t peers = __ballot(take && q == lq);
-      if (__lane_id() == leader) atomicAdd(&per_q[lq], static_cast<unsigned long long>(__popcll(peers)));
-      pend &= ~peers;
+      ++slot;
     }
   }
+  __syncthreads();
+  if (lds)
+    for (int j = threadIdx.x; j < a.nq_count; j += blockDim.x)
+      if (s_cnt[j]) atomicAdd(&per_q[j], static_cast<unsigned long long>(s_cnt[j]));
 }
 
 // Compaction of the shared node store (served queries): a node is live

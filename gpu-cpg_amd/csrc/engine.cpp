@@ -988,6 +988,7 @@ struct cpg_handle {
       wa.max_abs_distf = max_abs_distf; wa.max_abs_wgt = g.max_abs_wgt;
       wa.collect_stats = o.collect_stats;
       wa.step_limit = step_limit();
+      wa.lanes = g.m < 3 * static_cast<int64_t>(g.n) ? 2 : 4;
       const int64_t nkept = nroots - dropped;
       const bool probe = nkept > 0 && (o.bound_probe > 0 ||
                                        (o.bound_probe == 0 && nkept * (diameter + 1) > (1 << 20)));

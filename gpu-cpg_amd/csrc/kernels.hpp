@@ -211,6 +211,7 @@ struct WalkArgs {
   int collect_stats;
   int strict;             // emit children with cost < U (rounds) or <= U (bound probe)
   int step_limit;         // bound on one walk's steps: (levels + 2) * (max out-degree + 2)
+  int lanes;              // lanes per parent: 2 or 4 (see launch_walk)
 };
 
 void launch_roots(const int* srcs, const uint8_t* keep, int nsrc, const int* dist,

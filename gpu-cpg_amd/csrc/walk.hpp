@@ -1,4 +1,4 @@
-// One lane's walk over a parent path's suffix chain: the enumeration of
+// A walk over a parent path's suffix chain: the enumeration of
 // the parent's children shared by the single-query and multi-query PFXT.
 //
 // A child of a parent with cost c takes one deviation edge u->w at a vertex
@@ -16,83 +16,102 @@
 
 namespace cpg {
 
+// kLanes lanes walk one parent's chain together.  The walk is bound by the
+// latency of its dependent loads, so a step makes one round trip do all it
+// can: a vertex's record and deviation range were loaded in the step before,
+// and a step loads up to kLanes of its deviations, one per lane, beside the
+// next chain vertex's record and range (known from this one's).  A lane of
+// its own per parent took a trip for the record, one per deviation and one
+// for the deviation past the bound, on a quarter of the waves.
+template <int kLanes>
 struct ChainWalk {
-  int mode;   // 0: at a chain vertex, 1: scanning its deviations, 2: done
-  int v, j, je, sv, steps;
-  float c, X, dv;
+  int4 r;        // record of the chain vertex v: {min delta, nsv, succ, distf}
+  int2 di;       // its deviations {first, count}
+  int4 nr;       // the next chain vertex's, loaded while v's deviations are scanned
+  int2 ndi;
+  int v, nv;
+  int j, je;     // deviations of v still to scan
+  int steps;
+  bool alive, scan;
+  float c, X;
 
   // mag = 2 max|distf| + max|w| + 1 (a bound on the terms' magnitudes).
-  __device__ inline void start(bool active, float cost, int to, float U, bool bounded, float mag) {
-    mode = active && to != -1 ? 0 : 2;
+  __device__ inline void start(bool active, float cost, int to, float U, bool bounded, float mag, const int4* vrec,
+                               const int2* devinfo) {
     v = to;
-    j = je = 0;
-    sv = -1;
+    alive = active && to != -1;
+    scan = false;
     steps = 0;
+    j = je = 0;
+    nv = -1;
     c = cost;
     X = bounded ? (U - cost) + ldexpf(fabsf(U) + fabsf(cost) + mag, -17) : __builtin_huge_valf();
-    dv = 0.0f;
+    r = nr = make_int4(0, -1, -1, 0);
+    di = ndi = make_int2(0, 0);
+    if (alive) {
+      r = vrec[v];
+      di = devinfo[v];
+    }
   }
 
-  // One step.  Returns true when it found a child with cost < U (cost <= U
-  // when !strict); *cc, *cw and *from receive its cost, its deviation head
-  // w and the deviation vertex u.  A walk visits each chain vertex and each
-  // deviation at most once, so more than step_limit steps means a corrupt
-  // index: the walk stops and *err is raised.  *nonmono counts the children
-  // whose binary32 cost comes out below the parent's (a deviation whose
-  // int-scaled delta is 0, or a negative weight): where one sits at the
-  // bound, a path just below U can descend from a parent at or above U,
-  // which is never expanded.
+  // One step, by all lanes of the wave together.  Returns true on a lane that
+  // found a child with cost < U (cost <= U when !strict); *cc, *cw and *from
+  // receive its cost, its deviation head w and the deviation vertex u.  A
+  // walk visits each chain vertex and each deviation at most once, so more
+  // than step_limit steps means a corrupt index: the walk stops and *err is
+  // raised.  *nonmono counts the children whose binary32 cost comes out below
+  // the parent's (a deviation whose int-scaled delta is 0, or a negative
+  // weight): where one sits at the bound, a path just below U can descend
+  // from a parent at or above U, which is never expanded.
   __device__ inline bool step(const int4* vrec, const int2* devinfo, const int4* devs, float U,
                               bool strict, int step_limit, int* err, unsigned long long* hops,
                               unsigned long long* devv, unsigned long long* nonmono, float* cc,
                               int* cw, int* from) {
-    if (mode == 2) return false;
-    if (++steps > step_limit) {
+    const int sub = __lane_id() % kLanes;
+    if (alive && ++steps > step_limit) {
       atomicExch(err, 1);
-      mode = 2;
-      return false;
+      alive = scan = false;
     }
     *from = v;
-    if (mode == 0) {
-      // the vertex record and its deviation range are loaded together (one
-      // round trip where the walk stops here, not two); j and je are set
-      // either way, and only read once the walk scans this vertex
-      const int4 r = vrec[v];
-      const int2 di = devinfo[v];
-      ++*hops;
+    bool fresh = false;  // the next vertex's record is loaded in this step
+    if (alive && !scan) {
+      if (sub == 0) ++*hops;
+      scan = !(__int_as_float(r.x) > X);
+      nv = scan ? r.z : r.y;
       j = di.x;
       je = di.x + di.y;
-      if (__int_as_float(r.x) > X) {
-        v = r.y;
-        if (v == -1) mode = 2;
-      } else {
-        sv = r.z;
-        dv = __int_as_float(r.w);
-        mode = 1;
-      }
-      return false;
+      fresh = nv != -1;
     }
-    bool leave = j >= je;
+    int4 d = make_int4(0, 0, 0, 0);
+    const bool in = alive && scan && j + sub < je;
+    if (in) d = devs[j + sub];
+    if (fresh) {
+      nr = vrec[nv];
+      ndi = devinfo[nv];
+    }
     bool emit = false;
-    if (!leave) {
-      const int4 d = devs[j];
-      ++*devv;
-      if (__int_as_float(d.w) > X) {
-        leave = true;
-      } else {
-        const float x = ((c + __int_as_float(d.z)) + __int_as_float(d.y)) - dv;
-        ++j;
-        if (x < c) ++*nonmono;
-        if (strict ? x < U : x <= U) {
-          emit = true;
-          *cc = x;
-          *cw = d.x;
-        }
+    const bool ok = in && !(__int_as_float(d.w) > X);
+    if (in) ++*devv;
+    if (ok) {
+      const float x = ((c + __int_as_float(d.z)) + __int_as_float(d.y)) - __int_as_float(r.w);
+      if (x < c) ++*nonmono;
+      if (strict ? x < U : x <= U) {
+        emit = true;
+        *cc = x;
+        *cw = d.x;
       }
     }
-    if (leave) {
-      v = sv;
-      mode = v == -1 ? 2 : 0;
+    // the list is cut at its first delta > X: go on only when every lane of
+    // the group took one
+    const uint64_t took = __ballot(ok) >> (__lane_id() - sub);
+    constexpr uint64_t kAll = kLanes == 64 ? ~0ull : (1ull << kLanes) - 1;
+    j += kLanes;
+    if (alive && !(scan && (took & kAll) == kAll && j < je)) {
+      v = nv;
+      r = nr;
+      di = ndi;
+      scan = false;
+      alive = nv != -1;
     }
     return emit;
   }

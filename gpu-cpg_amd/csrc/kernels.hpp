@@ -154,7 +154,7 @@ int launch_sfxt_scheduled(const SfxtArgs& args, const SfxtSched& sched, int bloc
 // them to the relabelled ids (perm: original -> relabelled).
 void launch_sfxt_succ_relabel(int* succ, const int* perm, int n, hipStream_t stream);
 // Deviation records, their sort, the lift tables and the nsv pointers.
-// m: the graph's edge count (chooses thread- or wave-per-vertex records).
+// m: the graph's edge count (chooses the lanes per vertex of the deviation pass).
 void launch_sfxt_index(const SfxtArgs& args, int lift_levels, int64_t m, hipStream_t stream);
 constexpr int kSfxtLdsSort = 2048;  // longest deviation list sorted in LDS
 // best[] and deps[] hold kSfxtPad slots after their n vertices: the level

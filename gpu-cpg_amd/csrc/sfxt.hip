@@ -53,7 +53,6 @@ constexpr int kLdsQueue = 2048;
 #define CPG_SPIN_LIMIT (1u << 22)
 #endif
 constexpr unsigned kSpinLimit = CPG_SPIN_LIMIT;
-constexpr int kThreadSort = 16;    // deviation lists up to this length: one thread sorts
 constexpr int kWaveSort = 64;      // up to this length: one wave ranks them in registers
 constexpr int kLdsSort = kSfxtLdsSort;  // up to this length: one block sorts in LDS
 constexpr int kFaninUnroll = 8;   // fanin records (and their atomics) in flight per step
@@ -1281,11 +1280,24 @@ __global__ void __launch_bounds__(256) sfxt_sched_finish_kernel(SfxtArgs a, Sfxt
     top = max(top, lev);
     if (d != kIntMax) mx = fmaxf(mx, fabsf(df));
   }
+  // one atomic per block, and none where the word is there already (an
+  // atomic per wave, 16K on two words, took 160 of the pass's 190 us at 1.5M
+  // vertices)
+  __shared__ float s_mx[4];
+  __shared__ int s_top[4];
   mx = wave_max(mx);
   top = wave_max_int(top);
   if (__lane_id() == 0) {
-    atomicMax(&a.ctl->max_abs_distf_bits, __float_as_uint(mx));
-    if (top >= 0) atomicMax(&a.ctl->num_levels, top + 1);
+    s_mx[threadIdx.x >> 6] = mx;
+    s_top[threadIdx.x >> 6] = top;
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    mx = fmaxf(fmaxf(s_mx[0], s_mx[1]), fmaxf(s_mx[2], s_mx[3]));
+    top = max(max(s_top[0], s_top[1]), max(s_top[2], s_top[3]));
+    if (__float_as_uint(mx) > ld_devu32(&a.ctl->max_abs_distf_bits))
+      atomicMax(&a.ctl->max_abs_distf_bits, __float_as_uint(mx));
+    if (top + 1 > ld_dev32(&a.ctl->num_levels)) atomicMax(&a.ctl->num_levels, top + 1);
   }
   if (blockIdx.x == 0 && threadIdx.x == 0) a.ctl->levelized = static_cast<unsigned>(s.nl);
 }
@@ -1582,90 +1594,6 @@ __device__ __forceinline__ void succ_candidate(const SfxtArgs& a, int w, int dw,
   }
 }
 
-// Deviation records of every settled vertex in fanout order, their smallest
-// delta, and the vertex record without its nsv pointer.  Lists of up to
-// kThreadSort records are sorted here (stable insertion sort by delta);
-// longer ones are queued for sfxt_sort_mid_kernel (up to kWaveSort, from
-// the front of big[]) or sfxt_sort_big_kernel (from the back).  The loop
-// is wave-uniform so the queue reservations are wave-aggregated.
-// Each block takes one contiguous chunk of vertices and each XCD one range
-// of chunks (xcd_block): a vertex's fanouts sit on the levels just below
-// it, and with level-ordered ids their dist/distf words then lie in the
-// range the same XCD's L2 already holds.
-__global__ void __launch_bounds__(256) sfxt_devs_kernel(SfxtArgs a) {
-  const int chunk = static_cast<int>(((static_cast<int64_t>(a.n) + gridDim.x - 1) / gridDim.x + 255) / 256 * 256);
-  const int64_t lo64 = static_cast<int64_t>(xcd_block(blockIdx.x, gridDim.x)) * chunk;
-  const int lo = static_cast<int>(lo64 < a.n ? lo64 : a.n);
-  const int hi = static_cast<int>(lo64 + chunk < a.n ? lo64 + chunk : a.n);
-  for (int base = lo; base < hi; base += blockDim.x) {
-    const int u = base + threadIdx.x;
-    int cnt = 0;
-    bool sorted = true;
-    if (u < hi) {
-      const int b = a.oadjp[u], e = a.oadjp[u + 1];
-      if (a.level[u] < 0 || a.dist[u] == kIntMax) {  // unsettled or reaches no chosen sink
-        a.vrec[u] = default_vrec();
-        a.devinfo[u] = make_int2(b, 0);
-        if (a.find_succ) a.succ[u] = -1;
-      } else {
-        int s = -1;
-        if (a.find_succ) {
-          // update_successors_bu (gpucpg/gpucpg.cu:2606-2628): the largest id
-          // among the fanouts at the minimum
-          int bd = kIntMax, bt = -1;
-          for (int j = b; j < e; ++j) {
-            const int w = a.oadj[j];
-            succ_candidate(a, w, a.dist[w], a.owgt[j], bd, bt, s);
-          }
-          a.succ[u] = s;
-        } else {
-          s = a.succ[u];
-        }
-        const float df = a.distf[u];
-        float mind = __builtin_huge_valf();
-        for (int j = b; j < e; ++j) {
-          const int w = a.oadj[j];
-          if (w == s) continue;
-          if (a.dist[w] == kIntMax) continue;
-          const float fw = a.distf[w];
-          const float we = a.owgt[j];
-          const float delta = static_cast<float>(static_cast<double>(fw) +
-                                                 static_cast<double>(we) -
-                                                 static_cast<double>(df));
-          a.devs[b + cnt] =
-              make_int4(w, __float_as_int(we), __float_as_int(fw), __float_as_int(delta));
-          mind = fminf(mind, delta);
-          ++cnt;
-        }
-        if (cnt <= kThreadSort) {
-          for (int i = 1; i < cnt; ++i) {
-            const int4 rec = a.devs[b + i];
-            const float key = __int_as_float(rec.w);
-            int k = i;
-            while (k > 0) {
-              const int4 prev = a.devs[b + k - 1];
-              if (__int_as_float(prev.w) <= key) break;
-              a.devs[b + k] = prev;
-              --k;
-            }
-            if (k != i) a.devs[b + k] = rec;
-          }
-        } else {
-          sorted = false;
-        }
-        a.vrec[u] = make_int4(__float_as_int(mind), -1, s, __float_as_int(df));
-        a.devinfo[u] = make_int2(b, cnt);
-      }
-    }
-    const bool mid = !sorted && cnt <= kWaveSort;
-    const bool large = !sorted && cnt > kWaveSort;
-    const uint64_t sm = wave_reserve(reinterpret_cast<unsigned long long*>(&a.ctl->nbig), mid);
-    const uint64_t sl = wave_reserve(reinterpret_cast<unsigned long long*>(&a.ctl->nbig_l), large);
-    if (mid) a.big[sm] = u;
-    if (large) a.big[a.n - 1 - static_cast<int>(sl)] = u;
-  }
-}
-
 // Total order used to rank deviation records: float order with -0 == +0
 // (ties keep fanout order, as the insertion sort does); NaN ranks last.
 __device__ inline uint32_t delta_rank_key(int bits) {
@@ -1673,48 +1601,80 @@ __device__ inline uint32_t delta_rank_key(int bits) {
   return x == 0.0f ? kKeyPosZero : float_key(x);
 }
 
-// Deviation records with one wave per vertex, for graphs whose fanouts
-// are long on average: lanes take the fanout edges 64 at a time and a
-// ballot compacts the deviation records in fanout order.  A fanout of at
-// most 128 edges keeps its records in registers (two per lane), ranks them
-// there (ties in fanout order, as sfxt_sort_mid_kernel) and stores each
-// once, sorted: each valid record's key is broadcast once and compared
-// with both of a lane's keys, so ranking costs one shuffle per record.
-// Longer fanouts store their records in fanout order and are queued for
-// sfxt_sort_big_kernel.  vrec and devinfo as in sfxt_devs_kernel.
-__device__ inline bool devs_record(const SfxtArgs& a, int j, int s, float df, int4& rec) {
-  const int w = a.oadj[j];
-  if (w == s || a.dist[w] == kIntMax) return false;
-  const float fw = a.distf[w];
-  const float we = a.owgt[j];
-  const float delta = static_cast<float>(static_cast<double>(fw) + static_cast<double>(we) -
-                                         static_cast<double>(df));
-  rec = make_int4(w, __float_as_int(we), __float_as_int(fw), __float_as_int(delta));
-  return true;
-}
-
-__global__ void __launch_bounds__(256) sfxt_devs_wave_kernel(SfxtArgs a) {
-  const int lane = __lane_id();
-  const int wave = static_cast<int>((blockIdx.x * blockDim.x + threadIdx.x) >> 6);
-  const int nwaves = static_cast<int>((gridDim.x * blockDim.x) >> 6);
-  for (int u = wave; u < a.n; u += nwaves) {
-    const int b = a.oadjp[u], e = a.oadjp[u + 1];
-    if (a.level[u] < 0 || a.dist[u] == kIntMax) {  // unsettled or reaches no chosen sink
-      if (lane == 0) {
+// Deviation records of every settled vertex sorted by delta (ties in fanout
+// order), their smallest delta, and the vertex record without its nsv
+// pointer; with find_succ each vertex's successor too.
+//
+// kG lanes take a vertex.  A fanout of at most 2 kG edges stays in registers,
+// two edges per lane: the group's ballot counts the records, each valid
+// record's key is broadcast once and compared with both of a lane's keys,
+// and every record is stored once, at its rank.  Longer fanouts are stored in
+// fanout order and queued for sfxt_sort_mid_kernel (up to kWaveSort records,
+// from the front of big[]) or sfxt_sort_big_kernel (from the back).
+//
+// What bounds it: gathers of the fanouts' dist and distf, in flight for all
+// of a row's edges at once (a thread per vertex read them one by one: 256 us
+// at 1.5M vertices / 4.08M edges, 600 us at 1.1M / 5.7M).
+//
+// Each block takes one contiguous chunk of vertices and each XCD one range
+// of chunks (xcd_block): a vertex's fanouts sit on the levels just below it,
+// and with level-ordered ids their words then lie in the range the same
+// XCD's L2 already holds.
+template <int kG>
+__global__ void __launch_bounds__(256) sfxt_devs_kernel(SfxtArgs a) {
+  constexpr int kV = 256 / kG;  // vertices per block step
+  const int lane = __lane_id(), sub = lane % kG, gbase = lane - sub;
+  constexpr uint64_t kMask = kG == 64 ? ~0ull : (1ull << kG) - 1;
+  const int64_t per = (static_cast<int64_t>(a.n) + gridDim.x - 1) / gridDim.x;
+  const int64_t chunk = (per + kV - 1) / kV * kV;
+  const int64_t lo64 = static_cast<int64_t>(xcd_block(blockIdx.x, gridDim.x)) * chunk;
+  const int lo = static_cast<int>(lo64 < a.n ? lo64 : a.n);
+  const int hi = static_cast<int>(lo64 + chunk < a.n ? lo64 + chunk : a.n);
+  for (int base = lo; base < hi; base += kV) {  // block-uniform
+    const int u = base + static_cast<int>(threadIdx.x) / kG;
+    int b = 0, e = 0, s = -1;
+    float df = 0.0f;
+    bool settled = false;  // levelized and reaching a chosen sink
+    if (u < hi) {
+      b = a.oadjp[u];
+      e = a.oadjp[u + 1];
+      settled = a.level[u] >= 0 && a.dist[u] != kIntMax;
+      df = a.distf[u];
+      if (!settled && sub == 0) {
         a.vrec[u] = default_vrec();
         a.devinfo[u] = make_int2(b, 0);
         if (a.find_succ) a.succ[u] = -1;
       }
-      continue;
+      if (!settled) e = b;
+      else if (!a.find_succ) s = a.succ[u];
     }
-    int s = -1;
+    const bool wide = e - b > 2 * kG;
+    // this lane's first two edges
+    int w[2], dw[2];
+    float we[2], fw[2];
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+      const int j = b + q * kG + sub;
+      w[q] = j < e ? a.oadj[j] : -1;
+      we[q] = j < e ? a.owgt[j] : 0.0f;
+    }
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+      dw[q] = w[q] >= 0 ? a.dist[w[q]] : kIntMax;
+      fw[q] = w[q] >= 0 ? a.distf[w[q]] : 0.0f;
+    }
     if (a.find_succ) {
+      // update_successors_bu (gpucpg/gpucpg.cu:2606-2628): the largest id
+      // among the fanouts at the minimum
       int bd = kIntMax, bt = -1;
-      for (int j = b + lane; j < e; j += 64) {
-        const int w = a.oadj[j];
-        succ_candidate(a, w, a.dist[w], a.owgt[j], bd, bt, s);
+#pragma unroll
+      for (int q = 0; q < 2; ++q) succ_candidate(a, w[q], dw[q], we[q], bd, bt, s);
+      for (int j = b + 2 * kG + sub; j < e; j += kG) {
+        const int x = a.oadj[j];
+        succ_candidate(a, x, a.dist[x], a.owgt[j], bd, bt, s);
       }
-      for (int o = 32; o > 0; o >>= 1) {
+#pragma unroll
+      for (int o = 1; o < kG; o <<= 1) {
         const int od = __shfl_xor(bd, o), ot = __shfl_xor(bt, o), os = __shfl_xor(s, o);
         if (od < bd || (od == bd && ot > bt)) {
           bd = od;
@@ -1722,65 +1682,85 @@ __global__ void __launch_bounds__(256) sfxt_devs_wave_kernel(SfxtArgs a) {
           s = os;
         }
       }
-      if (lane == 0) a.succ[u] = s;
-    } else {
-      s = a.succ[u];
+      if (settled && sub == 0) a.succ[u] = s;
     }
-    const float df = a.distf[u];
+    auto delta_of = [&](float f, float x) {
+      return static_cast<float>(static_cast<double>(f) + static_cast<double>(x) - static_cast<double>(df));
+    };
     int cnt = 0;
     float mind = __builtin_huge_valf();
-    if (e - b <= 128) {
-      int4 r0 = make_int4(0, 0, 0, 0), r1 = make_int4(0, 0, 0, 0);
-      const bool ok0 = b + lane < e && devs_record(a, b + lane, s, df, r0);
-      const bool ok1 = b + 64 + lane < e && devs_record(a, b + 64 + lane, s, df, r1);
-      if (ok0) mind = fminf(mind, __int_as_float(r0.w));
-      if (ok1) mind = fminf(mind, __int_as_float(r1.w));
-      const uint64_t m0 = __ballot(ok0), m1 = __ballot(ok1);
-      cnt = static_cast<int>(__popcll(m0) + __popcll(m1));
-      const uint32_t k0 = ok0 ? delta_rank_key(r0.w) : 0u;
-      const uint32_t k1 = ok1 ? delta_rank_key(r1.w) : 0u;
-      // rank = records ordering before this one: a smaller key, or an
-      // equal key earlier in fanout order (every first-half record is
-      // earlier than every second-half one)
-      int rank0 = 0, rank1 = 0;
-      for (uint64_t mm = m0; mm; mm &= mm - 1) {
-        const int jj = static_cast<int>(__builtin_ctzll(mm));
-        const uint32_t kj = __shfl(k0, jj);
-        rank0 += (kj < k0 || (kj == k0 && jj < lane)) ? 1 : 0;
-        rank1 += kj <= k1 ? 1 : 0;
-      }
-      for (uint64_t mm = m1; mm; mm &= mm - 1) {
-        const int jj = static_cast<int>(__builtin_ctzll(mm));
-        const uint32_t kj = __shfl(k1, jj);
-        rank0 += kj < k0 ? 1 : 0;
-        rank1 += (kj < k1 || (kj == k1 && jj < lane)) ? 1 : 0;
-      }
-      if (ok0) a.devs[b + rank0] = r0;
-      if (ok1) a.devs[b + rank1] = r1;
-    } else {
-      for (int j0 = b; j0 < e; j0 += 64) {
-        int4 rec = make_int4(0, 0, 0, 0);
-        const bool ok = j0 + lane < e && devs_record(a, j0 + lane, s, df, rec);
-        if (ok) mind = fminf(mind, __int_as_float(rec.w));
-        const uint64_t bm = __ballot(ok);
-        if (ok) a.devs[b + cnt + static_cast<int>(__popcll(bm & lanemask_lt()))] = rec;  // sorted later
-        cnt += static_cast<int>(__popcll(bm));
-      }
-      if (lane == 0) {
-        const unsigned long long sl = atomicAdd(&a.ctl->nbig_l, 1ull);
-        a.big[a.n - 1 - static_cast<int>(sl)] = u;
+    // rows in registers: rank = records ordering before this one, a smaller
+    // key or an equal key earlier in fanout order
+    bool ok[2];
+    uint32_t key[2];
+    int rank[2] = {0, 0};
+    float dl[2];
+    uint64_t bal[2];
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+      ok[q] = !wide && w[q] >= 0 && w[q] != s && dw[q] != kIntMax;
+      dl[q] = delta_of(fw[q], we[q]);
+      if (ok[q]) mind = fminf(mind, dl[q]);
+      key[q] = ok[q] ? delta_rank_key(__float_as_int(dl[q])) : 0u;
+      bal[q] = __ballot(ok[q]);
+    }
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+      const uint64_t mine = (bal[q] >> gbase) & kMask;
+      cnt += static_cast<int>(__popcll(mine));
+      uint64_t any = bal[q];  // places in a group that hold a record in some group
+#pragma unroll
+      for (int o = 32; o >= kG; o >>= 1) any |= any >> o;
+      for (any &= kMask; any; any &= any - 1) {  // wave-uniform
+        const int jj = static_cast<int>(__builtin_ctzll(any));
+        const uint32_t kj = __shfl(key[q], gbase + jj);
+        if (!((mine >> jj) & 1ull)) continue;
+        rank[q] += (kj < key[q] || (kj == key[q] && jj < sub)) ? 1 : 0;
+        rank[q ^ 1] += (kj < key[q ^ 1] || (kj == key[q ^ 1] && q == 0)) ? 1 : 0;
       }
     }
-    for (int o = 32; o > 0; o >>= 1) mind = fminf(mind, __shfl_xor(mind, o));
-    if (lane == 0) {
+#pragma unroll
+    for (int q = 0; q < 2; ++q)
+      if (ok[q])
+        a.devs[b + rank[q]] =
+            make_int4(w[q], __float_as_int(we[q]), __float_as_int(fw[q]), __float_as_int(dl[q]));
+    // longer rows: fanout order, sorted later
+    if (__ballot(wide)) {
+      for (int j0 = b; __ballot(wide && j0 < e) != 0; j0 += kG) {
+        const int j = j0 + sub;
+        bool put = false;
+        int4 rec = make_int4(0, 0, 0, 0);
+        if (wide && j < e) {
+          const int x = a.oadj[j];
+          if (x != s && a.dist[x] != kIntMax) {
+            const float f = a.distf[x], xe = a.owgt[j];
+            const float d = delta_of(f, xe);
+            rec = make_int4(x, __float_as_int(xe), __float_as_int(f), __float_as_int(d));
+            mind = fminf(mind, d);
+            put = true;
+          }
+        }
+        const uint64_t m = (__ballot(put) >> gbase) & kMask;
+        if (put) a.devs[b + cnt + static_cast<int>(__popcll(m & ((1ull << sub) - 1)))] = rec;
+        cnt += static_cast<int>(__popcll(m));
+      }
+      const bool mid = wide && sub == 0 && cnt <= kWaveSort, large = wide && sub == 0 && cnt > kWaveSort;
+      const uint64_t sm = wave_reserve(reinterpret_cast<unsigned long long*>(&a.ctl->nbig), mid);
+      const uint64_t sl = wave_reserve(reinterpret_cast<unsigned long long*>(&a.ctl->nbig_l), large);
+      if (mid) a.big[sm] = u;
+      if (large) a.big[a.n - 1 - static_cast<int>(sl)] = u;
+    }
+#pragma unroll
+    for (int o = 1; o < kG; o <<= 1) mind = fminf(mind, __shfl_xor(mind, o));
+    if (settled && sub == 0) {
       a.vrec[u] = make_int4(__float_as_int(mind), -1, s, __float_as_int(df));
       a.devinfo[u] = make_int2(b, cnt);
     }
   }
 }
 
-// Stable sort by delta of the lists of kThreadSort+1 .. kWaveSort records,
-// one wave per list: lane i holds record i and its rank is the number of
+// Stable sort by delta of the queued lists of up to kWaveSort records, one
+// wave per list: lane i holds record i and its rank is the number of
 // records that order before it (shuffled keys), so the records land in
 // place with one store each.
 __global__ void __launch_bounds__(256) sfxt_sort_mid_kernel(SfxtArgs a) {
@@ -2108,13 +2088,24 @@ void launch_sfxt_levels_parts(const SfxtParts& parts, int total_blocks, hipStrea
 void launch_sfxt_index(const SfxtArgs& args, int lift_levels, int64_t m, hipStream_t stream) {
   const int cus = device_cus();
   const int g = flat_grid(args.n, cus);
-  if (args.n > 0 && m >= 8 * static_cast<int64_t>(args.n)) {
-    // mean fanout of 8 or more: one wave per vertex
-    const int64_t wb = (static_cast<int64_t>(args.n) + 3) / 4;
-    const int gw = static_cast<int>(std::min<int64_t>(wb, static_cast<int64_t>(cus) * 64));
-    hipLaunchKernelGGL(sfxt_devs_wave_kernel, dim3(gw), dim3(256), 0, stream, args);
-  } else {
-    hipLaunchKernelGGL(sfxt_devs_kernel, dim3(g), dim3(256), 0, stream, args);
+  // Lanes per vertex in the deviation pass: rows of up to twice as many edges
+  // stay in registers, and every longer one costs a place in the sort queue
+  // (one counter) and another pass, so 4.6 times the mean.  Index passes (ms)
+  // with 4 / 8 / 16 / 32 / 64 lanes: 1.5M vertices (mean 2.7) 0.55 / 0.28 /
+  // 0.34 / 0.48 / 0.77; 700K (3.3) 0.44 / 0.16 / 0.19 / 0.26 / 0.39; 1.1M (5.3)
+  // 1.07 / 0.62 / 0.36 / 0.47 / 0.70; 400K (20) 0.85 / 1.10 / 1.05 / 0.49 /
+  // 0.42; 250K (27) 0.77 / 0.95 / 1.03 / 0.56 / 0.31.
+  const double mean = static_cast<double>(m) / static_cast<double>(std::max(1, args.n));
+  int lanes = 4;
+  while (lanes < 64 && 2.0 * lanes < 4.6 * mean) lanes *= 2;
+  const int64_t steps = (static_cast<int64_t>(args.n) * lanes + 255) / 256;
+  const dim3 dg(static_cast<unsigned>(std::max<int64_t>(1, std::min<int64_t>(steps, static_cast<int64_t>(cus) * 32))));
+  switch (lanes) {
+    case 4: hipLaunchKernelGGL(sfxt_devs_kernel<4>, dg, dim3(256), 0, stream, args); break;
+    case 8: hipLaunchKernelGGL(sfxt_devs_kernel<8>, dg, dim3(256), 0, stream, args); break;
+    case 16: hipLaunchKernelGGL(sfxt_devs_kernel<16>, dg, dim3(256), 0, stream, args); break;
+    case 32: hipLaunchKernelGGL(sfxt_devs_kernel<32>, dg, dim3(256), 0, stream, args); break;
+    default: hipLaunchKernelGGL(sfxt_devs_kernel<64>, dg, dim3(256), 0, stream, args); break;
   }
   CPG_HIP(hipGetLastError());
   hipLaunchKernelGGL(sfxt_sort_mid_kernel, dim3(cus * 8), dim3(256), 0, stream, args);

@@ -488,13 +488,20 @@ struct cpg_handle {
     return static_cast<int>(std::min<int64_t>(128, std::max<int64_t>(16, (per_level + 255) / 256)));
   }
 
-  // Scheduled-loop grid: one block per CU, over all XCDs.  The loop has no
-  // barrier to pay for more blocks, and a CU's scattered-load rate bounds
-  // wide levels: on the 1.5M-vertex DAG 0.74 ms with 256 blocks, 0.87 with
-  // 128, 1.6 with 32; narrow levels measure the same from 32 up (50K-vertex
-  // DAG 0.14 ms).  Keeping the blocks on one XCD was slower on every graph
-  // wider than that one (1.6 ms and 0.74; 3.4 and 1.9 at 1.1M vertices).
-  int sched_blocks() const { return sfxt_blocks > 0 ? sfxt_blocks : std::max(1, grid / 8); }
+  // Scheduled-loop grid: two waves per chunk of an average level, 16 to 128
+  // blocks over all XCDs.  The loop has no barrier to pay for more blocks, and
+  // a CU's scattered-load rate bounds wide levels: on the 1.5M-vertex DAG 0.87
+  // ms with 128 blocks (0.74 with 256), 1.6 with 32; narrow levels measure the
+  // same from 16 up (50K-vertex DAG 0.14 ms).  128 blocks are a sixteenth of
+  // what the device holds, so the loops of 16 handles on streams of their own
+  // are resident together; a wave may wait for any other wave of its loop.
+  // Keeping the blocks on one XCD was slower on every graph wider than that
+  // one (1.6 ms and 0.74; 3.4 and 1.9 at 1.1M vertices).
+  int sched_blocks(int lanes) const {
+    if (sfxt_blocks > 0) return sfxt_blocks;
+    const int64_t chunks = static_cast<int64_t>(sched.np) * lanes / 64 / std::max(1, last_diameter);
+    return static_cast<int>(std::min<int64_t>(128, std::max<int64_t>(16, (chunks + 1) / 2)));
+  }
 
   // The endpoint subset of an n-byte mask as one flag per sink (in sink
   // order); empty when the mask is null or chooses every sink.
@@ -578,6 +585,17 @@ struct cpg_handle {
     sched.ofs = reinterpret_cast<const int*>(ofs_d);
     sched.edge = edge_d;
     sched_ready = true;
+  }
+
+  // The schedule of a graph whose level order is at hand, ahead of the next
+  // SFXT (graphs made resident to be queried many times).
+  void prepare_schedule() {
+    if (sched_ready || !order_ready || last_diameter <= 0 || g.n == 0) return;
+    SfxtArgs a{};
+    a.n = g.n;
+    a.oadjp = oadjp.p; a.oadj = oadj.p; a.owgt = owgt.p;
+    a.lvlp = lvlp.p; a.level = level.p;
+    build_schedule(a);
   }
 
   // Gives the schedule's memory back (a query under a device-byte budget
@@ -690,7 +708,7 @@ struct cpg_handle {
       else launch_sfxt_init(a, stream);
       if (kernel_timing) CPG_HIP(hipEventRecord(ev_levels.a, stream));
       a.find_succ = scheduled ? 1 : 0;
-      timing.sfxt_blocks = scheduled     ? launch_sfxt_scheduled(a, sched, sched_blocks(), stream)
+      timing.sfxt_blocks = scheduled     ? launch_sfxt_scheduled(a, sched, sched_blocks(sched.lanes), stream)
                            : dataflow    ? launch_sfxt_dataflow(a, df_grid, stream)
                            : method == 3 ? launch_sfxt_local(a, level_loop_blocks(), stream)
                            : method == 4 ? launch_sfxt_levels_nf(a, level_loop_blocks(), stream)
@@ -1762,6 +1780,7 @@ struct cpg_server {
     std::vector<int64_t> ids;
     std::vector<SfxtArgs> args;   // per query: its distance columns and index
     SfxtArgs base{};              // the group's shared level-loop arguments
+    bool scheduled = false;       // its loop runs in schedule order
     int lv = 0;                   // lift depth
     PinnedBuf<uint8_t> hmask;     // host copy of the subsets' sink flags (pinned: the copy is asynchronous)
     PinnedBuf<SfxtCtl> hctl;      // the group's SFXT controls, copied out before its event: graph's, then each query's
@@ -1906,6 +1925,7 @@ struct cpg_server {
     G->h->set_graph(el);
     G->h->upload_graph();
     G->h->run_sfxt(false);  // the level count (the same for every endpoint subset)
+    G->h->prepare_schedule();
     const int64_t n = G->h->g.n, m = G->h->g.m;
     G->index_bytes = 24 * n + 16 * m;  // vrec 16, devinfo 8 per vertex; devs 16 per edge
     graphs.push_back(std::move(G));
@@ -2063,7 +2083,10 @@ struct cpg_server {
   // only, so the lift depth is known from the graph's first SFXT.
   void start_groups(const std::vector<std::pair<int, std::vector<int64_t>>>& list) {
     const double t0 = now_ms();
-    SfxtParts parts{};
+    SfxtParts parts{};       // level loops (graphs without a schedule)
+    SfxtSchedParts sparts{};  // scheduled loops
+    SfxtMulti smm[kMaxParts]{};
+    int sn[kMaxParts]{};
     std::vector<int> part_of(list.size(), -1);
     for (size_t li = 0; li < list.size(); ++li) {
       const int gi = list[li].first;
@@ -2087,7 +2110,8 @@ struct cpg_server {
       h.big.reserve(n); h.sctl.reserve(1);
       if (h.g.max_out_degree > kSfxtLdsSort) h.devs_tmp.reserve(m);
       Graph::Multi& M = G.mm;
-      M.dv.reserve(n * Q); M.dist.reserve(n * Q); M.succ.reserve(n * Q); M.distf.reserve(n * Q);
+      G.scheduled = h.sched_ready;
+      M.dv.reserve((G.scheduled ? static_cast<size_t>(h.sched.np) : n) * Q); M.dist.reserve(n * Q); M.succ.reserve(n * Q); M.distf.reserve(n * Q);
       const size_t ns = h.g.sinks.size();
       M.masks.reserve(std::max<size_t>(1, ns * Q)); M.maxd.reserve(Q); M.ctls.reserve(Q);
       // one flag per sink (in sink order) and subset; padding subsets choose none
@@ -2119,7 +2143,18 @@ struct cpg_server {
       G.args.clear();
       G.base = a;
       G.lv = lv;
-      if (n > 0) {
+      if (n > 0 && G.scheduled) {
+        SfxtSchedPart& P = sparts.p[sparts.n];
+        P.s = h.sched;
+        P.masks = M.masks.p; P.dv = M.dv.p; P.ctl = h.sctl.p;
+        P.nsinks = a.nsinks;
+        P.q = Q;
+        P.lanes = sfxt_sched_multi_lanes(h.sched, Q, static_cast<double>(m) / static_cast<double>(n));
+        P.nb = h.sched_blocks(P.lanes);
+        smm[sparts.n] = mm;
+        sn[sparts.n++] = h.g.n;
+        CPG_HIP(hipMemsetAsync(M.maxd.p, 0, sizeof(unsigned) * Q, sstream));
+      } else if (n > 0) {
         launch_sfxt_init_multi(a, mm, sstream);
         // one wave per vertex: about one block per 8 vertices of an average level
         const int64_t per_level = h.diameter > 0 ? static_cast<int64_t>(n) / h.diameter : 4096;
@@ -2132,6 +2167,16 @@ struct cpg_server {
       G.ids = ids;
     }
     stats.peak_index_bytes = std::max(stats.peak_index_bytes, index_bytes);
+    if (sparts.n > 0) {
+      int total = 0;
+      for (int i = 0; i < sparts.n; ++i) {
+        sparts.p[i].nb = std::max(1, std::min(sparts.p[i].nb, parts_cap / sparts.n));
+        sparts.p[i].b0 = total;
+        total += sparts.p[i].nb;
+      }
+      launch_sfxt_sched_multi(sparts, total, sstream);
+      for (int i = 0; i < sparts.n; ++i) launch_sfxt_sched_multi_finish(sparts.p[i], smm[i], sn[i], sstream);
+    }
     if (parts.n > 0) {
       // fit every partition into one resident launch (admission forms at
       // most parts_cap groups, so one block each always fits)
@@ -2189,6 +2234,7 @@ struct cpg_server {
         aq.vrec = ix->vrec.p; aq.devinfo = ix->devinfo.p; aq.devs = ix->devs.p;
         aq.lift = h.lift.p;
         aq.ctl = G.mm.ctls.p + q;
+        aq.find_succ = G.scheduled ? 1 : 0;
         if (n > 0) launch_sfxt_index(aq, G.lv, h.g.m, h.stream);
         qq.index = std::move(ix);
         G.args.push_back(aq);
@@ -2300,8 +2346,9 @@ struct cpg_server {
       }
     }
     if (h.g.n > 0) {
+      if (c.err == 2) throw std::runtime_error("a suffix distance is out of the served loop's range");
       if (c.err) throw std::runtime_error("SFXT grid barrier did not complete");
-      if (c.num_levels != h.diameter) throw std::runtime_error("SFXT levels differ from the graph's");
+      if (!G.scheduled && c.num_levels != h.diameter) throw std::runtime_error("SFXT levels differ from the graph's");
       for (int q = 0; q < Q; ++q) {
         if (cq[q].nsv_err == 2) throw std::runtime_error("SFXT long deviation list without sort buffer");
         if (cq[q].nsv_err) throw std::runtime_error("SFXT next-smaller descent found no answer");

@@ -116,7 +116,8 @@ struct SfxtParts {
   int n;
   int pad;
 };
-// Blocks the partitioned level loop can keep resident at once.
+// Blocks the partitioned loops (level order found, or scheduled) can keep
+// resident at once.
 int sfxt_parts_capacity();
 // parts.p[0..n) cover the blocks [0, total_blocks) in ascending b0.
 void launch_sfxt_levels_parts(const SfxtParts& parts, int total_blocks, hipStream_t stream);
@@ -150,6 +151,32 @@ void launch_sfxt_sched_build(const SfxtArgs& args, const int* order, const int* 
 // succ[] left to the deviation pass (args.find_succ).  args.best holds a
 // state word per position.  Returns the working blocks.
 int launch_sfxt_scheduled(const SfxtArgs& args, const SfxtSched& sched, int blocks, hipStream_t stream);
+// One graph's multi-subset loop in schedule order, on the blocks [b0, b0 + nb)
+// of a launch holding several graphs' loops: q subsets (a power of two, at
+// most 64), dv the np x q settled distances, position-major; lanes a power of
+// two, at least q and the schedule's lanes.
+struct SfxtSchedPart {
+  SfxtSched s;
+  const uint8_t* masks;  // q x nsinks chosen-sink flags, as SfxtMulti
+  int* dv;
+  SfxtCtl* ctl;
+  int nsinks;
+  int q;
+  int lanes;             // lanes per vertex
+  int b0;
+  int nb;
+};
+struct SfxtSchedParts {
+  SfxtSchedPart p[kMaxParts];
+  int n;
+  int pad;
+};
+// Lanes per vertex for q subsets of a graph of mean out-degree `mean`.
+int sfxt_sched_multi_lanes(const SfxtSched& s, int q, double mean);
+// The loops (state words prepared first), then per graph its dist and distf
+// columns and maxd (m.dv is not used); succ[] is left to the deviation pass.
+void launch_sfxt_sched_multi(const SfxtSchedParts& parts, int total_blocks, hipStream_t stream);
+void launch_sfxt_sched_multi_finish(const SfxtSchedPart& part, const SfxtMulti& m, int n, hipStream_t stream);
 // Relabelled graph: succ[] holds original ids after a level loop; map
 // them to the relabelled ids (perm: original -> relabelled).
 void launch_sfxt_succ_relabel(int* succ, const int* perm, int n, hipStream_t stream);

@@ -1302,6 +1302,147 @@ __global__ void __launch_bounds__(256) sfxt_sched_finish_kernel(SfxtArgs a, Sfxt
   if (blockIdx.x == 0 && threadIdx.x == 0) a.ctl->levelized = static_cast<unsigned>(s.nl);
 }
 
+// Scheduled loop for Q endpoint subsets at once (served queries): lanes_ lanes
+// per vertex, lane l of them taking record l / Q of a step in subset l % Q, so
+// that a record's Q distances are one contiguous load.  A distance is its own
+// write-once state word (kMultiEmpty until settled); a vertex whose distance
+// comes out as exactly that value raises an error instead.  Otherwise as
+// sfxt_sched_kernel; levels are not computed (no served result holds them).
+// The level loop it replaces took 24-46 us a level (counters, queue, a grid
+// barrier, one wave per vertex).
+constexpr int kMultiEmpty = static_cast<int>(0x80000000u);
+
+__device__ void sched_multi_part(const SfxtSchedPart& P, unsigned bid, unsigned nblk) {
+  constexpr int kU = 4;
+  const int lane = __lane_id();
+  const int Q = P.q, LV = P.lanes, V = 64 / LV, R = LV / Q;
+  const int grp = lane / LV, in = lane % LV, sub = in % Q, rec = in / Q;
+  const int nw = static_cast<int>(nblk * (blockDim.x / 64u));
+  const int nchunk = P.s.np / V;
+  int c = P.s.first / V + static_cast<int>((threadIdx.x / 64u) * nblk + bid);
+  auto range = [&](int ch, int& b, int& e) {
+    b = e = 0;
+    if (ch < nchunk) {
+      b = P.s.ofs[ch * V + grp];
+      e = P.s.ofs[ch * V + grp + 1];
+    }
+  };
+  auto fetch = [&](int b, int e, int2* r) {
+#pragma unroll
+    for (int q = 0; q < kU; ++q) {
+      const int j = b + q * R + rec;
+      r[q] = P.s.edge[j < e ? j : 0];
+      if (j >= e) r[q].x = -1;
+    }
+  };
+  auto at = [&](int x) { return P.dv + static_cast<size_t>(x) * Q + sub; };
+  int b0, e0, b1, e1;
+  int2 r0[kU];
+  range(c, b0, e0);
+  fetch(b0, e0, r0);
+  range(c + nw, b1, e1);
+  for (; c < nchunk; c += nw) {
+    int bd = kIntMax;
+    int st[kU];
+    auto load = [&](const int2* r) {
+#pragma unroll
+      for (int q = 0; q < kU; ++q) st[q] = r[q].x >= 0 ? ld_dev32(at(r[q].x)) : kIntMax;
+    };
+    auto settle = [&](const int2* r) {
+      for (unsigned spins = 1;; ++spins) {
+        bool open = false;
+#pragma unroll
+        for (int q = 0; q < kU; ++q) open = open || st[q] == kMultiEmpty;
+        if (__ballot(open) == 0) break;
+        if (spins > kSpinLimit) { atomicExch(&P.ctl->err, 1); break; }
+        if ((spins & 255u) == 0u && __ballot(ld_dev32(&P.ctl->err) != 0) != 0) break;
+        __builtin_amdgcn_s_sleep(1);
+#pragma unroll
+        for (int q = 0; q < kU; ++q)
+          if (st[q] == kMultiEmpty) st[q] = ld_dev32(at(r[q].x));
+      }
+#pragma unroll
+      for (int q = 0; q < kU; ++q)
+        if (st[q] != kIntMax && st[q] != kMultiEmpty)
+          bd = min(bd, static_cast<int>(static_cast<unsigned>(st[q]) + static_cast<unsigned>(r[q].y)));
+    };
+    load(r0);
+    int2 r1[kU];
+    int b2, e2;
+    fetch(b1, e1, r1);
+    range(c + 2 * nw, b2, e2);
+    settle(r0);
+    for (int b = b0 + kU * R; __ballot(b < e0) != 0; b += kU * R) {  // longer rows
+      fetch(b, e0, r0);
+      load(r0);
+      settle(r0);
+    }
+    for (int o = Q; o < LV; o <<= 1) bd = min(bd, __shfl_xor(bd, o));
+    if (in < Q && b0 < e0) {
+      if (bd == kMultiEmpty) {
+        atomicExch(&P.ctl->err, 2);
+        bd = kIntMax;
+      }
+      st_dev32(at(c * V + grp), bd);
+    }
+#pragma unroll
+    for (int q = 0; q < kU; ++q) r0[q] = r1[q];
+    b0 = b1;
+    e0 = e1;
+    b1 = b2;
+    e1 = e2;
+  }
+}
+
+__global__ void __launch_bounds__(kSchedBlock) sfxt_sched_multi_kernel(SfxtSchedParts parts) {
+  __shared__ int s_part;
+  if (threadIdx.x == 0) {
+    int p = 0;
+    while (p + 1 < parts.n && static_cast<int>(blockIdx.x) >= parts.p[p + 1].b0) ++p;
+    s_part = p;
+  }
+  __syncthreads();
+  const SfxtSchedPart P = parts.p[s_part];
+  sched_multi_part(P, blockIdx.x - static_cast<unsigned>(P.b0), static_cast<unsigned>(P.nb));
+}
+
+__global__ void __launch_bounds__(256) sfxt_sched_multi_init_kernel(SfxtSchedPart P) {
+  const int64_t m = static_cast<int64_t>(P.s.np) * P.q;
+  for (int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x; i < m;
+       i += static_cast<int64_t>(gridDim.x) * blockDim.x) {
+    const int64_t p = i / P.q, q = i % P.q;
+    int d = kMultiEmpty;
+    if (p < P.nsinks) d = !P.masks || P.masks[q * P.nsinks + p] ? 0 : kIntMax;
+    P.dv[i] = d;
+  }
+}
+
+// Per subset the dist and distf columns and the largest finite |distf|: a
+// thread takes a vertex, so a column's stores are contiguous.
+__global__ void __launch_bounds__(256) sfxt_sched_multi_finish_kernel(SfxtSchedPart P, SfxtMulti m, int n) {
+  __shared__ unsigned s_max[64];
+  if (threadIdx.x < 64) s_max[threadIdx.x] = 0u;
+  __syncthreads();
+  for (int64_t base = static_cast<int64_t>(blockIdx.x) * blockDim.x; base < n;
+       base += static_cast<int64_t>(gridDim.x) * blockDim.x) {  // block-uniform
+    const int64_t v = base + threadIdx.x;
+    const int p = v < n ? P.s.pos[v] : -1;
+    for (int q = 0; q < P.q; ++q) {
+      const int d = p >= 0 ? P.dv[static_cast<size_t>(p) * P.q + q] : kIntMax;
+      const float df = static_cast<float>(d) / static_cast<float>(kScaleUp);
+      if (v < n) {
+        m.dist[static_cast<size_t>(q) * n + v] = d;
+        m.distf[static_cast<size_t>(q) * n + v] = df;
+      }
+      const float mx = wave_max(v < n && d != kIntMax ? fabsf(df) : 0.0f);
+      if (__lane_id() == 0) atomicMax(&s_max[q], __float_as_uint(mx));
+    }
+  }
+  __syncthreads();
+  if (static_cast<int>(threadIdx.x) < P.q && s_max[threadIdx.x] > ld_devu32(&m.maxd[threadIdx.x]))
+    atomicMax(&m.maxd[threadIdx.x], s_max[threadIdx.x]);
+}
+
 // Schedule build: positions and fanout counts, ...
 __global__ void __launch_bounds__(256) sfxt_sched_clear_kernel(int n, int np, int* pos, unsigned* ofs) {
   const int m = max(n, np + 1);
@@ -2016,6 +2157,36 @@ int launch_sfxt_scheduled(const SfxtArgs& args, const SfxtSched& s, int blocks, 
   return used;
 }
 
+int sfxt_sched_multi_lanes(const SfxtSched& s, int q, double mean) {
+  // a step of four records per lane takes about twice a mean row
+  int r = 1;
+  while (r < 64 && 2.0 * r < mean) r *= 2;
+  return std::min(64, std::max(s.lanes, q * r));
+}
+
+void launch_sfxt_sched_multi(const SfxtSchedParts& parts, int total_blocks, hipStream_t stream) {
+  if (parts.n < 1 || parts.n > kMaxParts || total_blocks > resident_blocks(sfxt_sched_multi_kernel, kSchedBlock))
+    throw std::runtime_error("scheduled loop partitions do not fit one resident launch");
+  const int cus = device_cus();
+  for (int i = 0; i < parts.n; ++i) {
+    const SfxtSchedPart& p = parts.p[i];
+    const int end = i + 1 < parts.n ? parts.p[i + 1].b0 : total_blocks;
+    if (p.nb < 1 || p.b0 + p.nb != end || (i == 0 && p.b0 != 0))
+      throw std::runtime_error("scheduled loop partitions must tile the launch");
+    if (p.q < 1 || p.q > 64 || p.lanes < p.q || p.lanes < p.s.lanes || p.lanes > 64 || (p.lanes & (p.lanes - 1)))
+      throw std::runtime_error("scheduled loop: bad lanes per vertex");
+    const int64_t words = std::min<int64_t>(static_cast<int64_t>(p.s.np) * p.q, 0x7fffffff);
+    hipLaunchKernelGGL(sfxt_sched_multi_init_kernel, dim3(flat_grid(static_cast<int>(words), cus)), dim3(256), 0, stream, p);
+    CPG_HIP(hipGetLastError());
+  }
+  launch_resident(sfxt_sched_multi_kernel, total_blocks, kSchedBlock, parts, stream);
+}
+
+void launch_sfxt_sched_multi_finish(const SfxtSchedPart& part, const SfxtMulti& m, int n, hipStream_t stream) {
+  hipLaunchKernelGGL(sfxt_sched_multi_finish_kernel, dim3(flat_grid(n, device_cus())), dim3(256), 0, stream, part, m, n);
+  CPG_HIP(hipGetLastError());
+}
+
 int sfxt_dataflow_grid(int blocks) {
   int per_cu = 0;
   CPG_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, sfxt_dataflow_kernel, kDfBlock, 0));
@@ -2072,7 +2243,10 @@ void launch_sfxt_init_multi(const SfxtArgs& args, const SfxtMulti& m, hipStream_
   CPG_HIP(hipGetLastError());
 }
 
-int sfxt_parts_capacity() { return resident_blocks(sfxt_levels_parts_kernel, kSfxtBlock); }
+int sfxt_parts_capacity() {
+  return std::min(resident_blocks(sfxt_levels_parts_kernel, kSfxtBlock),
+                  resident_blocks(sfxt_sched_multi_kernel, kSchedBlock));
+}
 
 void launch_sfxt_levels_parts(const SfxtParts& parts, int total_blocks, hipStream_t stream) {
   if (parts.n < 1 || parts.n > kMaxParts || total_blocks > sfxt_parts_capacity())

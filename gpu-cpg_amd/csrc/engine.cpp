@@ -175,6 +175,15 @@ double first_gap(const std::vector<float>& rc, float cmin, float max_abs_distf) 
                    std::fabs(static_cast<double>(cmin)) * 0x1p-8, static_cast<double>(max_abs_distf) * 0x1p-8, 1e-6});
 }
 
+// Parents a multi-query slot expands in its first round under a bound; the
+// rounds after it take four times the last, up to the target (as the single
+// query's rounds do; a batch of 48 designs 17.7 ms from the whole target, 16.0
+// from a quarter, 14.3 from a sixteenth, 14.4 from a 64th; 24 served queries
+// 25.6 / 23.6 / 24.4 / 24.3).
+unsigned long long first_target(unsigned long long target) {
+  return std::max<unsigned long long>(256, target / 16);
+}
+
 // A multi-query slot's first trial bound (see mq.hip).
 void start_trial(MqQuery& m, const std::vector<float>& rc, float cmin, float max_abs_distf) {
   m.trial = 1;
@@ -822,9 +831,10 @@ struct cpg_handle {
   // largest key of the histogram bin where the running count of the stored
   // paths reaches k (k distinct stored paths cost no more, so no path above
   // it can be among the k cheapest), and the roots count as expanded.
-  // Returns the bound's key, or kKeyInf when eight trials fall short, the
-  // roots and their children are fewer than k, or a trial overflows the
-  // node store (the rounds then start unbounded from the roots alone).
+  // Returns the bound's key, or kKeyInf when every trial falls short, the
+  // roots and their children are fewer than k, or no trial bound lies between
+  // too few paths and more than the node store holds (the rounds then start
+  // unbounded from the roots alone).
   uint32_t probe_bound(WalkArgs& wa, int64_t k, const std::vector<uint8_t>& kp,
                        const std::vector<int>& sd, float cmin, uint32_t klo, bool trace) {
     std::vector<float> rc;
@@ -836,31 +846,29 @@ struct cpg_handle {
     launch_iota(batch.p, nb, grid, stream);
     double gap = first_gap(rc, cmin, max_abs_distf);
     if (trace) std::fprintf(stderr, "probe: host preparation %.3f ms\n", now_ms() - tb0);
-    uint64_t prev_total = 0;
-    double prev_gap = gap;
+    uint64_t prev_total = 0;   // the widest trial that fell short
+    double prev_gap = 0.0;
+    double wide_gap = 0.0;     // the narrowest trial that overflowed the store (0: none)
     wa.strict = 0;  // a trial keeps the children at the trial bound itself
+    constexpr int kTrials = 24;
     int t = 0;
-    for (; t < 8; ++t) {
+    for (; t < kTrials; ++t) {
       const float u0 = static_cast<float>(static_cast<double>(cmin) + gap);
       const uint32_t uk = float_key(u0);
       launch_probe_setup(pctl.p, uk, window_shift(klo, uk), nb, nb, stream);
       launch_walk(wa, true, grid, stream);
       PfxtCtl pc = read_pctl();
       if (pc.err) throw std::runtime_error("PFXT walk exceeded its step bound");
-      if (pc.overflow) {  // the trial bound's children do not fit the store
-        probe_overflowed = true;
-        break;
-      }
       uint64_t roots_le = 0;
       for (float c : rc)
         if (c <= u0 && c != 0.0f) ++roots_le;
-      const uint64_t children = pc.node_n - nb;
+      const uint64_t children = pc.node_n - nb;  // counted past the store's end too
       const uint64_t total = roots_le + children;
       if (trace)
         std::fprintf(stderr, "probe %d bound %.9g roots %llu children %llu\n", t,
                      static_cast<double>(u0), static_cast<unsigned long long>(roots_le),
                      static_cast<unsigned long long>(children));
-      if (total >= static_cast<uint64_t>(k)) {
+      if (total >= static_cast<uint64_t>(k) && !pc.overflow) {
         // the stored roots and children give the crossing; the roots are
         // expanded (every child of theirs up to the trial bound is stored)
         CPG_HIP(hipMemsetAsync(n_flag.p, 1, nb, stream));
@@ -870,25 +878,39 @@ struct cpg_handle {
         timing.probes = t + 1;
         return pc.ukey;
       }
+      if (pc.overflow) wide_gap = gap;
       // a wider bound that finds nothing new means every child of every
       // root is already stored: k needs deeper paths, stop probing
-      if (t > 0 && total == prev_total) break;
-      // Counts grow steeply with the bound (children cluster in cost):
-      // model total ~ gap^alpha, alpha fitted to the last two trials (4 at
-      // first), aim 10% past k, and widen by at most 2x so that a
-      // successful trial stores at most the children of twice the needed
-      // width.
-      double alpha = 4.0;
-      if (t > 0 && prev_total > 0 && total > prev_total)
-        alpha = std::min(8.0, std::max(1.0, std::log(static_cast<double>(total) / prev_total) /
-                                                std::log(gap / prev_gap)));
-      prev_total = total;
-      prev_gap = gap;
+      else if (t > 0 && total == prev_total) break;
+      // Counts grow steeply with the bound (children cluster in cost): model
+      // total ~ gap^alpha, alpha fitted to this trial and the last that fell
+      // short (8 at first), aim 5% past k and widen by at most 1.5x, then 2x:
+      // the exponent itself grows with the gap (to ten and more on deep
+      // graphs).  A trial whose children do not fit the store narrows it
+      // instead; where nothing lies between the two (ties at one cost) the
+      // caller probes again in a larger store.
+      double alpha = 8.0;
+      if (prev_total > 0 && total > prev_total && gap > prev_gap)
+        alpha = std::min(32.0, std::max(1.0, std::log(static_cast<double>(total) / prev_total) /
+                                                 std::log(gap / prev_gap)));
       const double f = std::pow(static_cast<double>(k) / static_cast<double>(std::max<uint64_t>(total, 1)),
-                                1.0 / alpha) * 1.1;
-      gap *= std::min(2.0, std::max(1.1, f));
+                                1.0 / alpha) * 1.05;
+      double next = gap * (pc.overflow ? std::min(0.95, f) : std::min(prev_gap > 0.0 ? 2.0 : 1.5, std::max(1.05, f)));
+      if (!pc.overflow) {
+        prev_total = total;
+        prev_gap = gap;
+      }
+      if (wide_gap > 0.0) {
+        if (prev_gap >= wide_gap * 0.999) {
+          probe_overflowed = true;
+          break;
+        }
+        if (prev_gap > 0.0 && (next <= prev_gap || next >= wide_gap)) next = 0.5 * (prev_gap + wide_gap);
+      }
+      gap = next;
     }
-    timing.probes = std::min(t + 1, 8);
+    if (t == kTrials && wide_gap > 0.0) probe_overflowed = true;
+    timing.probes = std::min(t + 1, kTrials);
     launch_probe_setup(pctl.p, kKeyInf, window_shift(klo, kKeyInf), 0, nb, stream);
     CPG_HIP(hipMemsetAsync(hist_all.p, 0, sizeof(unsigned) * 2 * kHistBins, stream));
     return kKeyInf;
@@ -1039,6 +1061,19 @@ struct cpg_handle {
         launch_round_log(pctl.p, rlog.p, kRoundLog + 1, stream);
         CPG_HIP(hipEventRecord(round_event(0), stream));
       }
+      // Parents per round where k is past one batch: growing fourfold from
+      // k / 512.  While the bound is still loose the cheapest parents have
+      // hundreds of children under it, and a full first batch stores them all
+      // before the bound moves.  On 60K vertices of mean out-degree 26 and K =
+      // 900K a first round of 131K parents walked 51M children (the query 473
+      // ms, through a store overflow; 4.8 ms growing); on 189K / 14.5 49.8 ms
+      // and 4.4; on 1.5M / 2.7, K = 1M, 3.99 and 3.82.  Up to one batch the
+      // rounds start whole: there the loose round is bounded by k parents.
+      const bool grow = o.batch == 0 && static_cast<uint64_t>(k) > batch_target;
+      auto round_batch = [&](int round) {
+        return !grow || round >= 16 ? batch_target
+                                    : std::min<uint64_t>(batch_target, (static_cast<uint64_t>(k) / 512) << (2 * round));
+      };
       while (true) {
         if (r > 100000) throw std::runtime_error("PFXT round limit exceeded");
         if (now_ms() - tq0 > CPG_QUERY_LIMIT_MS) throw std::runtime_error("PFXT query exceeded its time limit");
@@ -1051,7 +1086,7 @@ struct cpg_handle {
           hist_nodes(0, true, false);
           // the first round expands every root, unless the probe already did
           const bool all_roots = r == 0 && !probed;
-          launch_select_batch(pctl.p, hist_pend.p, all_roots ? ~0ull : batch_target, stream);
+          launch_select_batch(pctl.p, hist_pend.p, all_roots ? ~0ull : round_batch(r), stream);
           launch_make_batch(ns, pctl.p, batch.p, grid, stream);
           if (kernel_timing) {
             ev_count.create();
@@ -1615,8 +1650,9 @@ struct cpg_batch {
       }
       m.shift = window_shift_bins(m.klo, m.ukey, kMqBins);
       m.k = static_cast<unsigned long long>(std::max<int64_t>(0, designs[q].k));
-      m.batch_target = std::max<unsigned long long>(
+      m.target_max = std::max<unsigned long long>(
           256, m.k / static_cast<unsigned long long>(std::max(1, tune.target_div[k_class(m.k)])));
+      m.batch_target = first_target(m.target_max);
       m.done = (cnt == 0 || m.k == 0) ? 1 : 0;
       m.vrec = uh.vrec.p;
       m.devinfo = uh.devinfo.p;
@@ -2035,7 +2071,8 @@ struct cpg_server {
     }
     m.shift = window_shift_bins(m.klo, m.ukey, kMqBins);
     m.k = static_cast<unsigned long long>(q.k);
-    m.batch_target = std::max<unsigned long long>(256, m.k / 8);
+    m.target_max = std::max<unsigned long long>(256, m.k / 8);
+    m.batch_target = first_target(m.target_max);
     m.done = (nkept == 0 || q.k == 0) ? 1 : 0;
     m.vrec = aq.vrec;
     m.devinfo = aq.devinfo;

@@ -276,7 +276,8 @@ struct MqQuery {
   uint32_t klo;                   // histogram window base key
   uint32_t shift;                 // histogram window shift
   unsigned long long k;           // paths asked for
-  unsigned long long batch_target;
+  unsigned long long batch_target;  // parents this round; grows fourfold a round up to target_max
+  unsigned long long target_max;
   int done;                       // nothing left to expand (or the slot is free)
   int rounds;
   // the query's deviation index: the batched designs share the union's,

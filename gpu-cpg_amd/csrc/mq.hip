@@ -334,11 +334,12 @@ __global__ void __launch_bounds__(kMqBlock) mq_walk_kernel(MqArgs a) {
 
 // Next bound of a query whose trial found too few paths (total < K_q).
 // Counts grow steeply with the bound: model total ~ gap^alpha, alpha fitted
-// to the last two trials (4 at first), aim 10% past K_q and widen by at most
-// 4x (a trial that is too wide stores nothing more, it only counts more).
-// Past every distance without a new path, or after kMqTrials, the query
-// goes on unbounded, all its roots at once.
-constexpr int kMqTrials = 16;
+// to the last two trials (8 at first), aim 5% past K_q and widen by at most
+// 1.5x, then 2x: the counts' exponent itself grows with the gap (to ten and
+// more on deep graphs), and a trial far too wide walks a hundred times the
+// paths of one more narrow trial.  Past every distance without a new path,
+// or after kMqTrials, the query goes on unbounded, all its roots at once.
+constexpr int kMqTrials = 24;
 __device__ inline void mq_widen(MqQuery* qs, unsigned long long total) {
   const double gap = qs->gap;
   qs->retry = 1;
@@ -348,14 +349,15 @@ __device__ inline void mq_widen(MqQuery* qs, unsigned long long total) {
     qs->ukey = kKeyInf;
     return;
   }
-  double alpha = 4.0;
+  double alpha = 8.0;
   if (qs->trial > 1 && qs->prev_total > 0 && total > qs->prev_total)
-    alpha = fmin(8.0, fmax(1.0, log(static_cast<double>(total) / static_cast<double>(qs->prev_total)) /
-                                    log(gap / qs->prev_gap)));
-  const double f = pow(static_cast<double>(qs->k) / static_cast<double>(total > 0 ? total : 1ull), 1.0 / alpha) * 1.1;
+    alpha = fmin(32.0, fmax(1.0, log(static_cast<double>(total) / static_cast<double>(qs->prev_total)) /
+                                     log(gap / qs->prev_gap)));
+  const double f = pow(static_cast<double>(qs->k) / static_cast<double>(total > 0 ? total : 1ull), 1.0 / alpha) * 1.05;
+  const double most = qs->trial == 1 ? 1.5 : 2.0;
   qs->prev_total = total;
   qs->prev_gap = gap;
-  qs->gap = gap * fmin(4.0, fmax(1.25, f));
+  qs->gap = gap * fmin(most, fmax(1.05, f));
   qs->trial += 1;
   qs->ukey = float_key(static_cast<float>(static_cast<double>(qs->cmin) + qs->gap));
 }
@@ -376,10 +378,14 @@ __global__ void __launch_bounds__(kMqSelBlock) mq_select_bound_kernel(MqArgs a) 
       const uint64_t up = static_cast<uint64_t>(qs->klo) + ((static_cast<uint64_t>(b) + 1) << qs->shift) - 1;
       if (up < uk) uk = static_cast<uint32_t>(up);
       qs->ukey = uk;
+      if (!qs->trial && qs->batch_target < qs->target_max)
+        qs->batch_target = qs->batch_target * 4 < qs->target_max ? qs->batch_target * 4 : qs->target_max;
       qs->trial = 0;
     } else if (qs->trial) {
       mq_widen(qs, total);
     }
+    else if (qs->batch_target < qs->target_max)
+      qs->batch_target = qs->batch_target * 4 < qs->target_max ? qs->batch_target * 4 : qs->target_max;
     qs->shift = mq_shift(qs->klo, qs->ukey);
     qs->rounds += 1;
   }

@@ -489,12 +489,21 @@ struct cpg_handle {
   // from the last levelization of this graph), within [16, 128] blocks; a
   // grid barrier per level costs more with more blocks.
   static constexpr int kXcds = 8;  // MI355X: 8 XCDs, workgroups dispatched round-robin
-  static constexpr int64_t kOneXcdRecords = 50000;  // fanin records per level kept on one XCD
+  static constexpr int64_t kOneXcdVertices = 2000;  // vertices per level kept on one XCD
+  int64_t level_width() const { return g.n / std::max(1, last_diameter); }
   int level_loop_blocks() const {
     if (sfxt_blocks > 0) return sfxt_blocks;
     if (last_diameter <= 0) return 64;
-    const int64_t per_level = g.n / last_diameter;
-    return static_cast<int>(std::min<int64_t>(128, std::max<int64_t>(16, (per_level + 255) / 256)));
+    return static_cast<int>(std::min<int64_t>(128, std::max<int64_t>(16, (level_width() + 255) / 256)));
+  }
+  // The edge-parallel loop's: about 8 queue entries per wave on one XCD, 16
+  // over all (where a level has work for every CU).
+  int edge_loop_blocks() const {
+    if (sfxt_blocks > 0) return sfxt_blocks;
+    if (last_diameter <= 0) return 64;
+    const int64_t w = level_width();
+    return static_cast<int>(w <= kOneXcdVertices ? std::min<int64_t>(64, std::max<int64_t>(16, w / 32))
+                                                 : std::min<int64_t>(128, std::max<int64_t>(64, w / 64)));
   }
 
   // Scheduled-loop grid: two waves per chunk of an average level, 16 to 128
@@ -673,29 +682,14 @@ struct cpg_handle {
       const bool scheduled = sfxt_method == 0 && sched_ready;
       if (!scheduled) order_ready = false;
       order_pending = !scheduled && (method == 1 || method >= 4);
-      // Its blocks on one XCD (round-robin dispatch puts every 8th block on
-      // the same XCD) while a level holds few fanin records, over all XCDs
-      // above that: on the 1.5M-vertex DAG (13.6K records per level) one
-      // XCD moves 459 MB per launch against 782 MB over all XCDs in the
-      // same time; the 30M-edge DAG (100K per level) runs 8.26 ms over all
-      // against 8.67 on one, the 256-design union graph 25 against 38 ms
-      const int64_t records_per_level = g.m / std::max(1, last_diameter);
-      a.place_stride = method == 5 && records_per_level <= kOneXcdRecords ? kXcds : 1;
-      // Queue entries per wave in that loop, on one XCD: as many as fill
-      // about one lane step of fanin records (64 x 3 records per step below
-      // a mean in-degree of 4, 64 x 8 above), at least 8, so that a level of
-      // few vertices with long in-degrees spreads over more waves.  The
-      // 2.6M-vertex graph of mean in-degree 27 (1,609 levels) takes 35.4 ms
-      // at 16 entries against 55.0 at 64, the 385K-vertex one 7.1 against
-      // 20.2; over all XCDs the 30M-edge DAG ran slower (11.2 against 8.4),
-      // so there every wave keeps 64.
-      int we = 64;
-      if (a.place_stride > 1) {
-        const double mean_in = static_cast<double>(g.m) / static_cast<double>(std::max(1, g.n));
-        const double per_step = 64.0 * (g.m < 4 * static_cast<int64_t>(g.n) ? 3 : 8);
-        while (we > 8 && we * mean_in > per_step) we >>= 1;
-      }
-      a.wave_entries = we;
+      // The edge-parallel loop's blocks share one XCD (round-robin dispatch
+      // puts every 8th block on the same one) where levels are narrow: the
+      // barrier is then cheaper (16 blocks 0.66 us, 0.87 over all XCDs).  Wide
+      // levels need more CUs for their atomics.  Best of one XCD / all: 447
+      // vertices a level 1.64 / 1.84 ms, 1,049 4.6 / 4.9, 5,000 (in-degree 2.7)
+      // 2.57 / 2.09, 5,000 (20) 1.92 / 1.38.  The first loop on a graph, its
+      // width unknown, runs over all.
+      a.place_stride = method == 5 && last_diameter > 0 && level_width() <= kOneXcdVertices ? kXcds : 1;
       const bool dataflow = method == 2;
       if (dataflow && relabelled)
         throw std::runtime_error("the dataflow SFXT loop does not run on a relabelled graph");
@@ -721,7 +715,7 @@ struct cpg_handle {
                            : dataflow    ? launch_sfxt_dataflow(a, df_grid, stream)
                            : method == 3 ? launch_sfxt_local(a, level_loop_blocks(), stream)
                            : method == 4 ? launch_sfxt_levels_nf(a, level_loop_blocks(), stream)
-                           : method == 5 ? launch_sfxt_levels_edges(a, level_loop_blocks(), stream)
+                           : method == 5 ? launch_sfxt_levels_edges(a, edge_loop_blocks(), stream)
                                          : launch_sfxt_levels(a, level_loop_blocks(), stream);
       if (kernel_timing) CPG_HIP(hipEventRecord(ev_levels.b, stream));
       if (relabelled && !scheduled) launch_sfxt_succ_relabel(succ.p, perm_d.p, g.n, stream);

@@ -36,7 +36,10 @@ constexpr size_t kScratchBytes = kOffLvlp + align_up(4ull * (kNoallocMaxVerts + 
 
 static __device__ __align__(256) unsigned char scratch[kScratchBytes];
 
-constexpr int kNoallocBlocks = 24;  // level-loop working blocks (levels of a few thousand vertices)
+// Level-loop working blocks, on one XCD: levels of at most about a thousand
+// vertices (the level count is not known before the loop).
+constexpr int kNoallocBlocks = 32;
+constexpr int kNoallocStride = 8;
 constexpr int kMaxDevices = 64;
 std::mutex g_mu;
 unsigned char* g_scratch[kMaxDevices] = {};
@@ -76,7 +79,7 @@ int sfxt_noalloc(int n, const int* oadjp, const int* iadjp, const int2* iedge, c
   unsigned char* base = scratch_ptr();
   SfxtArgs a{};
   a.n = n;
-  a.m = 0;  // list positions per lane step: 3 (the sparse case); the result does not depend on it
+  a.place_stride = kNoallocStride;
   a.nsinks = nsinks;
   a.oadjp = oadjp;
   a.iadjp = iadjp;

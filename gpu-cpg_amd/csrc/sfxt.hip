@@ -444,8 +444,11 @@ __device__ __forceinline__ int queue_entry(const SfxtArgs& a, unsigned i) {
 // as levels_loop<false>, with the fanin release spread over the records of
 // a wave's vertices instead of over one vertex per lane.
 //
-// A wave takes 64 queue entries at a time (one per lane; fewer, by
-// wave_entries, where in-degrees are long), settles them as above, and
+// A wave takes its share of the level's queue entries, at least 4 and at most
+// 64 (one per lane) at a time, so that narrow levels spread over every wave:
+// one CU does about 0.57 G scattered atomics a second, and a wave with 64
+// entries of a 350-vertex level kept six CUs busy and the others waiting.  It
+// settles them as above, and
 // prefix-sums their in-degrees over the wave; the wave's records
 // then form one flat list, handed out kS per lane step (lane l takes list
 // positions r0 + s*64 + l), and a lane finds the vertex owning its position
@@ -469,9 +472,6 @@ __device__ void levels_edges_loop(const SfxtArgs& a) {
   const int lane = __lane_id();
   const unsigned wave = static_cast<unsigned>(gtid) >> 6;
   const unsigned nwaves = nblocks * blockDim.x / 64u;
-  // entries per wave: fewer than 64 where in-degrees are long, so that a
-  // level's records spread over more waves (lanes past them hold none)
-  const unsigned we = a.wave_entries > 0 && a.wave_entries < 64 ? static_cast<unsigned>(a.wave_entries) : 64u;
   if (threadIdx.x == 0) s_qn = 0;
   __syncthreads();
 
@@ -487,7 +487,9 @@ __device__ void levels_edges_loop(const SfxtArgs& a) {
   float local_max = 0.0f;
   while (true) {
     if (gtid == 0) a.lvlp[d] = static_cast<int>(lb);
-    // wave-uniform loop over we-entry chunks of the level
+    // wave-uniform loop over we-entry chunks of the level (lanes past we hold
+    // no entry)
+    const unsigned we = min(64u, max(4u, (le - lb + nwaves - 1) / nwaves));
     for (unsigned i0 = lb + wave * we; i0 < le; i0 += nwaves * we) {
       const unsigned i = i0 + static_cast<unsigned>(lane);
       int b = 0, deg = 0, du = kIntMax, tie = 0;
@@ -577,10 +579,10 @@ __device__ void levels_edges_loop(const SfxtArgs& a) {
   }
 }
 
-// 3 list positions per lane step where the mean in-degree is under 4 (a
-// wave's 64 vertices then hold about 64 x 2.7 records: one step), 8 above.
-__global__ void __launch_bounds__(kSfxtBlock) sfxt_levels_e3_kernel(SfxtArgs a) { levels_edges_loop<3>(a); }
-__global__ void __launch_bounds__(kSfxtBlock) sfxt_levels_e8_kernel(SfxtArgs a) { levels_edges_loop<8>(a); }
+// One list position per lane step where the blocks share an XCD, two over all
+// XCDs (launch_sfxt_levels_edges).
+__global__ void __launch_bounds__(kSfxtBlock) sfxt_levels_e1_kernel(SfxtArgs a) { levels_edges_loop<1>(a); }
+__global__ void __launch_bounds__(kSfxtBlock) sfxt_levels_e2_kernel(SfxtArgs a) { levels_edges_loop<2>(a); }
 
 // ---------------------------------------------------------------------------
 // Dataflow loop: the same levelize / relax / successor results as the level
@@ -2094,9 +2096,11 @@ int launch_sfxt_levels_nf(const SfxtArgs& args, int blocks, hipStream_t stream) 
 }
 
 int launch_sfxt_levels_edges(const SfxtArgs& args, int blocks, hipStream_t stream) {
-  // mean in-degree m / n: under 4 -> 3 list positions per lane step, else 8
-  const int64_t m = args.m, n = std::max(1, args.n);
-  auto k = m < 4 * n ? sfxt_levels_e3_kernel : sfxt_levels_e8_kernel;
+  // positions past a wave's last record issue no-op atomics, so few per step:
+  // 1 / 2 / 3 / 8 positions take 1.52 / 1.55 / 1.67 / 2.65 ms on a 120K-vertex
+  // graph of 346 levels (one XCD), 2.23 / 2.09 / 2.19 / 3.09 on 1.5M vertices of
+  // 300 levels (all XCDs)
+  auto k = args.place_stride > 1 ? sfxt_levels_e1_kernel : sfxt_levels_e2_kernel;
   // place_stride launch blocks per working block (the others return at once)
   const int stride = std::max(1, args.place_stride);
   const int working = loop_grid(blocks, resident_blocks(k, kSfxtBlock) / stride);

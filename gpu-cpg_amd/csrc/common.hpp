@@ -61,6 +61,17 @@ __host__ __device__ inline uint32_t window_shift(uint32_t klo, uint32_t khi) {
   return window_shift_bins(klo, khi, kHistBins);
 }
 
+// Device-scope (relaxed) accesses to words that blocks of one launch pass to
+// each other.
+template <class T>
+__device__ inline T dev_load(const T* p) {
+  return __hip_atomic_load(const_cast<T*>(p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+template <class T>
+__device__ inline void dev_store(T* p, T v) {
+  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
 __device__ inline uint64_t lanemask_lt() { return __lanemask_lt(); }
 // Wave-aggregated reservation of one slot per lane with want != 0 on a
 // 64-bit counter; returns the lane's slot (undefined where want == 0).

@@ -812,10 +812,12 @@ struct cpg_handle {
     return NodeStore{n_cost.p, n_to.p, n_from.p, n_parent.p, n_level.p, n_key.p, n_flag.p, node_cap};
   }
 
-  // Histograms of the stored paths at or below the bound (see launch_hist_nodes).
-  void hist_nodes(int mode, bool with_pend, bool accumulate) {
-    launch_hist_nodes(node_store(), ckeys.p, node_cap, pctl.p, mode, with_pend, hist_part.p,
-                      hist_all.p, hist_pend.p, accumulate, stream);
+  // Histograms of the stored paths at or below the bound and the choice that
+  // follows (see launch_hist_select).
+  void hist_select(int mode, bool with_pend, bool accumulate, HistSelect select, unsigned long long target,
+                   unsigned long long nroots = 0) {
+    launch_hist_select(node_store(), ckeys.p, node_cap, pctl.p, mode, with_pend, hist_part.p, hist_all.p,
+                       hist_pend.p, accumulate, select, target, nroots, stream);
   }
 
   // Finds a finite first bound without walking the roots' whole chains:
@@ -866,8 +868,7 @@ struct cpg_handle {
         // the stored roots and children give the crossing; the roots are
         // expanded (every child of theirs up to the trial bound is stored)
         CPG_HIP(hipMemsetAsync(n_flag.p, 1, nb, stream));
-        hist_nodes(0, false, false);
-        launch_probe_finish(pctl.p, hist_all.p, static_cast<unsigned long long>(k), nb, stream);
+        hist_select(0, false, false, kSelectProbe, static_cast<unsigned long long>(k), nb);
         pc = read_pctl();
         timing.probes = t + 1;
         return pc.ukey;
@@ -906,7 +907,6 @@ struct cpg_handle {
     if (t == kTrials && wide_gap > 0.0) probe_overflowed = true;
     timing.probes = std::min(t + 1, kTrials);
     launch_probe_setup(pctl.p, kKeyInf, window_shift(klo, kKeyInf), 0, nb, stream);
-    CPG_HIP(hipMemsetAsync(hist_all.p, 0, sizeof(unsigned) * 2 * kHistBins, stream));
     return kKeyInf;
   }
 
@@ -1077,10 +1077,9 @@ struct cpg_handle {
         const bool count_pass = two_pass || ukey_host == kKeyInf;
         const int group = (!kernel_timing && !count_pass && bound_from_store) ? 4 : 1;
         for (int gi = 0; gi < group; ++gi, ++r) {
-          hist_nodes(0, true, false);
           // the first round expands every root, unless the probe already did
           const bool all_roots = r == 0 && !probed;
-          launch_select_batch(pctl.p, hist_pend.p, all_roots ? ~0ull : round_batch(r), stream);
+          hist_select(0, true, false, kSelectBatch, all_roots ? ~0ull : round_batch(r));
           launch_make_batch(ns, pctl.p, batch.p, grid, stream);
           if (kernel_timing) {
             ev_count.create();
@@ -1090,9 +1089,8 @@ struct cpg_handle {
           if (count_pass) {
             wa.strict = ukey_host == kKeyInf || bound_from_store ? 1 : 0;
             launch_walk(wa, false, grid, stream);
-            hist_nodes(2, false, true);
             if (kernel_timing) CPG_HIP(hipEventRecord(ev_count.b, stream));
-            launch_select_bound(pctl.p, hist_all.p, static_cast<unsigned long long>(k), stream);
+            hist_select(2, false, true, kSelectBound, static_cast<unsigned long long>(k));
             if (kernel_timing) CPG_HIP(hipEventRecord(ev_fill.a, stream));
             wa.strict = 0;
             launch_walk(wa, true, grid, stream);
@@ -1105,8 +1103,7 @@ struct cpg_handle {
             }
             launch_walk(wa, true, grid, stream);
             if (kernel_timing) CPG_HIP(hipEventRecord(ev_fill.b, stream));
-            hist_nodes(1, false, true);
-            launch_select_bound(pctl.p, hist_all.p, static_cast<unsigned long long>(k), stream);
+            hist_select(1, false, true, kSelectBound, static_cast<unsigned long long>(k));
           }
           if (step_times && r < kRoundLog) {
             launch_round_log(pctl.p, rlog.p, kRoundLog + 1, stream);

@@ -209,6 +209,8 @@ struct PfxtCtl {
   int rounds;
   int err;                         // a walk exceeded its step bound (corrupt index)
   unsigned long long nonmono;      // children whose cost came out below their parent's
+  unsigned ticket;                 // blocks of a histogram reduction that have finished (0 between launches)
+  unsigned pad;
 };
 
 // Prefix-tree node store: one slot per generated path, roots first.
@@ -245,23 +247,24 @@ void launch_roots(const int* srcs, const uint8_t* keep, int nsrc, const int* dis
 void launch_probe_setup(PfxtCtl* ctl, uint32_t ukey, uint32_t shift, unsigned long long nb,
                         unsigned long long nroots, hipStream_t s);
 void launch_iota(uint32_t* p, uint64_t n, int grid, hipStream_t s);
-void launch_probe_finish(PfxtCtl* ctl, unsigned* hist_all, unsigned long long k,
-                         unsigned long long nroots, hipStream_t s);
 // Histograms of stored paths (mode 0: all, 1: this round's children, 2: the
 // keys of the last count pass) into
 // hist_all (2 x kHistBins: counts of nonzero keys <= U, then each bin's
-// largest key) and, with_pend, hist_pend (unexpanded paths with key < U).
+// largest key) and, with_pend, hist_pend (unexpanded paths with key < U), and
+// the choice that follows from them, made by the reduction's last block:
+//   kSelectBatch  the batch threshold (target unexpanded paths), the round's
+//                 counters
+//   kSelectBound  the bound (the largest key of the bin where the count
+//                 reaches target)
+//   kSelectProbe  the bound of a successful probe over nroots roots
 // part holds 3 x kHistParts x kHistBins per-block partials.
-void launch_hist_nodes(const NodeStore& nodes, const uint32_t* ckeys, uint64_t ckeys_cap,
-                       PfxtCtl* ctl, int mode, bool with_pend, unsigned* part, unsigned* hist_all,
-                       unsigned* hist_pend, bool accumulate, hipStream_t s);
-void launch_select_batch(PfxtCtl* ctl, unsigned* hist_pend, unsigned long long batch_target,
-                         hipStream_t s);
+enum HistSelect { kSelectBatch, kSelectBound, kSelectProbe };
+void launch_hist_select(const NodeStore& nodes, const uint32_t* ckeys, uint64_t ckeys_cap, PfxtCtl* ctl, int mode,
+                        bool with_pend, unsigned* part, unsigned* hist_all, unsigned* hist_pend, bool accumulate,
+                        HistSelect select, unsigned long long target, unsigned long long nroots, hipStream_t s);
 void launch_make_batch(const NodeStore& nodes, PfxtCtl* ctl, uint32_t* batch, int grid,
                        hipStream_t s);
 void launch_walk(const WalkArgs& a, bool fill, int grid, hipStream_t s);
-void launch_select_bound(PfxtCtl* ctl, unsigned* hist_all, unsigned long long k,
-                         hipStream_t s);
 // rlog[rounds] = paths stored once `rounds` rounds have completed (rounds < cap).
 void launch_round_log(const PfxtCtl* ctl, unsigned long long* rlog, int cap, hipStream_t s);
 

@@ -39,51 +39,55 @@ namespace {
 
 constexpr int kBlock = 256;
 constexpr int kSelBlock = 1024;
+constexpr int kHistBlock = 1024;
 
 __device__ inline unsigned long long ld_u64(const unsigned long long* p) { return *p; }
 
-// Block-wide search for the first bin at which the running sum of h
-// reaches target (1-based count).  Returns kHistBins if the total is
-// smaller; *total receives the sum.  Must be called by all threads of a
-// kSelBlock block.
+// Block-wide search for the first bin at which the running sum of h (words
+// other blocks of the launch wrote) reaches target (1-based count).  Returns
+// kHistBins if the total is smaller; *total receives the sum.  Must be called
+// by all threads of a kSelBlock block.
 __device__ uint32_t find_crossing(const unsigned* h, unsigned long long target,
                                   unsigned long long* total) {
-  constexpr int kPer = kHistBins / kSelBlock;
-  __shared__ unsigned long long s_part[kSelBlock];
+  constexpr int kPer = kHistBins / kSelBlock, kW = kSelBlock / 64;
+  __shared__ unsigned s_wave[kW];
   __shared__ unsigned s_bin;
-  const int t = threadIdx.x;
-  unsigned long long mine = 0;
-  for (int i = 0; i < kPer; ++i) mine += h[t * kPer + i];
-  s_part[t] = mine;
+  const int t = threadIdx.x, lane = __lane_id(), wave = t >> 6;
+  unsigned v[kPer], mine = 0;  // a node store holds fewer than 2^31 paths
+#pragma unroll
+  for (int i = 0; i < kPer; ++i) {
+    v[i] = dev_load(h + t * kPer + i);
+    mine += v[i];
+  }
+  unsigned incl = mine;
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const unsigned x = __shfl_up(incl, o);
+    if (lane >= o) incl += x;
+  }
+  if (lane == 63) s_wave[wave] = incl;
   if (t == 0) s_bin = kHistBins;
   __syncthreads();
-  // inclusive scan (Hillis-Steele) over kSelBlock partial sums
-  for (int off = 1; off < kSelBlock; off <<= 1) {
-    const unsigned long long v = t >= off ? s_part[t - off] : 0ull;
-    __syncthreads();
-    s_part[t] += v;
-    __syncthreads();
+  unsigned before = 0, sum = 0;
+#pragma unroll
+  for (int w = 0; w < kW; ++w) {
+    const unsigned x = s_wave[w];
+    if (w < wave) before += x;
+    sum += x;
   }
-  const unsigned long long incl = s_part[t];
-  const unsigned long long excl = incl - mine;
-  *total = s_part[kSelBlock - 1];
-  if (excl < target && incl >= target) {
-    unsigned long long run = excl;
+  *total = sum;
+  unsigned long long run = before + incl - mine;
+  if (run < target && run + mine >= target) {
+#pragma unroll
     for (int i = 0; i < kPer; ++i) {
-      run += h[t * kPer + i];
-      if (run >= target) { s_bin = static_cast<uint32_t>(t * kPer + i); break; }
+      if (run < target && run + v[i] >= target) s_bin = static_cast<uint32_t>(t * kPer + i);
+      run += v[i];
     }
   }
   __syncthreads();
   const uint32_t b = s_bin;
   __syncthreads();
   return b;
-}
-
-// Clears a bound histogram: kHistBins counts followed by kHistBins per-bin
-// maximum keys.
-__device__ inline void clear_hist(unsigned* h) {
-  for (int i = threadIdx.x; i < 2 * kHistBins; i += blockDim.x) h[i] = 0;
 }
 
 __global__ void __launch_bounds__(kBlock) roots_kernel(const int* srcs, const uint8_t* keep, int nsrc,
@@ -111,6 +115,35 @@ __global__ void __launch_bounds__(kBlock) roots_kernel(const int* srcs, const ui
   }
 }
 
+// Slots one histogram pass covers: every stored path, this round's children,
+// or the keys a count pass wrote; [lo, nn) lies within the buffer (after a
+// node-store overflow node_n and fill_node_base exceed the capacity, and the
+// vector loop reads the group of four holding lo, so lo must not pass nn).
+__device__ inline void hist_range(const PfxtCtl* ctl, int mode, uint64_t cap, uint64_t ckeys_cap, uint64_t& lo,
+                                  uint64_t& nn) {
+  lo = 0;
+  if (mode == 2) {
+    const uint64_t c = ctl->child_n;
+    nn = c < ckeys_cap ? c : ckeys_cap;
+  } else {
+    const uint64_t c = ctl->node_n;
+    nn = c < cap ? c : cap;
+    if (mode == 1) {
+      const uint64_t b = ctl->fill_node_base;
+      lo = b < nn ? b : nn;
+    }
+  }
+}
+
+// Blocks that take part in a pass over that many slots: each leaves one
+// partial histogram of 48 KB, which the reduction reads again, so a small
+// store uses few (8,192 slots per block; one block up to there).
+constexpr uint64_t kHistChunk = 8192;
+__device__ inline unsigned hist_parts(uint64_t lo, uint64_t nn) {
+  const uint64_t p = (nn - lo + kHistChunk - 1) / kHistChunk;
+  return static_cast<unsigned>(p < 1 ? 1 : p > kHistParts ? kHistParts : p);
+}
+
 // Per-block histograms over the window (klo, shift), counted in LDS and
 // written out as one partial per block: the nonzero keys <= U with the
 // largest key of each bin, and (with_pend) the unexpanded paths with key
@@ -119,42 +152,31 @@ __global__ void __launch_bounds__(kBlock) roots_kernel(const int* srcs, const ui
 // (ckeys, no flags).  Each thread reads four consecutive keys and flags
 // with one vector load each (the arrays are padded to a multiple of four
 // slots).
-__global__ void __launch_bounds__(kBlock) hist_nodes_kernel(NodeStore nodes, const uint32_t* ckeys,
-                                                            uint64_t ckeys_cap, PfxtCtl* ctl,
-                                                            int mode, int with_pend,
-                                                            unsigned* part_all, unsigned* part_pend,
-                                                            unsigned* part_max) {
+__global__ void __launch_bounds__(kHistBlock) hist_nodes_kernel(NodeStore nodes, const uint32_t* ckeys,
+                                                                uint64_t ckeys_cap, const PfxtCtl* ctl,
+                                                                int mode, int with_pend,
+                                                                unsigned* part_all, unsigned* part_pend,
+                                                                unsigned* part_max) {
   __shared__ unsigned h_all[kHistBins];
   __shared__ unsigned h_pend[kHistBins];
   __shared__ unsigned h_max[kHistBins];
+  if (ctl->done) return;
+  uint64_t lo, nn;
+  hist_range(ctl, mode, nodes.cap, ckeys_cap, lo, nn);
+  const unsigned parts = hist_parts(lo, nn);
+  if (blockIdx.x >= parts) return;
   for (int j = threadIdx.x; j < kHistBins; j += blockDim.x) {
     h_all[j] = 0;
-    h_pend[j] = 0;
     h_max[j] = 0;
+    if (with_pend) h_pend[j] = 0;
   }
   __syncthreads();
-  // [lo, nn) within the buffer: after a node-store overflow node_n and
-  // fill_node_base exceed the capacity, and the vector loop below reads
-  // the group of four holding lo, so lo must not pass nn
-  uint64_t nn, lo = 0;
-  if (mode == 2) {
-    const uint64_t c = ctl->child_n;
-    nn = c < ckeys_cap ? c : ckeys_cap;
-  } else {
-    const uint64_t c = ctl->node_n;
-    nn = c < nodes.cap ? c : nodes.cap;
-    if (mode == 1) {
-      const uint64_t b = ctl->fill_node_base;
-      lo = b < nn ? b : nn;
-    }
-  }
-  if (ctl->done) lo = nn = 0;  // nothing left: write empty partials
   const uint32_t uk = ctl->ukey;
   const uint32_t klo = ctl->klo, shift = ctl->shift;
   const uint4* key4 = reinterpret_cast<const uint4*>(mode == 2 ? ckeys : nodes.key);
   const uint32_t* flag4 = reinterpret_cast<const uint32_t*>(nodes.flag);
   for (uint64_t g = lo / 4 + static_cast<uint64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-       g < (nn + 3) / 4; g += static_cast<uint64_t>(gridDim.x) * blockDim.x) {
+       g < (nn + 3) / 4; g += static_cast<uint64_t>(parts) * blockDim.x) {
     const uint4 kv = key4[g];
     const uint32_t fv = with_pend ? flag4[g] : 0u;
     const uint32_t ks[4] = {kv.x, kv.y, kv.z, kv.w};
@@ -172,69 +194,97 @@ __global__ void __launch_bounds__(kBlock) hist_nodes_kernel(NodeStore nodes, con
     }
   }
   __syncthreads();
-  unsigned* pa = part_all + static_cast<size_t>(blockIdx.x) * kHistBins;
-  unsigned* pp = part_pend + static_cast<size_t>(blockIdx.x) * kHistBins;
-  unsigned* pm = part_max + static_cast<size_t>(blockIdx.x) * kHistBins;
+  const size_t at = static_cast<size_t>(blockIdx.x) * kHistBins;
   for (int j = threadIdx.x; j < kHistBins; j += blockDim.x) {
-    pa[j] = h_all[j];
-    pm[j] = h_max[j];
-    if (with_pend) pp[j] = h_pend[j];
+    part_all[at + j] = h_all[j];
+    part_max[at + j] = h_max[j];
+    if (with_pend) part_pend[at + j] = h_pend[j];
   }
 }
 
-// Sums (or, take_max, takes the maximum of) the kHistParts per-block
-// partial histograms into out, combined with out when accumulate and
-// written over it otherwise.  A block of kRedBlock
-// threads covers 64 bins: each of its kRedBlock / 64 groups adds an
-// interleaved share of the partials with all its loads in flight, and the
-// groups' sums meet in LDS.
-constexpr int kRedBlock = 1024;
-constexpr int kRedGroups = kRedBlock / 64;
-constexpr int kRedPer = kHistParts / kRedGroups;
-static_assert(kHistParts % kRedGroups == 0, "partials split evenly over groups");
-
-__global__ void __launch_bounds__(kRedBlock) reduce_hist_kernel(const unsigned* part, unsigned* out,
-                                                                int accumulate, int take_max) {
-  __shared__ unsigned s_sum[kRedGroups][64];
+// Sums the pass's partials into hist_all (and hist_pend), takes the maximum of
+// the per-bin largest keys, combined with what is there when accumulate and
+// written over it otherwise; then the last block to finish makes the choice
+// (HistSelect).  A block of kSelBlock threads covers 64 bins of one plane
+// (blockIdx.y: counts, largest keys, unexpanded): its 16 groups of 64 lanes
+// add an interleaved share of the partials and meet in LDS.  What was a
+// reduction per plane and a one-block selection, four launches of about 3 us
+// each, twice a round, is one: on a 5K-vertex query the two kinds of kernels
+// took 330 of 850 us.
+__global__ void __launch_bounds__(kSelBlock) reduce_select_kernel(const unsigned* part, unsigned* hist_all,
+                                                                  unsigned* hist_pend, PfxtCtl* ctl, uint64_t cap,
+                                                                  uint64_t ckeys_cap, int mode, int accumulate,
+                                                                  int select, unsigned long long target,
+                                                                  unsigned long long nroots) {
+  constexpr int kGroups = kSelBlock / 64;
+  __shared__ unsigned s_sum[kGroups][64];
+  __shared__ int s_last;
+  if (ctl->done) return;
+  const size_t plane = static_cast<size_t>(kHistParts) * kHistBins;
+  uint64_t lo, nn;
+  hist_range(ctl, mode, cap, ckeys_cap, lo, nn);
+  const unsigned parts = hist_parts(lo, nn);
   const int lane = threadIdx.x & 63, grp = threadIdx.x >> 6;
   const int j = blockIdx.x * 64 + lane;
-  unsigned v[kRedPer];
-#pragma unroll
-  for (int q = 0; q < kRedPer; ++q)
-    v[q] = part[static_cast<size_t>(grp + q * kRedGroups) * kHistBins + j];
+  const bool take_max = blockIdx.y == 1;
+  // planes of part: counts, unexpanded, largest keys
+  const unsigned* src = part + (blockIdx.y == 0 ? 0 : blockIdx.y == 1 ? 2 * plane : plane);
+  unsigned* out = blockIdx.y == 0 ? hist_all : blockIdx.y == 1 ? hist_all + kHistBins : hist_pend;
   unsigned sum = 0;
-#pragma unroll
-  for (int q = 0; q < kRedPer; ++q) sum = take_max ? max(sum, v[q]) : sum + v[q];
+#pragma unroll 4
+  for (unsigned q = static_cast<unsigned>(grp); q < parts; q += kGroups) {
+    const unsigned v = src[static_cast<size_t>(q) * kHistBins + j];
+    sum = take_max ? max(sum, v) : sum + v;
+  }
   s_sum[grp][lane] = sum;
   __syncthreads();
   if (grp == 0) {
     unsigned tot = accumulate ? out[j] : 0u;
-    for (int g2 = 0; g2 < kRedGroups; ++g2)
-      tot = take_max ? max(tot, s_sum[g2][lane]) : tot + s_sum[g2][lane];
-    out[j] = tot;
+#pragma unroll
+    for (int g2 = 0; g2 < kGroups; ++g2) tot = take_max ? max(tot, s_sum[g2][lane]) : tot + s_sum[g2][lane];
+    dev_store(out + j, tot);
+    __builtin_amdgcn_s_waitcnt(0);  // landed before this block is counted
   }
-}
-
-__global__ void __launch_bounds__(kSelBlock) select_batch_kernel(PfxtCtl* ctl, unsigned* hist_pend,
-                                                                 unsigned long long target) {
-  if (ctl->done) return;
   __syncthreads();
   if (threadIdx.x == 0) {
+    const unsigned n = gridDim.x * gridDim.y;
+    s_last = __hip_atomic_fetch_add(&ctl->ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == n - 1;
+  }
+  __syncthreads();
+  if (!s_last) return;
+  unsigned long long total = 0;
+  const uint32_t b = find_crossing(select == kSelectBatch ? hist_pend : hist_all, target, &total);
+  if (threadIdx.x != 0) return;
+  ctl->ticket = 0;
+  const uint32_t uk = ctl->ukey;
+  if (select == kSelectBatch) {
     ctl->batch_n = 0;
     ctl->child_n = 0;
     ctl->fill_node_base = ctl->node_n;
-  }
-  unsigned long long total = 0;
-  const uint32_t b = find_crossing(hist_pend, target, &total);
-  if (threadIdx.x == 0) {
     if (total == 0) {
       ctl->done = 1;
     } else if (b >= static_cast<uint32_t>(kHistBins)) {
-      ctl->thkey = ctl->ukey;
+      ctl->thkey = uk;
     } else {
       const uint32_t up = bin_upper_key(b, ctl->klo, ctl->shift);
-      ctl->thkey = up < ctl->ukey ? up : ctl->ukey;
+      ctl->thkey = up < uk ? up : uk;
     }
+    return;
+  }
+  uint32_t nk = uk;
+  if (b < static_cast<uint32_t>(kHistBins)) {
+    const uint32_t top = dev_load(hist_all + kHistBins + b);  // largest key in the crossing bin
+    if (top < nk) nk = top;
+  }
+  ctl->ukey = nk;
+  ctl->shift = window_shift(ctl->klo, nk);
+  if (select == kSelectBound) {
+    ctl->expanded += ctl->batch_n;
+    ctl->rounds += 1;
+  } else {  // a probe's bound: at least target nonzero paths are stored, the roots count as expanded
+    ctl->batch_n = 0;
+    ctl->child_n = 0;
+    ctl->expanded += nroots;
   }
 }
 
@@ -400,26 +450,6 @@ __global__ void __launch_bounds__(kBlock) walk_kernel(WalkArgs a) {
   }
 }
 
-__global__ void __launch_bounds__(kSelBlock) select_bound_kernel(PfxtCtl* ctl, unsigned* hist_all,
-                                                                 unsigned long long k) {
-  if (ctl->done) return;
-  unsigned long long total = 0;
-  const uint32_t b = find_crossing(hist_all, k, &total);
-  if (threadIdx.x == 0) {
-    uint32_t uk = ctl->ukey;
-    if (b < static_cast<uint32_t>(kHistBins)) {
-      const uint32_t top = hist_all[kHistBins + b];  // largest key in the crossing bin
-      if (top < uk) uk = top;
-    }
-    ctl->ukey = uk;
-    ctl->shift = window_shift(ctl->klo, uk);
-    ctl->expanded += ctl->batch_n;
-    ctl->rounds += 1;
-  }
-  __syncthreads();
-  clear_hist(hist_all);
-}
-
 // Bound probe: the walk's inputs for one trial bound ukey over the roots
 // (node slots 0..nroots-1, listed in batch by iota_kernel); the node store
 // is cut back to the roots, dropping an earlier trial's children.
@@ -439,30 +469,6 @@ __global__ void iota_kernel(uint32_t* p, uint64_t n) {
   for (uint64_t i = static_cast<uint64_t>(blockIdx.x) * blockDim.x + threadIdx.x; i < n;
        i += static_cast<uint64_t>(gridDim.x) * blockDim.x)
     p[i] = static_cast<uint32_t>(i);
-}
-
-// Bound probe succeeded (at least k nonzero paths with cost <= the trial
-// bound are stored): the bound becomes the largest key of the bin where
-// the running count reaches k, and the nroots roots count as expanded.
-__global__ void __launch_bounds__(kSelBlock) probe_finish_kernel(PfxtCtl* ctl, unsigned* hist_all,
-                                                                 unsigned long long k,
-                                                                 unsigned long long nroots) {
-  unsigned long long total = 0;
-  const uint32_t b = find_crossing(hist_all, k, &total);
-  if (threadIdx.x == 0) {
-    uint32_t uk = ctl->ukey;
-    if (b < static_cast<uint32_t>(kHistBins)) {
-      const uint32_t top = hist_all[kHistBins + b];  // largest key in the crossing bin
-      if (top < uk) uk = top;
-    }
-    ctl->ukey = uk;
-    ctl->shift = window_shift(ctl->klo, uk);
-    ctl->batch_n = 0;
-    ctl->child_n = 0;
-    ctl->expanded += nroots;
-  }
-  __syncthreads();
-  clear_hist(hist_all);
 }
 
 }  // namespace
@@ -488,39 +494,16 @@ void launch_iota(uint32_t* p, uint64_t n, int grid, hipStream_t s) {
   CPG_HIP(hipGetLastError());
 }
 
-void launch_probe_finish(PfxtCtl* ctl, unsigned* hist_all, unsigned long long k,
-                         unsigned long long nroots, hipStream_t s) {
-  hipLaunchKernelGGL(probe_finish_kernel, dim3(1), dim3(kSelBlock), 0, s, ctl, hist_all, k, nroots);
-  CPG_HIP(hipGetLastError());
-}
-
-void launch_hist_nodes(const NodeStore& nodes, const uint32_t* ckeys, uint64_t ckeys_cap,
-                       PfxtCtl* ctl, int mode, bool with_pend, unsigned* part, unsigned* hist_all,
-                       unsigned* hist_pend, bool accumulate, hipStream_t s) {
+void launch_hist_select(const NodeStore& nodes, const uint32_t* ckeys, uint64_t ckeys_cap, PfxtCtl* ctl, int mode,
+                        bool with_pend, unsigned* part, unsigned* hist_all, unsigned* hist_pend, bool accumulate,
+                        HistSelect select, unsigned long long target, unsigned long long nroots, hipStream_t s) {
   const size_t plane = static_cast<size_t>(kHistParts) * kHistBins;
-  unsigned* part_all = part;
-  unsigned* part_pend = part + plane;
-  unsigned* part_max = part + 2 * plane;
-  hipLaunchKernelGGL(hist_nodes_kernel, dim3(kHistParts), dim3(kBlock), 0, s, nodes, ckeys,
-                     ckeys_cap, ctl, mode, with_pend ? 1 : 0, part_all, part_pend, part_max);
+  hipLaunchKernelGGL(hist_nodes_kernel, dim3(kHistParts), dim3(kHistBlock), 0, s, nodes, ckeys, ckeys_cap, ctl, mode,
+                     with_pend ? 1 : 0, part, part + plane, part + 2 * plane);
   CPG_HIP(hipGetLastError());
-  const int rg = kHistBins / 64;
-  const int acc = accumulate ? 1 : 0;
-  hipLaunchKernelGGL(reduce_hist_kernel, dim3(rg), dim3(kRedBlock), 0, s, part_all, hist_all, acc, 0);
-  CPG_HIP(hipGetLastError());
-  hipLaunchKernelGGL(reduce_hist_kernel, dim3(rg), dim3(kRedBlock), 0, s, part_max,
-                     hist_all + kHistBins, acc, 1);
-  CPG_HIP(hipGetLastError());
-  if (with_pend) {
-    hipLaunchKernelGGL(reduce_hist_kernel, dim3(rg), dim3(kRedBlock), 0, s, part_pend, hist_pend,
-                       acc, 0);
-    CPG_HIP(hipGetLastError());
-  }
-}
-
-void launch_select_batch(PfxtCtl* ctl, unsigned* hist_pend, unsigned long long target,
-                         hipStream_t s) {
-  hipLaunchKernelGGL(select_batch_kernel, dim3(1), dim3(kSelBlock), 0, s, ctl, hist_pend, target);
+  hipLaunchKernelGGL(reduce_select_kernel, dim3(kHistBins / 64, with_pend ? 3 : 2), dim3(kSelBlock), 0, s, part,
+                     hist_all, hist_pend, ctl, nodes.cap, ckeys_cap, mode, accumulate ? 1 : 0,
+                     static_cast<int>(select), target, nroots);
   CPG_HIP(hipGetLastError());
 }
 
@@ -557,11 +540,6 @@ __global__ void round_log_kernel(const PfxtCtl* ctl, unsigned long long* rlog, i
 
 void launch_round_log(const PfxtCtl* ctl, unsigned long long* rlog, int cap, hipStream_t s) {
   hipLaunchKernelGGL(round_log_kernel, dim3(1), dim3(1), 0, s, ctl, rlog, cap);
-  CPG_HIP(hipGetLastError());
-}
-
-void launch_select_bound(PfxtCtl* ctl, unsigned* hist_all, unsigned long long k, hipStream_t s) {
-  hipLaunchKernelGGL(select_bound_kernel, dim3(1), dim3(kSelBlock), 0, s, ctl, hist_all, k);
   CPG_HIP(hipGetLastError());
 }
 

@@ -47,3 +47,11 @@ def test_gpu_round_batches(fan, levels, width, ties):
 @pytest.mark.parametrize("nodes", [3000, 20000, 200000])
 def test_gpu_probe_in_a_small_store(nodes, ties):
     check(cpgamd, rows(12, 40, 60, 9, ties), [2000], bound_probe=1, max_nodes=nodes)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("probe", [1, -1])
+def test_gpu_histogram_parts(probe):
+    """Stores of one histogram block (8,192 paths) and just past it, of a few,
+    and of more than there are partials for."""
+    check(cpgamd, rows(6, 30, 300, 11, False), [2, 2000, 4000, 8000, 16000, 33000, 700000], bound_probe=probe)

@@ -1177,8 +1177,16 @@ struct cpg_handle {
     const unsigned long long nl = *h_nsel.p;
     ghist.reserve(sort_ghist_len(nl));
     SortBufs sb{{skey[0].p, skey[1].p}, {sval[0].p, sval[1].p}, ghist.p, nl};
-    const int bytes[6] = {0, 1, 4, 5, 6, 7};
-    const int res = radix_sort_pairs(sb, nl, bytes, 6, stream);
+    // Bytes in which the keys can differ: a path's level is at most the rounds
+    // (and the probe) that led to it, and with no child below its parent every
+    // cost lies between the cheapest root's and the bound.
+    int bytes[6], nbytes = 0;
+    bytes[nbytes++] = 0;
+    if (c.rounds + 2 >= 256) bytes[nbytes++] = 1;
+    const uint32_t differ = c.nonmono ? ~0u : float_key(minc) ^ c.ukey;
+    for (int b = 0; b < 4; ++b)
+      if (b == 0 || (differ >> (8 * b)) != 0) bytes[nbytes++] = 4 + b;
+    const int res = radix_sort_pairs(sb, nl, bytes, nbytes, stream);
     const uint64_t nout = std::min<uint64_t>(static_cast<uint64_t>(k), nl);
     r_cost.reserve(std::max<uint64_t>(1, nout));
     r_level.reserve(std::max<uint64_t>(1, nout)); r_from.reserve(std::max<uint64_t>(1, nout));

@@ -387,8 +387,9 @@ void launch_bvss_unpack(const uint64_t* key, uint64_t n, int vbits, int* of, int
                         hipStream_t s);
 
 // ---------------- final selection ----------------
-// Stable LSD radix sort of (key, value) pairs over the given key bytes (keys
-// alone where the value buffers are null).
+// Stable LSD radix sort of (key, value) pairs over the given key bytes, the
+// others being equal in all keys (keys alone where the value buffers are
+// null).  Returns the buffer the result is in.
 struct SortBufs {
   uint64_t* key[2];
   uint32_t* val[2];

@@ -15,14 +15,18 @@ namespace cpg {
 namespace {
 
 constexpr int kSortBlock = 256;
-constexpr int kItems = 16;
-constexpr int kTile = kSortBlock * kItems;
+// Keys per thread and tile: few up to kFewItems keys, where larger tiles
+// leave CUs idle and every tile works through its keys in 256-key steps.
+constexpr int kItemsFew = 4, kItemsMany = 16;
+constexpr uint64_t kFewItems = uint64_t(1) << 21;
 constexpr int kWaves = kSortBlock / 64;
 constexpr int kScanBlock = 1024;
 
+template <int kItems>
 __global__ void __launch_bounds__(kSortBlock) sort_hist_kernel(const uint64_t* key, uint64_t n,
                                                                int shift, unsigned* ghist,
                                                                uint64_t ntiles) {
+  constexpr int kTile = kSortBlock * kItems;
   __shared__ unsigned h[256];
   h[threadIdx.x] = 0;
   __syncthreads();
@@ -130,10 +134,12 @@ __global__ void __launch_bounds__(kRowBlock) sort_rowscan_kernel(unsigned* ghist
 }
 
 // goff: the row-scanned counts and, after them, the 256 digit totals.
+template <int kItems>
 __global__ void __launch_bounds__(kSortBlock) sort_scatter_kernel(const uint64_t* kin, const uint32_t* vin,
                                                                   uint64_t* kout, uint32_t* vout,
                                                                   uint64_t n, int shift,
                                                                   const unsigned* goff, uint64_t ntiles) {
+  constexpr int kTile = kSortBlock * kItems;
   __shared__ unsigned wcnt[kWaves][256];
   __shared__ unsigned run[256];
   __shared__ unsigned base[256];
@@ -180,6 +186,35 @@ __global__ void __launch_bounds__(kSortBlock) sort_scatter_kernel(const uint64_t
     }
     run[tid] += tot;
     __syncthreads();
+  }
+}
+
+// Up to kRankSort keys in one launch: a key's place is the number of keys
+// that order before it (smaller, or equal and earlier), counted against every
+// key in LDS tiles.  n^2 comparisons, but no pass over digits: 100 keys took
+// 90 us in six radix passes of three launches, most of it launches.
+constexpr uint64_t kRankSort = 8192;
+__global__ void __launch_bounds__(kSortBlock) rank_sort_kernel(const uint64_t* kin, const uint32_t* vin, uint64_t* kout,
+                                                               uint32_t* vout, unsigned n) {
+  constexpr unsigned kT = 1024;
+  __shared__ uint64_t s_key[kT];
+  const unsigned i = blockIdx.x * kSortBlock + threadIdx.x;
+  const uint64_t mine = i < n ? kin[i] : 0;
+  unsigned rank = 0;
+  for (unsigned t = 0; t < n; t += kT) {
+    const unsigned m = min(kT, n - t);
+    __syncthreads();
+    // places past the last key hold the largest value: they order before none
+    for (unsigned j = threadIdx.x; j < kT; j += kSortBlock) s_key[j] = j < m ? kin[t + j] : ~0ull;
+    __syncthreads();
+    // keys of the tile before i count when equal too
+    const unsigned before = i > t ? min(i - t, m) : 0u;
+#pragma unroll 8
+    for (unsigned j = 0; j < m; ++j) rank += s_key[j] < mine || (s_key[j] == mine && j < before) ? 1u : 0u;
+  }
+  if (i < n) {
+    kout[rank] = mine;
+    if (vin) vout[rank] = vin[i];
   }
 }
 
@@ -258,7 +293,10 @@ int grid_for(uint64_t n, int block) {
 
 }  // namespace
 
-uint64_t sort_tiles(uint64_t n) { return (n + kTile - 1) / kTile; }
+uint64_t sort_tiles(uint64_t n) {
+  const uint64_t tile = static_cast<uint64_t>(kSortBlock) * (n <= kFewItems ? kItemsFew : kItemsMany);
+  return (n + tile - 1) / tile;
+}
 uint64_t sort_ghist_len(uint64_t n) { return 256 * (std::max<uint64_t>(1, sort_tiles(n)) + 1); }
 
 void launch_exclusive_scan_u32(unsigned* p, uint64_t len, hipStream_t s) {
@@ -267,19 +305,33 @@ void launch_exclusive_scan_u32(unsigned* p, uint64_t len, hipStream_t s) {
   CPG_HIP(hipGetLastError());
 }
 
+namespace {
+template <int kItems>
+void sort_pass(const SortBufs& b, int cur, uint64_t n, int shift, uint64_t ntiles, hipStream_t s) {
+  const dim3 g(static_cast<unsigned>(ntiles));
+  hipLaunchKernelGGL(sort_hist_kernel<kItems>, g, dim3(kSortBlock), 0, s, b.key[cur], n, shift, b.ghist, ntiles);
+  CPG_HIP(hipGetLastError());
+  hipLaunchKernelGGL(sort_rowscan_kernel, dim3(256), dim3(kRowBlock), 0, s, b.ghist, ntiles);
+  CPG_HIP(hipGetLastError());
+  hipLaunchKernelGGL(sort_scatter_kernel<kItems>, g, dim3(kSortBlock), 0, s, b.key[cur], b.val[cur], b.key[cur ^ 1],
+                     b.val[cur ^ 1], n, shift, b.ghist, ntiles);
+  CPG_HIP(hipGetLastError());
+}
+}  // namespace
+
 int radix_sort_pairs(SortBufs& b, uint64_t n, const int* bytes, int nbytes, hipStream_t s) {
   int cur = 0;
   if (n <= 1) return cur;
+  if (n <= kRankSort) {
+    hipLaunchKernelGGL(rank_sort_kernel, dim3(static_cast<unsigned>((n + kSortBlock - 1) / kSortBlock)),
+                       dim3(kSortBlock), 0, s, b.key[0], b.val[0], b.key[1], b.val[1], static_cast<unsigned>(n));
+    CPG_HIP(hipGetLastError());
+    return 1;
+  }
   const uint64_t ntiles = sort_tiles(n);
   for (int p = 0; p < nbytes; ++p) {
-    const int shift = 8 * bytes[p];
-    hipLaunchKernelGGL(sort_hist_kernel, dim3(static_cast<unsigned>(ntiles)), dim3(kSortBlock), 0, s, b.key[cur], n, shift, b.ghist, ntiles);
-    CPG_HIP(hipGetLastError());
-    hipLaunchKernelGGL(sort_rowscan_kernel, dim3(256), dim3(kRowBlock), 0, s, b.ghist, ntiles);
-    CPG_HIP(hipGetLastError());
-    hipLaunchKernelGGL(sort_scatter_kernel, dim3(static_cast<unsigned>(ntiles)), dim3(kSortBlock), 0, s, 
-        b.key[cur], b.val[cur], b.key[cur ^ 1], b.val[cur ^ 1], n, shift, b.ghist, ntiles);
-    CPG_HIP(hipGetLastError());
+    if (n <= kFewItems) sort_pass<kItemsFew>(b, cur, n, 8 * bytes[p], ntiles, s);
+    else sort_pass<kItemsMany>(b, cur, n, 8 * bytes[p], ntiles, s);
     cur ^= 1;
   }
   return cur;

@@ -1653,6 +1653,7 @@ struct cpg_batch {
           256, m.k / static_cast<unsigned long long>(std::max(1, tune.target_div[k_class(m.k)])));
       m.batch_target = first_target(m.target_max);
       m.done = (cnt == 0 || m.k == 0) ? 1 : 0;
+      m.rebuild = 1;
       m.vrec = uh.vrec.p;
       m.devinfo = uh.devinfo.p;
       m.devs = uh.devs.p;
@@ -2073,6 +2074,7 @@ struct cpg_server {
     m.target_max = std::max<unsigned long long>(256, m.k / 8);
     m.batch_target = first_target(m.target_max);
     m.done = (nkept == 0 || q.k == 0) ? 1 : 0;
+    m.rebuild = 1;
     m.vrec = aq.vrec;
     m.devinfo = aq.devinfo;
     m.devs = aq.devs;

@@ -295,6 +295,8 @@ struct MqQuery {
   // trial's distance and path count
   int trial;
   int retry;                      // this round's trial fell short: nothing is stored
+  int rebuild;                    // the histograms are to be counted again from the store
+  int pad;
   float cmin;
   double gap;
   double prev_gap;
@@ -308,7 +310,7 @@ struct MqCtl {
   int overflow;
   int err;
   int active;                     // queries with unexpanded paths this round
-  int pad;
+  int rebuild;                    // queries whose histograms this round counts again
   unsigned long long nonmono;     // children whose cost came out below their parent's
 };
 
@@ -349,7 +351,6 @@ void launch_mq_compact(const MqArgs& a, uint64_t n, const NodeStore& dst, int* d
                        const unsigned* tile_off, int* newidx, uint64_t n_live, int grid,
                        hipStream_t s);
 void launch_exclusive_scan_u32(unsigned* p, uint64_t len, hipStream_t s);
-void launch_zero_active(MqCtl* ctl, hipStream_t s);
 
 // ---------------- BVSS deviation discovery ----------------
 struct BvssCtl {

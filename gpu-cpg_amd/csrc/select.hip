@@ -191,28 +191,35 @@ __global__ void __launch_bounds__(kSortBlock) sort_scatter_kernel(const uint64_t
 
 // Up to kRankSort keys in one launch: a key's place is the number of keys
 // that order before it (smaller, or equal and earlier), counted against every
-// key in LDS tiles.  n^2 comparisons, but no pass over digits: 100 keys took
-// 90 us in six radix passes of three launches, most of it launches.
+// key in LDS tiles by kRankLanes lanes per key.  n^2 comparisons, but no pass
+// over digits: 100 keys took 90 us in six radix passes of three launches,
+// most of it launches.
 constexpr uint64_t kRankSort = 8192;
+constexpr unsigned kRankLanes = 8;
 __global__ void __launch_bounds__(kSortBlock) rank_sort_kernel(const uint64_t* kin, const uint32_t* vin, uint64_t* kout,
                                                                uint32_t* vout, unsigned n) {
-  constexpr unsigned kT = 1024;
+  constexpr unsigned kT = 2048;
   __shared__ uint64_t s_key[kT];
-  const unsigned i = blockIdx.x * kSortBlock + threadIdx.x;
+  const unsigned sub = threadIdx.x % kRankLanes;
+  const unsigned i = (blockIdx.x * kSortBlock + threadIdx.x) / kRankLanes;
   const uint64_t mine = i < n ? kin[i] : 0;
   unsigned rank = 0;
   for (unsigned t = 0; t < n; t += kT) {
     const unsigned m = min(kT, n - t);
     __syncthreads();
-    // places past the last key hold the largest value: they order before none
-    for (unsigned j = threadIdx.x; j < kT; j += kSortBlock) s_key[j] = j < m ? kin[t + j] : ~0ull;
+    for (unsigned j = threadIdx.x; j < m; j += kSortBlock) s_key[j] = kin[t + j];
     __syncthreads();
     // keys of the tile before i count when equal too
     const unsigned before = i > t ? min(i - t, m) : 0u;
 #pragma unroll 8
-    for (unsigned j = 0; j < m; ++j) rank += s_key[j] < mine || (s_key[j] == mine && j < before) ? 1u : 0u;
+    for (unsigned j = sub; j < m; j += kRankLanes) {
+      const uint64_t k = s_key[j];
+      rank += k < mine || (k == mine && j < before) ? 1u : 0u;
+    }
   }
-  if (i < n) {
+#pragma unroll
+  for (unsigned o = 1; o < kRankLanes; o <<= 1) rank += __shfl_xor(rank, static_cast<int>(o));
+  if (i < n && sub == 0) {
     kout[rank] = mine;
     if (vin) vout[rank] = vin[i];
   }
@@ -323,7 +330,7 @@ int radix_sort_pairs(SortBufs& b, uint64_t n, const int* bytes, int nbytes, hipS
   int cur = 0;
   if (n <= 1) return cur;
   if (n <= kRankSort) {
-    hipLaunchKernelGGL(rank_sort_kernel, dim3(static_cast<unsigned>((n + kSortBlock - 1) / kSortBlock)),
+    hipLaunchKernelGGL(rank_sort_kernel, dim3(static_cast<unsigned>((n * kRankLanes + kSortBlock - 1) / kSortBlock)),
                        dim3(kSortBlock), 0, s, b.key[0], b.val[0], b.key[1], b.val[1], static_cast<unsigned>(n));
     CPG_HIP(hipGetLastError());
     return 1;

@@ -226,41 +226,37 @@ __global__ void __launch_bounds__(kSortBlock) rank_sort_kernel(const uint64_t* k
 }
 
 // Sort input: the stored paths with a nonzero key <= U as
-// (key << 32 | level) -> node index; *count receives their number.  A
-// thread takes eight consecutive slots (two 16-byte key loads).
+// (key << 32 | level) -> node index; *count receives their number.  Tiles as
+// make_batch_kernel's.
 __global__ void __launch_bounds__(256) build_keys_kernel(NodeStore nodes, const PfxtCtl* ctl,
                                                          uint64_t* key, uint32_t* val,
                                                          unsigned long long* count) {
   const uint64_t n = ctl->node_n < nodes.cap ? ctl->node_n : nodes.cap;
   const uint32_t uk = ctl->ukey;
-  constexpr uint64_t kT = 256ull * 8;
+  constexpr int kSub = 4;
+  constexpr uint64_t kStep = 256ull * 8, kT = kStep * kSub;
   const uint4* key4 = reinterpret_cast<const uint4*>(nodes.key);
   for (uint64_t base = static_cast<uint64_t>(blockIdx.x) * kT; base < n;
        base += static_cast<uint64_t>(gridDim.x) * kT) {
     const uint64_t i0 = base + 8ull * threadIdx.x;
-    unsigned mask = 0, cnt = 0;
-    uint32_t ks[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-    if (i0 < n) {
-      const uint4 ka = key4[i0 / 4], kb = key4[i0 / 4 + 1];
-      ks[0] = ka.x; ks[1] = ka.y; ks[2] = ka.z; ks[3] = ka.w;
-      ks[4] = kb.x; ks[5] = kb.y; ks[6] = kb.z; ks[7] = kb.w;
+    uint32_t mask = 0;  // byte s: the thread's slots of step s
 #pragma unroll
-      for (int q = 0; q < 8; ++q) {
-        if (i0 + q < n && ks[q] <= uk && !key_is_zero(ks[q])) {
-          mask |= 1u << q;
-          ++cnt;
-        }
-      }
+    for (int s = 0; s < kSub; ++s) {
+      const uint64_t i = i0 + s * kStep;
+      if (i >= n) continue;
+      const uint4 ka = key4[i / 4], kb = key4[i / 4 + 1];
+      const uint32_t ks[8] = {ka.x, ka.y, ka.z, ka.w, kb.x, kb.y, kb.z, kb.w};
+#pragma unroll
+      for (int q = 0; q < 8; ++q)
+        if (i + q < n && ks[q] <= uk && !key_is_zero(ks[q])) mask |= 1u << (8 * s + q);
     }
-    uint64_t slot = block_reserve<256>(count, cnt);
-#pragma unroll
-    for (int q = 0; q < 8; ++q) {
-      if (mask & (1u << q)) {
-        key[slot] = (static_cast<uint64_t>(ks[q]) << 32) |
-                    static_cast<uint32_t>(nodes.level[i0 + q]);
-        val[slot] = static_cast<uint32_t>(i0 + q);
-        ++slot;
-      }
+    uint64_t slot = block_reserve<256>(count, static_cast<unsigned>(__popcll(mask)));
+    for (; mask; mask &= mask - 1) {
+      const int j = __ffsll(static_cast<long long>(mask)) - 1;
+      const uint64_t i = i0 + static_cast<uint64_t>(j >> 3) * kStep + static_cast<uint64_t>(j & 7);
+      key[slot] = (static_cast<uint64_t>(nodes.key[i]) << 32) | static_cast<uint32_t>(nodes.level[i]);
+      val[slot] = static_cast<uint32_t>(i);
+      ++slot;
     }
   }
 }

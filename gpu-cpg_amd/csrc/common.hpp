@@ -73,6 +73,26 @@ __device__ inline void dev_store(T* p, T v) {
 }
 
 __device__ inline uint64_t lanemask_lt() { return __lanemask_lt(); }
+// v of another lane of the same row of 16, by a DPP move (a few cycles; a
+// shuffle through LDS takes about a hundred).
+template <int kCtrl>
+__device__ __forceinline__ int dpp_move(int v) {
+  return __builtin_amdgcn_update_dpp(v, v, kCtrl, 0xf, 0xf, false);
+}
+// op over each aligned group of kLanes lanes, the result in all of them: lane
+// exchanges within a quad, mirrored halves of 8 and 16 (a quad's lanes, then a
+// half row's, hold one value by then), shuffles across rows.
+template <int kLanes, class Op>
+__device__ __forceinline__ int group_reduce(int v, Op op) {
+  if (kLanes > 1) v = op(v, dpp_move<0xB1>(v));   // quad_perm 1 0 3 2
+  if (kLanes > 2) v = op(v, dpp_move<0x4E>(v));   // quad_perm 2 3 0 1
+  if (kLanes > 4) v = op(v, dpp_move<0x141>(v));  // row_half_mirror
+  if (kLanes > 8) v = op(v, dpp_move<0x140>(v));  // row_mirror
+  if (kLanes > 16) v = op(v, __shfl_xor(v, 16));
+  if (kLanes > 32) v = op(v, __shfl_xor(v, 32));
+  return v;
+}
+
 // Wave-aggregated reservation of one slot per lane with want != 0 on a
 // 64-bit counter; returns the lane's slot (undefined where want == 0).
 __device__ inline uint64_t wave_reserve(unsigned long long* counter, bool want) {

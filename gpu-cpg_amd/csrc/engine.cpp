@@ -599,6 +599,13 @@ struct cpg_handle {
     sched.first = L > 1 ? pad[1] : static_cast<int>(np);
     sched.nl = nl;
     sched.lanes = lanes;
+    // A row past one load costs its level another round trip, and on narrow
+    // levels every level waits for its longest row: four records per lane
+    // there when some row needs them (250K vertices, out-degrees to 108: 1.63
+    // -> 1.28 ms; 200K, to 32: 0.65 -> 0.62).  Wide levels have other chunks to
+    // turn to, and the empty places cost them loads (1.5M vertices: 0.67 ->
+    // 0.72 ms).
+    sched.steps = L > 0 && nl / L <= kOneXcdVertices && g.max_out_degree > 3 * lanes ? 4 : 2;
     sched.pos = pos_d;
     sched.ofs = reinterpret_cast<const int*>(ofs_d);
     sched.edge = edge_d;

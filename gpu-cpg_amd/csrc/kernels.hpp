@@ -77,6 +77,7 @@ struct SfxtSched {
   int first;         // first position of level 1 (level 0: the sinks, in list order)
   int nl;            // levelized vertices
   int lanes;         // lanes per vertex: 1, 2, 4, 8, 16, 32 or 64
+  int steps;         // records a lane has in flight: 2, or 4 (4 to 32 lanes)
   const int* pos;    // position of each vertex (-1: never levelized), n
   const int* ofs;    // fanout records of each position, np + 1
   const int2* edge;  // {position of w, (int)(w_e * 10000.0f)}

@@ -1234,11 +1234,8 @@ __global__ void __launch_bounds__(kSchedBlock) sfxt_sched_kernel(SchedArgs a) {
       load(r0);
       settle(r0);
     }
-#pragma unroll
-    for (int o = 1; o < kLanes; o <<= 1) {
-      bd = min(bd, __shfl_xor(bd, o));
-      lev = max(lev, __shfl_xor(lev, o));
-    }
+    bd = group_reduce<kLanes>(bd, [](int x, int y) { return min(x, y); });
+    lev = group_reduce<kLanes>(lev, [](int x, int y) { return max(x, y); });
     if (sub == 0 && b0 < e0)  // a padding position has no records and is never read
       st_dev64(a.state + c * kV + grp,
                (static_cast<unsigned long long>(static_cast<uint32_t>(lev)) << 32) | static_cast<uint32_t>(bd));
@@ -2148,10 +2145,10 @@ int launch_sfxt_scheduled(const SfxtArgs& args, const SfxtSched& s, int blocks, 
     switch (s.lanes) {
       case 1: used = launch_sched_loop<1, 4>(a, blocks, stream); break;
       case 2: used = launch_sched_loop<2, 4>(a, blocks, stream); break;
-      case 4: used = launch_sched_loop<4, 2>(a, blocks, stream); break;
-      case 8: used = launch_sched_loop<8, 2>(a, blocks, stream); break;
-      case 16: used = launch_sched_loop<16, 2>(a, blocks, stream); break;
-      case 32: used = launch_sched_loop<32, 2>(a, blocks, stream); break;
+      case 4: used = s.steps > 2 ? launch_sched_loop<4, 4>(a, blocks, stream) : launch_sched_loop<4, 2>(a, blocks, stream); break;
+      case 8: used = s.steps > 2 ? launch_sched_loop<8, 4>(a, blocks, stream) : launch_sched_loop<8, 2>(a, blocks, stream); break;
+      case 16: used = s.steps > 2 ? launch_sched_loop<16, 4>(a, blocks, stream) : launch_sched_loop<16, 2>(a, blocks, stream); break;
+      case 32: used = s.steps > 2 ? launch_sched_loop<32, 4>(a, blocks, stream) : launch_sched_loop<32, 2>(a, blocks, stream); break;
       case 64: used = launch_sched_loop<64, 2>(a, blocks, stream); break;
       default: throw std::runtime_error("scheduled SFXT loop: lanes per vertex must be a power of two up to 64");
     }

@@ -154,6 +154,17 @@ inline simt_v4i __builtin_amdgcn_mfma_i32_16x16x64_i8(simt_v4i a, simt_v4i b, si
   return d;
 }
 // every live lane of the wave meets here, as the wave does in lockstep
+// DPP moves within rows of 16 lanes: quad permutations, mirrored half rows
+// and rows (row and bank masks all set).
+inline int __builtin_amdgcn_update_dpp(int, int v, int ctrl, int, int, bool) {
+  const int l = __lane_id();
+  int from = l;
+  if (ctrl < 0x100) from = (l & ~3) | ((ctrl >> (2 * (l & 3))) & 3);
+  else if (ctrl == 0x140) from = l ^ 15;
+  else if (ctrl == 0x141) from = l ^ 7;
+  else std::abort();
+  return __shfl(v, from);
+}
 inline void __builtin_amdgcn_wave_barrier() { (void)simt::wave_sync(0); }
 
 template <class T>

@@ -46,6 +46,9 @@ SHAPES = {
     "mean6": lambda: layered([33, 100, 31, 32, 17], 6, 3),
     "mean12": lambda: layered([50, 60, 70, 20], 12, 4),
     "dense_hub": lambda: layered([20, 90, 90, 40], 24, 5, hub=200),
+    "sparse_hub": lambda: layered([9, 70, 130, 64, 30], 1, 8, hub=60),
+    "mean3_hub": lambda: layered([40] * 9, 3, 9, hub=90),
+    "mean6_hub": lambda: layered([33, 100, 31, 32, 17], 6, 10, hub=120),
     "chain": lambda: (19, np.arange(18, dtype=np.int32), np.arange(1, 19, dtype=np.int32),
                       np.linspace(0.01, 0.9, 18, dtype=np.float32)),
     "one_edge": lambda: (2, np.array([1], np.int32), np.array([0], np.int32), np.array([0.5], np.float32)),

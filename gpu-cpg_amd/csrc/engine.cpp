@@ -1031,8 +1031,16 @@ struct cpg_handle {
       wa.step_limit = step_limit();
       wa.lanes = g.m < 3 * static_cast<int64_t>(g.n) ? 2 : 4;
       const int64_t nkept = nroots - dropped;
-      const bool probe = nkept > 0 && (o.bound_probe > 0 ||
-                                       (o.bound_probe == 0 && nkept * (diameter + 1) > (1 << 20)));
+      // Without a probe the first round walks every root's whole chain and all
+      // its deviations, so the probe runs where those are many: chain vertices,
+      // or edges off them (400K vertices, 8,000 roots of 80 levels, mean
+      // out-degree 20: 2.24 ms without, 1.92 with; 129K of 231 levels, 9.9: 1.30
+      // and 1.09; 98K of 312, 3.5, a quarter of the line: 1.95 and 2.16).
+      const int64_t chain = nkept * (static_cast<int64_t>(diameter) + 1);
+      const bool long_walks = chain > (1 << 20) ||
+                              static_cast<double>(chain) * static_cast<double>(g.m) >
+                                  static_cast<double>(1 << 22) * static_cast<double>(g.n);
+      const bool probe = nkept > 0 && (o.bound_probe > 0 || (o.bound_probe == 0 && long_walks));
       uint32_t ukey_host = kKeyInf;
       const double tpr0 = now_ms();
       if (trace) std::fprintf(stderr, "query roots: buffers, flags and root launch %.3f ms\n", tpr0 - tp0);
@@ -1082,7 +1090,9 @@ struct cpg_handle {
         // the same fill-only sequence and every kernel does nothing after
         // the done flag is set: launch a group of rounds per host sync.
         const bool count_pass = two_pass || ukey_host == kKeyInf;
-        const int group = (!kernel_timing && !count_pass && bound_from_store) ? 4 : 1;
+        // A small last batch is near the end: two rounds, so that few are
+        // launched after it.
+        const int group = (!kernel_timing && !count_pass && bound_from_store) ? (r > 0 && c.batch_n < 256 ? 2 : 4) : 1;
         for (int gi = 0; gi < group; ++gi, ++r) {
           // the first round expands every root, unless the probe already did
           const bool all_roots = r == 0 && !probed;

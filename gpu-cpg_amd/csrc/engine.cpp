@@ -1700,7 +1700,7 @@ struct cpg_batch {
         const int group = r == 0 ? 1 : std::max(1, tune.group);
         const int rgrid = std::max(1, uh.grid / 8 * std::max(1, tune.grid_mult));
         if (r == 0) {
-          launch_mq_round(a, false, rgrid, stream);
+          launch_mq_round(a, rgrid, stream);
         } else {
           // the captured round holds buffer addresses and sizes: capture
           // again whenever any of them changed (node store growth, designs
@@ -1709,7 +1709,7 @@ struct cpg_batch {
             drop_graph();
           if (!graph_exec) {
             CPG_HIP(hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal));
-            launch_mq_round(a, false, rgrid, stream);
+            launch_mq_round(a, rgrid, stream);
             CPG_HIP(hipStreamEndCapture(stream, &graph));
             CPG_HIP(hipGraphInstantiate(&graph_exec, graph, nullptr, nullptr, 0));
             graph_args = a;
@@ -1789,9 +1789,9 @@ struct cpg_batch {
 //
 // A query is admitted between rounds when a slot is free and the device
 // bytes of the in-flight queries' deviation indexes stay within the
-// budget.  Admission runs the query's SFXT for its endpoint subset on its
-// graph's handle and takes the index buffers over (a buffer swap, no
-// copy), then appends its roots to the shared node store; every round then
+// budget.  Its graph's admission group runs the SFXT for its endpoint
+// subset into index buffers of its own; its roots are then appended to the
+// shared node store with a trial bound; every round then
 // expands every in-flight query at once (the multi-query kernels of
 // mq.hip, each query reading its own index).  A query whose expansion is
 // done is extracted at the end of that round (its paths sorted by cost),
@@ -1853,7 +1853,7 @@ struct cpg_server {
     int state = 0;              // 0 queued, 1 in flight, 2 done
     std::unique_ptr<IndexSet> index;
     std::vector<int> roots;     // kept roots (vertex ids, ascending)
-    uint64_t seed_n = 0;        // paths of the first-bound probe left in the graph handle's store
+    uint64_t seed_n = 0;        // roots left in the graph handle's store until admission
     int64_t node_est = 0;       // node-store estimate held while admitted (0 = not held)
     MqQuery init{};             // slot state at admission
     std::vector<float> result;
@@ -1928,7 +1928,7 @@ struct cpg_server {
   bool ready = false;
   hipStream_t sstream = nullptr;  // level-loop launches of admission groups
   hipEvent_t ev_levels = nullptr;
-  std::mutex stats_mu;  // statistics the probes of several graphs update
+  std::mutex stats_mu;  // statistics the seedings of several graphs update
   int parts_cap = 1;              // blocks one partitioned level-loop launch keeps resident
 
   uint64_t first_cap = uint64_t(1) << 24;
@@ -2014,14 +2014,11 @@ struct cpg_server {
     return a;
   }
 
-  // The first bound of query q, whose SFXT columns and index are in place:
-  // its roots, then the single query's probe on the graph handle's own node
-  // store, which stores the roots (expanded) and their children up to a
-  // bound u0 under which at least k paths lie (admission copies them into
-  // the shared store, so the query's rounds start where a single query's
-  // would).  A probe that finds no bound leaves the roots alone (u0 = no
-  // bound, the first round expands them all).
-  void probe_query(Query& q, cpg_handle& h, const SfxtArgs& aq, float max_abs_distf) {
+  // Seeds query q, whose SFXT columns and index are in place: its roots
+  // (unexpanded) in the graph handle's own node store, from which admission
+  // copies them into the shared store, and its first bound: the k-th root's
+  // cost or a trial bound that the shared rounds widen or confirm.
+  void seed_query(Query& q, cpg_handle& h, const SfxtArgs& aq, float max_abs_distf) {
     const int nsrc = static_cast<int>(h.g.srcs.size());
     std::vector<int> sd(nsrc);
     h.src_dist.reserve(std::max(1, nsrc));
@@ -2037,8 +2034,7 @@ struct cpg_server {
     uint32_t u0 = kKeyInf;
     q.seed_n = 0;
     // At least k nonzero roots: the k-th smallest root cost bounds the
-    // answer already (roots are paths), and the rounds start from the
-    // roots alone, unexpanded, with no probe walks.
+    // answer already (roots are paths), and needs no trial.
     std::vector<float> rc;
     for (int i = 0; i < nsrc; ++i)
       if (kp[i]) {
@@ -2048,8 +2044,8 @@ struct cpg_server {
     // The K-th root cost bounds the answer, but loosely: the children of
     // the cheapest roots are cheaper than the K-th root, and a first round
     // under that bound stores every child up to it.  It is taken only
-    // where the roots' chains are short (the single query's rule for
-    // skipping its probe); otherwise the probe finds a tight bound.
+    // where the roots' chains are short; otherwise a trial finds a tighter
+    // bound.
     const bool short_chains = nkept * (static_cast<int64_t>(h.diameter) + 1) <= (int64_t(1) << 20);
     bool trial = false;
     // the roots in the graph handle's node store, for admission to copy
@@ -2100,7 +2096,7 @@ struct cpg_server {
     q.init = m;
   }
 
-  // Puts q in its reserved slot and copies its first-bound paths (still in
+  // Puts q in its reserved slot and copies its roots (still in
   // the graph handle's node store) into the shared store.  The server
   // stream must be idle (no round running).
   void admit_one(Query& q) {
@@ -2317,11 +2313,11 @@ struct cpg_server {
   }
 
   // Completes started groups whose stream work has finished: checks each
-  // group's level loop and indexes, then gives every query its first bound
-  // and admits it.  The server stream must be idle.  A graph's queries are
-  // probed one after another (a probe leaves its paths in the graph
-  // handle's node store until admission has copied them), but the graphs'
-  // probes run on host threads of their own, each on its graph's stream;
+  // group's level loop and indexes, then seeds every query and admits it.
+  // The server stream must be idle.  A graph's queries are seeded one after
+  // another (the roots stay in the graph handle's node store until
+  // admission has copied them), but the graphs'
+  // seedings run on host threads of their own, each on its graph's stream;
   // admissions, which use the shared store and the server stream, take a
   // lock one at a time.
   void finish_groups(const std::vector<int>& gis) {
@@ -2349,7 +2345,7 @@ struct cpg_server {
         Query& qq = *qp[i][q];
         float mad = 0.0f;
         std::memcpy(&mad, &maxd[i][q], 4);
-        probe_query(qq, *G.h, G.args[q], mad);
+        seed_query(qq, *G.h, G.args[q], mad);
         if (mu) {
           std::lock_guard<std::mutex> lk(*mu);
           admit_one(qq);
@@ -2686,7 +2682,7 @@ struct cpg_server {
     if (in_flight > 0) {
       const double t0 = now_ms();
       MqArgs a = args();
-      launch_mq_round(a, false, grid, stream);
+      launch_mq_round(a, grid, stream);
       MqCtl mc{};
       d2h(&mc, mctl.p, 1, stream);
       d2h(hq.data(), qs.p, nslots, stream);

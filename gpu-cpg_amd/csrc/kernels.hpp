@@ -328,8 +328,8 @@ struct MqArgs {
 };
 
 void launch_mq_roots(const MqArgs& a, const int* root_v, const int* root_q, int nroots, hipStream_t s);
-// One round for every query (all: the batch takes every unexpanded path).
-void launch_mq_round(const MqArgs& a, bool all, int grid, hipStream_t s);
+// One round for every query.
+void launch_mq_round(const MqArgs& a, int grid, hipStream_t s);
 // sel: one byte per query slot choosing the queries whose paths are taken
 // (null = every query).
 void launch_mq_build_keys(const MqArgs& a, const uint8_t* sel, uint64_t nmax, uint64_t* key,

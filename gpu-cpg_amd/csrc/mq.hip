@@ -155,14 +155,14 @@ __global__ void __launch_bounds__(kMqBlock) mq_hist_kernel(MqArgs a) {
 // the bound); a query with none left is done.  The bins the batch takes are
 // cleared.  (The counts may hold a path at the bound itself, which is never
 // expanded: that costs a round with nothing to expand, not a missed one.)
-__global__ void __launch_bounds__(kMqSelBlock) mq_select_batch_kernel(MqArgs a, int all) {
+__global__ void __launch_bounds__(kMqSelBlock) mq_select_batch_kernel(MqArgs a) {
   const int q = blockIdx.x;
   if (q == 0 && threadIdx.x == 0) a.ctl->rebuild = 0;
   MqQuery* qs = a.qs + q;
   if (qs->done) return;
   unsigned* h = a.hist + static_cast<size_t>(q) * kMqHistStride + kMqBins;
   unsigned long long total = 0;
-  const bool take_all = all || qs->all || qs->trial;
+  const bool take_all = qs->all || qs->trial;
   const uint32_t last = mq_bin(qs->ukey, qs->klo, qs->shift);
   const uint32_t b = mq_crossing(h, last, take_all ? ~0ull : qs->batch_target, &total);
   for (uint32_t j = threadIdx.x; j <= b && j < static_cast<uint32_t>(kMqBins); j += blockDim.x) h[j] = 0u;
@@ -570,8 +570,8 @@ __global__ void __launch_bounds__(kMqBlock) mq_compact_kernel(MqArgs a, uint64_t
   }
 }
 
-// Appends a single-query node store's first cnt paths (a bound probe's
-// roots and children) at dst[base..) for query slot q, parents shifted.
+// Appends a single-query node store's first cnt paths (a
+// query's roots) at dst[base..) for query slot q, parents shifted.
 __global__ void mq_seed_kernel(NodeStore src, uint64_t cnt, NodeStore dst, int* dst_nq,
                                uint64_t base, int q) {
   for (uint64_t i = static_cast<uint64_t>(blockIdx.x) * blockDim.x + threadIdx.x; i < cnt;
@@ -626,12 +626,12 @@ void launch_mq_roots(const MqArgs& a, const int* root_v, const int* root_q, int 
   CPG_HIP(hipGetLastError());
 }
 
-void launch_mq_round(const MqArgs& a, bool all, int grid, hipStream_t s) {
+void launch_mq_round(const MqArgs& a, int grid, hipStream_t s) {
   hipLaunchKernelGGL(mq_open_kernel, dim3(a.nq_count), dim3(kMqSelBlock), 0, s, a);
   CPG_HIP(hipGetLastError());
   hipLaunchKernelGGL(mq_hist_kernel, dim3(grid), dim3(kMqBlock), 0, s, a);
   CPG_HIP(hipGetLastError());
-  hipLaunchKernelGGL(mq_select_batch_kernel, dim3(a.nq_count), dim3(kMqSelBlock), 0, s, a, all ? 1 : 0);
+  hipLaunchKernelGGL(mq_select_batch_kernel, dim3(a.nq_count), dim3(kMqSelBlock), 0, s, a);
   CPG_HIP(hipGetLastError());
   hipLaunchKernelGGL(mq_make_batch_kernel, dim3(grid), dim3(kMqBlock), 0, s, a);
   CPG_HIP(hipGetLastError());

@@ -56,10 +56,12 @@ typedef struct {
   int kernel_timing;        /* 1: time the SFXT and walk kernels with HIP events
                                on the engine's stream (cpg_timing.*_kernel_ms) */
   int sfxt_blocks;          /* SFXT level-loop grid in blocks (0 = automatic) */
-  int bound_probe;          /* first bound from pruned count passes: 0 = when the
-                               roots' chains are long (automatic), 1 = always,
+  int bound_probe;          /* first bound from pruned passes: 0 = when the roots'
+                               walks are long (automatic), 1 = always,
                                -1 = never (the first round walks unbounded)   */
-  int sfxt_method;          /* SFXT loop: 0 automatic (5), 1 level-synchronous
+  int sfxt_method;          /* SFXT loop: 0 automatic (5 on a graph's first SFXT,
+                               then its vertices in the level order that one
+                               left, without a barrier), 1 level-synchronous
                                loop with a global
                                queue and a fenced grid barrier, 2 barrier-free
                                dataflow loop, 3 level-synchronous loop with
@@ -271,12 +273,13 @@ typedef struct {
   int64_t node_cap;          /* current store capacity                       */
   int64_t peak_index_bytes;  /* in-flight deviation indexes, device bytes    */
   int64_t in_flight, queued;
-  int64_t sfxt_groups;       /* level loops run (each for a group of queries)  */
+  int64_t sfxt_groups;       /* suffix forests run (each for a group of queries) */
   int64_t nonmonotone;       /* children whose cost came out below their parent's */
   int64_t root_bounds;       /* queries whose first bound came from their roots */
   double sfxt_ms;            /* host time starting and checking groups' SFXTs  */
   double group_wait_ms;      /* host time waiting for a group, none in flight  */
-  double probe_ms, round_ms, extract_ms, compact_ms;  /* host wall time      */
+  double probe_ms;           /* 0 (first bounds are found in the rounds)       */
+  double round_ms, extract_ms, compact_ms;  /* host wall time                */
 } cpg_server_stats;
 /* budget_bytes: device bytes for in-flight indexes (0 = 64 GiB);
  * max_in_flight: query slots, at most 256 (0 = 64); initial_nodes: first

@@ -1752,9 +1752,12 @@ __device__ inline uint32_t delta_rank_key(int bits) {
 // fanout order and queued for sfxt_sort_mid_kernel (up to kWaveSort records,
 // from the front of big[]) or sfxt_sort_big_kernel (from the back).
 //
-// What bounds it: gathers of the fanouts' dist and distf, in flight for all
-// of a row's edges at once (a thread per vertex read them one by one: 256 us
-// at 1.5M vertices / 4.08M edges, 600 us at 1.1M / 5.7M).
+// What bounds it: gathers of the fanouts' dist, in flight for all of a row's
+// edges at once (a thread per vertex read them one by one: 256 us at 1.5M
+// vertices / 4.08M edges, 600 us at 1.1M / 5.7M).  Their distf is divided out
+// of dist again, as the settling kernels do it, instead of a second gather,
+// and a whole wave's keys are broadcast by scalar reads (400K vertices / 7.7M
+// edges 362 -> 292 us, 1.5M / 4.08M 132 -> 122).
 //
 // Each block takes one contiguous chunk of vertices and each XCD one range
 // of chunks (xcd_block): a vertex's fanouts sit on the levels just below it,
@@ -1801,7 +1804,7 @@ __global__ void __launch_bounds__(256) sfxt_devs_kernel(SfxtArgs a) {
 #pragma unroll
     for (int q = 0; q < 2; ++q) {
       dw[q] = w[q] >= 0 ? a.dist[w[q]] : kIntMax;
-      fw[q] = w[q] >= 0 ? a.distf[w[q]] : 0.0f;
+      fw[q] = static_cast<float>(dw[q]) / static_cast<float>(kScaleUp);
     }
     if (a.find_succ) {
       // update_successors_bu (gpucpg/gpucpg.cu:2606-2628): the largest id
@@ -1853,8 +1856,13 @@ __global__ void __launch_bounds__(256) sfxt_devs_kernel(SfxtArgs a) {
       for (int o = 32; o >= kG; o >>= 1) any |= any >> o;
       for (any &= kMask; any; any &= any - 1) {  // wave-uniform
         const int jj = static_cast<int>(__builtin_ctzll(any));
-        const uint32_t kj = __shfl(key[q], gbase + jj);
-        if (!((mine >> jj) & 1ull)) continue;
+        uint32_t kj;
+        if constexpr (kG == 64) {
+          kj = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(key[q]), jj));
+        } else {
+          kj = __shfl(key[q], gbase + jj);
+          if (!((mine >> jj) & 1ull)) continue;
+        }
         rank[q] += (kj < key[q] || (kj == key[q] && jj < sub)) ? 1 : 0;
         rank[q ^ 1] += (kj < key[q ^ 1] || (kj == key[q ^ 1] && q == 0)) ? 1 : 0;
       }
@@ -1872,8 +1880,9 @@ __global__ void __launch_bounds__(256) sfxt_devs_kernel(SfxtArgs a) {
         int4 rec = make_int4(0, 0, 0, 0);
         if (wide && j < e) {
           const int x = a.oadj[j];
-          if (x != s && a.dist[x] != kIntMax) {
-            const float f = a.distf[x], xe = a.owgt[j];
+          const int dx = a.dist[x];
+          if (x != s && dx != kIntMax) {
+            const float f = static_cast<float>(dx) / static_cast<float>(kScaleUp), xe = a.owgt[j];
             const float d = delta_of(f, xe);
             rec = make_int4(x, __float_as_int(xe), __float_as_int(f), __float_as_int(d));
             mind = fminf(mind, d);

@@ -48,6 +48,11 @@ double now_ms() {
       .count();
 }
 
+// The device has no memory left for a buffer.
+struct DeviceFull : std::runtime_error {
+  using std::runtime_error::runtime_error;
+};
+
 template <class T>
 struct DevBuf {
   T* p = nullptr;
@@ -55,8 +60,27 @@ struct DevBuf {
   void reserve(size_t want) {
     if (want <= n && p) return;
     release();
-    CPG_HIP(hipMalloc(&p, sizeof(T) * (want ? want : 1)));
+    if (!take(want)) throw DeviceFull("HIP error: out of device memory for " + std::to_string(sizeof(T) * want) + " bytes");
+  }
+  // As reserve(), but false where the device has no memory for it: what the
+  // buffer held stays.
+  bool try_reserve(size_t want) {
+    if (want <= n && p) return true;
+    DevBuf bigger;
+    if (!bigger.take(want)) return false;
+    swap(bigger);
+    return true;
+  }
+  bool take(size_t want) {  // of an empty buffer
+    const hipError_t e = hipMalloc(&p, sizeof(T) * (want ? want : 1));
+    if (e == hipErrorOutOfMemory) {
+      p = nullptr;
+      (void)hipGetLastError();  // answered here: no launch check reports it
+      return false;
+    }
+    CPG_HIP(e);
     n = want;
+    return true;
   }
   void release() {
     if (p) (void)hipFree(p);
@@ -582,13 +606,18 @@ struct cpg_handle {
     }
     pad[static_cast<size_t>(L)] = static_cast<int>(np);
     const size_t ints = n + (static_cast<size_t>(np) + 1) + pad.size() + sfxt_sched_tiles(static_cast<int>(np));
-    sc_mem.reserve(std::max<size_t>(m, 1) + (ints + 1) / 2);
+    // no room for it beside what the card holds: the level loop again
+    if (!sc_mem.try_reserve(std::max<size_t>(m, 1) + (ints + 1) / 2) ||
+        !best.try_reserve(static_cast<size_t>(std::max<int64_t>(np, g.n)) + kSfxtPad)) {
+      sc_mem.release();
+      order_ready = false;
+      return;
+    }
     int2* edge_d = sc_mem.p;
     int* pos_d = reinterpret_cast<int*>(edge_d + std::max<size_t>(m, 1));
     unsigned* ofs_d = reinterpret_cast<unsigned*>(pos_d + n);
     int* pad_d = reinterpret_cast<int*>(ofs_d + np + 1);
     unsigned* tiles_d = reinterpret_cast<unsigned*>(pad_d + pad.size());
-    best.reserve(static_cast<size_t>(std::max<int64_t>(np, g.n)) + kSfxtPad);
     a.best = best.p;
     h2d(pad_d, pad.data(), pad.size(), stream);
     launch_sfxt_sched_build(a, relabelled ? nullptr : queue.p, pad_d, nl, static_cast<int>(np), pos_d, ofs_d, edge_d,
@@ -2865,7 +2894,15 @@ int cpg_query(cpg_handle* h, int64_t k, const cpg_query_opts* o) {
         throw std::runtime_error("cpg_query_opts.struct_size mismatch");
       d = *o;
     }
-    h->query(k, d);
+    try {
+      h->query(k, d);
+    } catch (const DeviceFull&) {
+      // a schedule laid out meanwhile may hold what this query needs
+      if (!h->sched_ready) throw;
+      h->drop_schedule();
+      h->order_ready = false;  // this query's SFXT takes the level loop
+      h->query(k, d);
+    }
     return 0;
   });
 }

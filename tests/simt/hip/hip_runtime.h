@@ -211,6 +211,7 @@ inline T atomicMin(T* p, T v) {
 // ---------------------------------------------------------------- host API
 typedef int hipError_t;
 constexpr hipError_t hipSuccess = 0;
+constexpr hipError_t hipErrorOutOfMemory = 2;
 constexpr hipError_t hipErrorNotReady = 600;
 constexpr unsigned hipEventDisableTiming = 2;
 typedef struct simt_stream* hipStream_t;

@@ -385,7 +385,13 @@ struct GuardInit {
     sigaction(SIGSEGV, &sa, nullptr);
   }
 } g_guard_init;
+// Device allocations from now until one fails (negative: none does).
+static std::atomic<int> g_fail_in{-1};
+extern "C" void simt_fail_malloc(int in) { g_fail_in = in; }
+
 hipError_t simt_malloc(void** p, size_t bytes) {
+  *p = nullptr;
+  if (g_fail_in >= 0 && g_fail_in-- == 0) return hipErrorOutOfMemory;
   if (!bytes) bytes = 1;
   if (!guard_on()) {
     *p = std::calloc(1, bytes);

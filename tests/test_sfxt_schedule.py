@@ -112,6 +112,33 @@ def test_emulated_schedule_follows_the_loaded_graph(emu):  # noqa: F811
         g.close()
 
 
+@pytest.mark.parametrize("nth", range(8))
+def test_emulated_full_device_leaves_the_schedule_out(emu, nth):  # noqa: F811
+    """One device allocation fails on the run that lays the schedule out, its
+    own or a later one of the query (which grows its node store): the query
+    is answered as without a schedule."""
+    n, u, v, w = SHAPES["mean3"]()
+    og = pyoracle.OracleGraph.from_edges(n, u, v, w)
+    dist, succ, level, _ = og.sfxt()
+    g = emu.CpGen()
+    try:
+        g.load_edges(n, u, v, w)
+        g.report_paths(1)
+        for k in (2000, 2000):
+            g.reset()
+            emu._lib.simt_fail_malloc(nth)
+            try:
+                g.report_paths(k)
+            finally:
+                emu._lib.simt_fail_malloc(-1)
+            for got, want in zip(g.sfxt(), (dist, succ, level)):
+                np.testing.assert_array_equal(got, want)
+            want, _ = og.topk(dist, succ, k)
+            assert bits_equal(want, g.get_slacks(k))
+    finally:
+        g.close()
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("reorder", [False, True])
 @pytest.mark.parametrize("shape", sorted(SHAPES))

@@ -2001,13 +2001,24 @@ struct cpg_server {
     ready = true;
   }
 
+  // Whether no path's int-scaled sum can reach either end of the 32-bit range
+  // (a path has fewer edges than the graph has levels): the scheduled
+  // multi-subset loop keeps the lowest value as its empty word, so a graph
+  // that might settle a vertex there takes the level loop.
+  static bool sums_in_range(const cpg_handle& h) {
+    const double most = 2147483646.0 / (static_cast<double>(kScaleUp) * 1.000001 * std::max(1, h.diameter));
+    for (float w : h.g.owgt)
+      if (!(std::fabs(static_cast<double>(w)) <= most)) return false;
+    return true;
+  }
+
   int add_graph(const EdgeList& el) {
     auto G = std::make_unique<Graph>();
     G->h = std::make_unique<cpg_handle>();
     G->h->set_graph(el);
     G->h->upload_graph();
     G->h->run_sfxt(false);  // the level count (the same for every endpoint subset)
-    G->h->prepare_schedule();
+    if (sums_in_range(*G->h)) G->h->prepare_schedule();
     const int64_t n = G->h->g.n, m = G->h->g.m;
     G->index_bytes = 24 * n + 16 * m;  // vrec 16, devinfo 8 per vertex; devs 16 per edge
     graphs.push_back(std::move(G));
@@ -2426,7 +2437,6 @@ struct cpg_server {
       }
     }
     if (h.g.n > 0) {
-      if (c.err == 2) throw std::runtime_error("a suffix distance is out of the served loop's range");
       if (c.err) throw std::runtime_error("SFXT grid barrier did not complete");
       if (!G.scheduled && c.num_levels != h.diameter) throw std::runtime_error("SFXT levels differ from the graph's");
       for (int q = 0; q < Q; ++q) {

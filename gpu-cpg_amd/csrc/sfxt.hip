@@ -1304,9 +1304,10 @@ __global__ void __launch_bounds__(256) sfxt_sched_finish_kernel(SfxtArgs a, Sfxt
 // Scheduled loop for Q endpoint subsets at once (served queries): lanes_ lanes
 // per vertex, lane l of them taking record l / Q of a step in subset l % Q, so
 // that a record's Q distances are one contiguous load.  A distance is its own
-// write-once state word (kMultiEmpty until settled); a vertex whose distance
-// comes out as exactly that value raises an error instead.  Otherwise as
-// sfxt_sched_kernel; levels are not computed (no served result holds them).
+// write-once state word, kMultiEmpty until settled: the loop is for graphs
+// none of whose path sums can reach that value (the host checks; others take
+// the level loop).  Otherwise as sfxt_sched_kernel; levels are not computed
+// (no served result holds them).
 // The level loop it replaces took 24-46 us a level (counters, queue, a grid
 // barrier, one wave per vertex).
 constexpr int kMultiEmpty = static_cast<int>(0x80000000u);
@@ -1377,13 +1378,7 @@ __device__ void sched_multi_part(const SfxtSchedPart& P, unsigned bid, unsigned 
       settle(r0);
     }
     for (int o = Q; o < LV; o <<= 1) bd = min(bd, __shfl_xor(bd, o));
-    if (in < Q && b0 < e0) {
-      if (bd == kMultiEmpty) {
-        atomicExch(&P.ctl->err, 2);
-        bd = kIntMax;
-      }
-      st_dev32(at(c * V + grp), bd);
-    }
+    if (in < Q && b0 < e0) st_dev32(at(c * V + grp), bd);
 #pragma unroll
     for (int q = 0; q < kU; ++q) r0[q] = r1[q];
     b0 = b1;

@@ -12,13 +12,25 @@ from test_sfxt_schedule import SHAPES
 from test_simt_emulator import bits_equal, emu  # noqa: F401  (fixture)
 
 
+def with_lowest():
+    """One source whose only path sums to the lowest 32-bit distance."""
+    n, u, v, w = SHAPES["mean3"]()
+    sink = np.setdiff1d(v, u)[0]
+    return (n + 1, np.append(u, n).astype(np.int32), np.append(v, sink).astype(np.int32),
+            np.append(w, np.float32(-214748.3648)))
+
+
+def shape(name):
+    return with_lowest() if name == "lowest" else SHAPES[name]()
+
+
 def check(lib, shapes, queries, ks):
     rng = np.random.default_rng(queries)
     s = lib.Server(max_in_flight=64)
     try:
         jobs = []
         for name in shapes:
-            n, u, v, w = SHAPES[name]()
+            n, u, v, w = shape(name)
             gid = s.add_graph(n, u, v, w)
             og = pyoracle.OracleGraph.from_edges(n, u, v, w)
             sinks = np.nonzero(np.bincount(u, minlength=n)[:n] == 0)[0]
@@ -40,6 +52,17 @@ def check(lib, shapes, queries, ks):
 
 def test_emulated_served_groups(emu):  # noqa: F811
     check(emu, ["mean3", "cycle"], 3, [5])
+
+
+def test_emulated_lowest_distance_is_served(emu):  # noqa: F811
+    dist = pyoracle.OracleGraph.from_edges(*with_lowest()).sfxt()[0]
+    assert dist[-1] == -2**31
+    check(emu, ["lowest", "chain"], 3, [5, 40])
+
+
+@pytest.mark.gpu
+def test_gpu_lowest_distance_is_served():
+    check(cpgamd, ["lowest", "chain"], 3, [5, 40])
 
 
 @pytest.mark.gpu

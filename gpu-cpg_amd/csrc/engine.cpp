@@ -415,6 +415,7 @@ struct cpg_handle {
   void upload_graph() {
     if (graph_on_device) return;
     ensure_stream();
+    drop_schedule();  // the graph it was laid out for is no longer resident
     const size_t n = static_cast<size_t>(g.n), m = static_cast<size_t>(g.m);
     oadjp.reserve(n + 1); oadj.reserve(m); owgt.reserve(m);
     iadjp.reserve(n + 1); iedge.reserve(m); srcs.reserve(g.srcs.size());
@@ -439,7 +440,7 @@ struct cpg_handle {
     graph_on_device = true;
     sfxt_valid = false;
     relabelled = false;
-    order_ready = sched_ready = false;
+    order_ready = false;
     if (csr_reorder == 1) relabel_graph();
   }
 
@@ -500,7 +501,7 @@ struct cpg_handle {
     oadjp.swap(nadjp); oadj.swap(nadj); owgt.swap(nw); iadjp.swap(niadjp_d); iedge.swap(nie);
     relabelled = true;
     sfxt_valid = false;
-    order_ready = sched_ready = false;
+    order_ready = false;  // of the ids before (their one SFXT laid out no schedule)
     h_succ.clear();
     hb.valid = false;
     reorder_ms = now_ms() - t0;
@@ -655,8 +656,8 @@ struct cpg_handle {
   // Gives the schedule's memory back (a query under a device-byte budget
   // holds what it held without one; the level order stays).
   void drop_schedule() {
-    if (!sched_ready) return;
     sched_ready = false;
+    if (!sc_mem.p) return;
     sc_mem.release();
     if (best.n > static_cast<size_t>(g.n) + kSfxtPad) best.release();
   }

@@ -139,6 +139,48 @@ def test_emulated_full_device_leaves_the_schedule_out(emu, nth):  # noqa: F811
         g.close()
 
 
+def budget_after(lib, n, u, v, w, change):
+    """The graph of a handle that holds a schedule is loaded again, or
+    relabelled: a budget of what a new handle holds for it is still enough,
+    with as many node slots."""
+    def load(g):
+        g.load_edges(n, u, v, w)
+
+    def ask(g, budget):
+        g.reset()
+        g.report_paths(20, mem_budget_bytes=budget, max_nodes=20000)
+        return g.get_slacks(20).copy(), g.timings()
+
+    steps = {"load": load, "reorder": lambda g: g.set_csr_reorder(1)}
+    with lib.CpGen() as g:
+        load(g)
+        ask(g, 0)
+        steps[change](g)
+        ask(g, 0)
+        want, ref = ask(g, 1 << 40)  # a budget: no schedule is held
+    held = ref["device_bytes"]
+    with lib.CpGen() as g:
+        load(g)
+        for _ in range(2):
+            ask(g, 0)
+        steps[change](g)
+        ask(g, 0)
+        got, t = ask(g, held)
+    assert bits_equal(want, got)
+    assert t["device_bytes"] <= held and t["node_slots"] == ref["node_slots"]
+
+
+@pytest.mark.parametrize("change", ["load", "reorder"])
+def test_emulated_schedule_ends_with_its_graph(emu, change):  # noqa: F811
+    budget_after(emu, *SHAPES["mean6"](), change)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("change", ["load", "reorder"])
+def test_gpu_schedule_ends_with_its_graph(change):
+    budget_after(cpgamd, *layered([300] * 150, 4, 8), change)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("reorder", [False, True])
 @pytest.mark.parametrize("shape", sorted(SHAPES))

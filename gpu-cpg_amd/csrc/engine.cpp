@@ -278,6 +278,7 @@ struct cpg_handle {
   bool order_ready = false;    // queue, level and lvlp hold a finished level loop of the resident graph
   bool order_pending = false;  // the queued SFXT will leave them so
   bool budgeted = false;       // the query has a device-byte budget: no schedule
+  bool schedule_off = false;   // the device had no room beside one: the level loop until the graph changes
   bool sfxt_valid = false;
   std::vector<uint8_t> sfxt_sinks;  // endpoint subset of the current SFXT, per sink (empty = all)
   DevBuf<uint8_t> emask;
@@ -416,6 +417,7 @@ struct cpg_handle {
     if (graph_on_device) return;
     ensure_stream();
     drop_schedule();  // the graph it was laid out for is no longer resident
+    schedule_off = false;
     const size_t n = static_cast<size_t>(g.n), m = static_cast<size_t>(g.m);
     oadjp.reserve(n + 1); oadj.reserve(m); owgt.reserve(m);
     iadjp.reserve(n + 1); iedge.reserve(m); srcs.reserve(g.srcs.size());
@@ -601,17 +603,17 @@ struct cpg_handle {
       pad[static_cast<size_t>(d)] = static_cast<int>(np);
       np += (static_cast<int64_t>(first[static_cast<size_t>(d) + 1] - first[static_cast<size_t>(d)]) + per - 1) / per * per;
       if (np > 0x7fffff00ll) {  // positions are 32-bit: such a graph keeps the level loop
-        order_ready = false;
+        schedule_off = true;
         return;
       }
     }
     pad[static_cast<size_t>(L)] = static_cast<int>(np);
     const size_t ints = n + (static_cast<size_t>(np) + 1) + pad.size() + sfxt_sched_tiles(static_cast<int>(np));
-    // no room for it beside what the card holds: the level loop again
+    // no room for it beside what the card holds: the level loop from now on
     if (!sc_mem.try_reserve(std::max<size_t>(m, 1) + (ints + 1) / 2) ||
         !best.try_reserve(static_cast<size_t>(std::max<int64_t>(np, g.n)) + kSfxtPad)) {
       sc_mem.release();
-      order_ready = false;
+      schedule_off = true;
       return;
     }
     int2* edge_d = sc_mem.p;
@@ -645,7 +647,7 @@ struct cpg_handle {
   // The schedule of a graph whose level order is at hand, ahead of the next
   // SFXT (graphs made resident to be queried many times).
   void prepare_schedule() {
-    if (sched_ready || !order_ready || last_diameter <= 0 || g.n == 0) return;
+    if (sched_ready || schedule_off || !order_ready || last_diameter <= 0 || g.n == 0) return;
     SfxtArgs a{};
     a.n = g.n;
     a.oadjp = oadjp.p; a.oadj = oadj.p; a.owgt = owgt.p;
@@ -715,7 +717,8 @@ struct cpg_handle {
       // has left its level order, before that the edge-parallel fence-free
       // level loop
       const int method = sfxt_method == 0 ? 5 : sfxt_method;
-      if (sfxt_method == 0 && !budgeted && !sched_ready && order_ready && last_diameter > 0) build_schedule(a);
+      if (sfxt_method == 0 && !budgeted && !sched_ready && !schedule_off && order_ready && last_diameter > 0)
+        build_schedule(a);
       const bool scheduled = sfxt_method == 0 && sched_ready;
       if (!scheduled) order_ready = false;
       order_pending = !scheduled && (method == 1 || method >= 4);
@@ -2911,7 +2914,7 @@ int cpg_query(cpg_handle* h, int64_t k, const cpg_query_opts* o) {
       // a schedule laid out meanwhile may hold what this query needs
       if (!h->sched_ready) throw;
       h->drop_schedule();
-      h->order_ready = false;  // this query's SFXT takes the level loop
+      h->schedule_off = true;  // this query's SFXT takes the level loop, and later ones
       h->query(k, d);
     }
     return 0;

@@ -139,6 +139,29 @@ def test_emulated_full_device_leaves_the_schedule_out(emu, nth):  # noqa: F811
         g.close()
 
 
+def test_emulated_layout_is_not_tried_again(emu):  # noqa: F811
+    """A device with no room for the schedule: the level loop stays until the
+    graph is loaded again, without another attempt at each query."""
+    def held(g):
+        g.reset()
+        g.report_paths(5, max_nodes=4000)
+        return g.timings()["device_bytes"]
+
+    n, u, v, w = SHAPES["mean3"]()
+    with emu.CpGen() as g:
+        g.load_edges(n, u, v, w)
+        without = held(g)
+        emu._lib.simt_fail_malloc(0)
+        try:
+            assert held(g) == without
+        finally:
+            emu._lib.simt_fail_malloc(-1)
+        assert held(g) == without
+        g.load_edges(n, u, v, w)
+        assert held(g) == without
+        assert held(g) > without
+
+
 def budget_after(lib, n, u, v, w, change):
     """The graph of a handle that holds a schedule is loaded again, or
     relabelled: a budget of what a new handle holds for it is still enough,

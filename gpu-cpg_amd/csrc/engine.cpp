@@ -664,6 +664,16 @@ struct cpg_handle {
     if (best.n > static_cast<size_t>(g.n) + kSfxtPad) best.release();
   }
 
+  // On a full device: gives up the schedule for as long as the graph stays
+  // (false: none is held).
+  bool give_back_schedule() {
+    if (!sc_mem.p) return false;
+    CPG_HIP(hipStreamSynchronize(stream));  // a loop may be reading it
+    drop_schedule();
+    schedule_off = true;
+    return true;
+  }
+
   // The SFXT in two halves, so that a caller can put its own work on the
   // stream before the one synchronisation: sfxt_enqueue puts the kernels on
   // the stream (false: the cached SFXT stands, nothing was queued), and
@@ -2794,6 +2804,18 @@ R guarded(R fail_value, F&& f) {
   }
 }
 
+// Runs f (a call that may be started over) and, where the device is full and
+// the handle's schedule may hold what it needs, once more without the schedule.
+template <class F>
+auto with_room(cpg_handle& h, F&& f) -> decltype(f()) {
+  try {
+    return f();
+  } catch (const DeviceFull&) {
+    if (!h.give_back_schedule()) throw;
+  }
+  return f();
+}
+
 #define CPG_CHECK_HANDLE(h, fail_value)                 \
   if (!(h)) {                                           \
     g_last_error = "null handle";                       \
@@ -2908,15 +2930,7 @@ int cpg_query(cpg_handle* h, int64_t k, const cpg_query_opts* o) {
         throw std::runtime_error("cpg_query_opts.struct_size mismatch");
       d = *o;
     }
-    try {
-      h->query(k, d);
-    } catch (const DeviceFull&) {
-      // a schedule laid out meanwhile may hold what this query needs
-      if (!h->sched_ready) throw;
-      h->drop_schedule();
-      h->schedule_off = true;  // this query's SFXT takes the level loop, and later ones
-      h->query(k, d);
-    }
+    with_room(*h, [&]() { h->query(k, d); });
     return 0;
   });
 }
@@ -2960,7 +2974,7 @@ int64_t cpg_get_nodes(cpg_handle* h, int64_t k, cpg_node* out) {
 int64_t cpg_get_path_vertices(cpg_handle* h, int64_t i, int* out, int64_t cap) {
   CPG_CHECK_HANDLE(h, -1)
   return guarded<int64_t>(-1, [&]() {
-    const std::vector<int> path = h->path_vertices(i);
+    const std::vector<int> path = with_room(*h, [&]() { return h->path_vertices(i); });
     const int64_t len = static_cast<int64_t>(path.size());
     if (len > cap) return -len - 1000;
     if (out) std::memcpy(out, path.data(), sizeof(int) * len);
@@ -3016,7 +3030,7 @@ int cpg_sfxt(cpg_handle* h) {
   CPG_CHECK_HANDLE(h, -1)
   return guarded<int>(-1, [&]() {
     if (!h->loaded) throw std::runtime_error("no graph loaded");
-    h->timing.sfxt_ms = h->run_sfxt(false);
+    h->timing.sfxt_ms = with_room(*h, [&]() { return h->run_sfxt(false); });
     return 0;
   });
 }
@@ -3025,7 +3039,7 @@ int cpg_get_sfxt(cpg_handle* h, int* dist_out, int* succ_out, int* level_out) {
   CPG_CHECK_HANDLE(h, -1)
   return guarded<int>(-1, [&]() {
     if (!h->loaded) throw std::runtime_error("no graph loaded");
-    if (!h->sfxt_valid) h->run_sfxt(false);
+    if (!h->sfxt_valid) with_room(*h, [&]() { return h->run_sfxt(false); });
     const size_t n = static_cast<size_t>(h->g.n);
     if (!h->relabelled) {
       if (dist_out) d2h(dist_out, h->dist.p, n, h->stream);
@@ -3055,7 +3069,7 @@ int cpg_bvss_build(cpg_handle* h) {
   CPG_CHECK_HANDLE(h, -1)
   return guarded<int>(-1, [&]() {
     if (!h->loaded) throw std::runtime_error("no graph loaded");
-    h->bvss_build();
+    with_room(*h, [&]() { h->bvss_build(); });
     return 0;
   });
 }
@@ -3099,7 +3113,8 @@ int64_t cpg_bvss_discover(cpg_handle* h, int nfront, const int* fptr, const int*
   CPG_CHECK_HANDLE(h, -1)
   return guarded<int64_t>(-1, [&]() -> int64_t {
     if (!h->loaded) throw std::runtime_error("no graph loaded");
-    return h->bvss_discover(nfront, fptr, fsrc, mode, dense_min, out_f, out_u, out_v, cap);
+    return with_room(
+        *h, [&]() { return h->bvss_discover(nfront, fptr, fsrc, mode, dense_min, out_f, out_u, out_v, cap); });
   });
 }
 

@@ -139,6 +139,29 @@ def test_emulated_full_device_leaves_the_schedule_out(emu, nth):  # noqa: F811
         g.close()
 
 
+@pytest.mark.parametrize("nth", range(10))
+def test_emulated_full_device_in_discovery(emu, nth):  # noqa: F811
+    """An allocation of a deviation discovery fails on a handle that holds a
+    schedule: the schedule is given back and the call answered."""
+    n, u, v, w = SHAPES["mean3"]()
+    front = [np.arange(i, n, 7, dtype=np.int32) for i in range(3)]
+    with emu.CpGen() as g:
+        g.load_edges(n, u, v, w)
+        want = g.bvss_discover(front)
+    with emu.CpGen() as g:
+        g.load_edges(n, u, v, w)
+        for _ in range(2):
+            g.reset()
+            g.run_sfxt()
+        emu._lib.simt_fail_malloc(nth)
+        try:
+            got = g.bvss_discover(front)
+        finally:
+            emu._lib.simt_fail_malloc(-1)
+    for a, b in zip(want, got):
+        np.testing.assert_array_equal(a, b)
+
+
 def test_emulated_layout_is_not_tried_again(emu):  # noqa: F811
     """A device with no room for the schedule: the level loop stays until the
     graph is loaded again, without another attempt at each query."""

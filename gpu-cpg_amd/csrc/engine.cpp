@@ -1499,6 +1499,18 @@ struct cpg_handle {
   }
 };
 
+// Runs f (a call that may be started over) and, where the device is full and
+// the handle's schedule may hold what it needs, once more without the schedule.
+template <class F>
+auto with_room(cpg_handle& h, F&& f) -> decltype(f()) {
+  try {
+    return f();
+  } catch (const DeviceFull&) {
+    if (!h.give_back_schedule()) throw;
+  }
+  return f();
+}
+
 // Batched queries: the disjoint union of several designs, one top-K query
 // each, expanded together by the multi-query PFXT (mq.hip).  The union's
 // SFXT is every design's own SFXT, so one level loop serves all of them;
@@ -1638,6 +1650,10 @@ struct cpg_batch {
   }
 
   void run(const cpg_query_opts& o) {
+    with_room(uh, [&]() { run_once(o); });
+  }
+
+  void run_once(const cpg_query_opts& o) {
     if (designs.empty()) throw std::runtime_error("no designs in the batch");
     if (!built) build_union();
     timing = cpg_timing{};
@@ -2802,18 +2818,6 @@ R guarded(R fail_value, F&& f) {
     g_last_error = "unknown error";
     return fail_value;
   }
-}
-
-// Runs f (a call that may be started over) and, where the device is full and
-// the handle's schedule may hold what it needs, once more without the schedule.
-template <class F>
-auto with_room(cpg_handle& h, F&& f) -> decltype(f()) {
-  try {
-    return f();
-  } catch (const DeviceFull&) {
-    if (!h.give_back_schedule()) throw;
-  }
-  return f();
 }
 
 #define CPG_CHECK_HANDLE(h, fail_value)                 \

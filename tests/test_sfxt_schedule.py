@@ -162,6 +162,31 @@ def test_emulated_full_device_in_discovery(emu, nth):  # noqa: F811
         np.testing.assert_array_equal(a, b)
 
 
+@pytest.mark.parametrize("nth", range(6))
+def test_emulated_full_device_in_a_batch(emu, nth):  # noqa: F811
+    """An allocation fails on the batch's run that holds a schedule of the
+    union graph (larger rounds store more paths than the first run's, so its
+    buffers grow)."""
+    graphs = [SHAPES["mean12"](), SHAPES["mean3"]()]
+    k = 3000
+    with emu.Batch() as b:
+        for g in graphs:
+            b.add(*g, k)
+        b.set_tuning(target_div=(32, 32, 32))
+        b.run()
+        want = [b.get_slacks(q, k).copy() for q in range(2)]
+        stored = b.timings()["generated"]
+        b.set_tuning(target_div=(1, 1, 1))
+        emu._lib.simt_fail_malloc(nth)
+        try:
+            b.run()
+        finally:
+            emu._lib.simt_fail_malloc(-1)
+        assert b.timings()["generated"] > stored
+        for q in range(2):
+            assert bits_equal(want[q], b.get_slacks(q, k))
+
+
 def test_emulated_layout_is_not_tried_again(emu):  # noqa: F811
     """A device with no room for the schedule: the level loop stays until the
     graph is loaded again, without another attempt at each query."""

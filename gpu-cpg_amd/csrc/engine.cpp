@@ -1988,6 +1988,7 @@ struct cpg_server {
   hipStream_t sstream = nullptr;  // level-loop launches of admission groups
   hipEvent_t ev_levels = nullptr;
   std::mutex stats_mu;  // statistics the seedings of several graphs update
+  std::mutex room_mu;   // likewise the giving back of schedules
   int parts_cap = 1;              // blocks one partitioned level-loop launch keeps resident
 
   uint64_t first_cap = uint64_t(1) << 24;
@@ -2003,30 +2004,50 @@ struct cpg_server {
     if (stream) (void)hipStreamDestroy(stream);
   }
 
+  // Runs f (reservations, or a step that may be started over) and, where the
+  // device is full, once more without the graphs' schedules, which their
+  // groups' loops have read once the loops' stream is idle.  The groups that
+  // follow take the level loop.
+  template <class F>
+  void room(F&& f) {
+    try {
+      f();
+      return;
+    } catch (const DeviceFull&) {
+      std::lock_guard<std::mutex> lk(room_mu);
+      if (sstream) CPG_HIP(hipStreamSynchronize(sstream));
+      for (auto& G : graphs) G->h->give_back_schedule();
+    }
+    f();
+  }
+
   void init() {
     if (ready) return;
-    CPG_HIP(hipStreamCreateWithFlags(&stream, hipStreamNonBlocking));
-    CPG_HIP(hipStreamCreateWithFlags(&sstream, hipStreamNonBlocking));
+    if (!stream) CPG_HIP(hipStreamCreateWithFlags(&stream, hipStreamNonBlocking));
+    if (!sstream) CPG_HIP(hipStreamCreateWithFlags(&sstream, hipStreamNonBlocking));
     parts_cap = sfxt_parts_capacity();
     int dev = 0, cus = 0;
     CPG_HIP(hipGetDevice(&dev));
     CPG_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
     grid = std::max(1, cus) * 8;
+    room([&]() {
+      qs.reserve(nslots);
+      hist.reserve(static_cast<size_t>(nslots) * kMqHistStride);
+      mctl.reserve(1);
+      sel.reserve(nslots);
+      per_q.reserve(nslots);
+      st[0].reserve(first_cap);
+      batch.reserve(st[0].cap);
+    });
     slot_query.assign(nslots, -1);
     slot_reserved.assign(nslots, 0);
+    free_slots.clear();
     for (int i = nslots - 1; i >= 0; --i) free_slots.push_back(i);
     hq.assign(nslots, MqQuery{});
     for (auto& m : hq) m.done = 1;
-    qs.reserve(nslots);
     h2d(qs.p, hq.data(), nslots, stream);
-    hist.reserve(static_cast<size_t>(nslots) * kMqHistStride);
-    mctl.reserve(1);
     const MqCtl z{};
     h2d(mctl.p, &z, 1, stream);
-    sel.reserve(nslots);
-    per_q.reserve(nslots);
-    st[0].reserve(first_cap);
-    batch.reserve(st[0].cap);
     CPG_HIP(hipStreamSynchronize(stream));
     ready = true;
   }
@@ -2044,10 +2065,12 @@ struct cpg_server {
 
   int add_graph(const EdgeList& el) {
     auto G = std::make_unique<Graph>();
-    G->h = std::make_unique<cpg_handle>();
-    G->h->set_graph(el);
-    G->h->upload_graph();
-    G->h->run_sfxt(false);  // the level count (the same for every endpoint subset)
+    room([&]() {
+      G->h = std::make_unique<cpg_handle>();
+      G->h->set_graph(el);
+      G->h->upload_graph();
+      G->h->run_sfxt(false);  // the level count (the same for every endpoint subset)
+    });
     if (sums_in_range(*G->h)) G->h->prepare_schedule();
     const int64_t n = G->h->g.n, m = G->h->g.m;
     G->index_bytes = 24 * n + 16 * m;  // vrec 16, devinfo 8 per vertex; devs 16 per edge
@@ -2091,7 +2114,7 @@ struct cpg_server {
   void seed_query(Query& q, cpg_handle& h, const SfxtArgs& aq, float max_abs_distf) {
     const int nsrc = static_cast<int>(h.g.srcs.size());
     std::vector<int> sd(nsrc);
-    h.src_dist.reserve(std::max(1, nsrc));
+    room([&]() { h.src_dist.reserve(std::max(1, nsrc)); });
     launch_gather_int(aq.dist, h.srcs.p, nsrc, h.src_dist.p, h.stream);
     d2h(sd.data(), h.src_dist.p, nsrc, h.stream);
     CPG_HIP(hipStreamSynchronize(h.stream));
@@ -2121,12 +2144,14 @@ struct cpg_server {
     // the roots in the graph handle's node store, for admission to copy
     auto seed_roots = [&]() {
       const uint64_t cap = std::max<uint64_t>(uint64_t(1) << 16, static_cast<uint64_t>(nkept));
-      h.ensure_pfxt_buffers(std::max<uint64_t>(cap, h.node_cap));
+      room([&]() {
+        h.ensure_pfxt_buffers(std::max<uint64_t>(cap, h.node_cap));
+        h.keep.reserve(std::max(1, nsrc));
+      });
       PfxtCtl init{};
       init.ukey = kKeyInf;
       init.node_cap = h.node_cap;
       h2d(h.pctl.p, &init, 1, h.stream);
-      h.keep.reserve(std::max(1, nsrc));
       h2d(h.keep.p, kp.data(), nsrc, h.stream);
       launch_roots(h.srcs.p, h.keep.p, nsrc, aq.dist, aq.distf, h.node_store(), h.pctl.p, h.stream);
       q.seed_n = h.read_pctl().node_n;
@@ -2209,14 +2234,32 @@ struct cpg_server {
     SfxtMulti smm[kMaxParts]{};
     int sn[kMaxParts]{};
     std::vector<int> part_of(list.size(), -1);
+    auto padded = [](size_t queries) {  // subsets of a group, a power of two
+      size_t q = 1;
+      while (q < queries) q <<= 1;
+      return q;
+    };
+    room([&]() {  // every group's buffers first: giving schedules back changes what the groups need
+      for (const auto& part : list) {
+        cpg_handle& h = *graphs[part.first]->h;
+        Graph::Multi& M = graphs[part.first]->mm;
+        const size_t n = static_cast<size_t>(h.g.n), Q = padded(part.second.size());
+        h.deps.reserve(n + kSfxtPad); h.queue.reserve(n); h.lvlp.reserve(n + 2); h.level.reserve(n);
+        h.big.reserve(n); h.sctl.reserve(1);
+        if (h.g.max_out_degree > kSfxtLdsSort) h.devs_tmp.reserve(static_cast<size_t>(h.g.m));
+        h.lift.reserve(static_cast<size_t>(sfxt_lift_levels(h.diameter)) * std::max<size_t>(n, 1));
+        M.dv.reserve((h.sched_ready ? static_cast<size_t>(h.sched.np) : n) * Q);
+        M.dist.reserve(n * Q); M.succ.reserve(n * Q); M.distf.reserve(n * Q);
+        M.masks.reserve(std::max<size_t>(1, h.g.sinks.size() * Q)); M.maxd.reserve(Q); M.ctls.reserve(Q);
+      }
+    });
     for (size_t li = 0; li < list.size(); ++li) {
       const int gi = list[li].first;
       const std::vector<int64_t>& ids = list[li].second;
       Graph& G = *graphs[gi];
       cpg_handle& h = *G.h;
       const size_t n = static_cast<size_t>(h.g.n), m = static_cast<size_t>(h.g.m);
-      int Q = 1;
-      while (Q < static_cast<int>(ids.size())) Q <<= 1;
+      const int Q = static_cast<int>(padded(ids.size()));
       for (int64_t id : ids) {
         Query& q = *queries[id];
         q.slot = free_slots.back();
@@ -2227,14 +2270,9 @@ struct cpg_server {
         q.node_est = node_estimate(q);
         nodes_held += q.node_est;
       }
-      h.deps.reserve(n + kSfxtPad); h.queue.reserve(n); h.lvlp.reserve(n + 2); h.level.reserve(n);
-      h.big.reserve(n); h.sctl.reserve(1);
-      if (h.g.max_out_degree > kSfxtLdsSort) h.devs_tmp.reserve(m);
       Graph::Multi& M = G.mm;
       G.scheduled = h.sched_ready;
-      M.dv.reserve((G.scheduled ? static_cast<size_t>(h.sched.np) : n) * Q); M.dist.reserve(n * Q); M.succ.reserve(n * Q); M.distf.reserve(n * Q);
       const size_t ns = h.g.sinks.size();
-      M.masks.reserve(std::max<size_t>(1, ns * Q)); M.maxd.reserve(Q); M.ctls.reserve(Q);
       // one flag per sink (in sink order) and subset; padding subsets choose none
       G.hmask.reserve(std::max<size_t>(1, ns * Q));  // kept until the group finishes (asynchronous copy)
       std::memset(G.hmask.p, 0, ns * Q);
@@ -2260,7 +2298,6 @@ struct cpg_server {
       mm.masks = M.masks.p; mm.dv = M.dv.p; mm.dist = M.dist.p; mm.succ = M.succ.p;
       mm.distf = M.distf.p; mm.maxd = M.maxd.p;
       const int lv = sfxt_lift_levels(h.diameter);
-      h.lift.reserve(static_cast<size_t>(lv) * std::max<size_t>(n, 1));
       G.args.clear();
       G.base = a;
       G.lv = lv;
@@ -2345,9 +2382,11 @@ struct cpg_server {
         } else {
           ix = std::make_unique<IndexSet>();
         }
-        ix->vrec.reserve(std::max<size_t>(n, 1));
-        ix->devinfo.reserve(std::max<size_t>(n, 1));
-        ix->devs.reserve(std::max<size_t>(m, 1));
+        room([&]() {
+          ix->vrec.reserve(std::max<size_t>(n, 1));
+          ix->devinfo.reserve(std::max<size_t>(n, 1));
+          ix->devs.reserve(std::max<size_t>(m, 1));
+        });
         SfxtArgs aq = G.base;
         aq.dist = G.mm.dist.p + q * n;
         aq.succ = G.mm.succ.p + q * n;
@@ -2507,7 +2546,7 @@ struct cpg_server {
     const double t0 = now_ms();
     const uint64_t n = node_n;
     const uint64_t nt = mq_compact_tiles(n);
-    tiles.reserve(nt + 1);
+    room([&]() { tiles.reserve(nt + 1); });
     launch_zero_u32(tiles.p + nt, 1, stream);
     MqArgs a = args();
     launch_mq_count_live(a, n, tiles.p, stream);
@@ -2516,8 +2555,10 @@ struct cpg_server {
     d2h(&live, tiles.p + nt, 1, stream);
     CPG_HIP(hipStreamSynchronize(stream));
     Store& d = st[cur ^ 1];
-    d.reserve(std::max<uint64_t>({want, st[cur].cap, 1}));
-    newidx.reserve(std::max<uint64_t>(n, 1));
+    room([&]() {
+      d.reserve(std::max<uint64_t>({want, st[cur].cap, 1}));
+      newidx.reserve(std::max<uint64_t>(n, 1));
+    });
     launch_mq_compact(a, n, d.view(), d.nq.p, tiles.p, newidx.p, live, grid, stream);
     cur ^= 1;
     node_n = live;
@@ -2525,7 +2566,7 @@ struct cpg_server {
     c.node_n = live;
     nonmono_base = stats.nonmonotone;
     h2d(mctl.p, &c, 1, stream);
-    batch.reserve(st[cur].cap);
+    room([&]() { batch.reserve(st[cur].cap); });
     CPG_HIP(hipStreamSynchronize(stream));
     for (int sl : dead_slots) free_slots.push_back(sl);
     dead_slots.clear();
@@ -2651,9 +2692,11 @@ struct cpg_server {
     for (int sl : fin) hs[sl] = 1;
     h2d(sel.p, hs.data(), nslots, stream);
     const uint64_t nn = std::min<uint64_t>(node_n, st[cur].cap);
-    skey[0].reserve(std::max<uint64_t>(1, nn)); skey[1].reserve(std::max<uint64_t>(1, nn));
-    sval[0].reserve(std::max<uint64_t>(1, nn)); sval[1].reserve(std::max<uint64_t>(1, nn));
-    nsel.reserve(1);
+    room([&]() {
+      for (auto& b : skey) b.reserve(std::max<uint64_t>(1, nn));
+      for (auto& b : sval) b.reserve(std::max<uint64_t>(1, nn));
+      nsel.reserve(1);
+    });
     CPG_HIP(hipMemsetAsync(nsel.p, 0, sizeof(unsigned long long), stream));
     CPG_HIP(hipMemsetAsync(per_q.p, 0, sizeof(unsigned long long) * nslots, stream));
     launch_mq_build_keys(args(), sel.p, nn, skey[0].p, sval[0].p, nsel.p, per_q.p, grid, stream);
@@ -2662,11 +2705,13 @@ struct cpg_server {
     d2h(&nl, nsel.p, 1, stream);
     d2h(pq.data(), per_q.p, nslots, stream);
     CPG_HIP(hipStreamSynchronize(stream));
-    ghist.reserve(sort_ghist_len(nl));
+    room([&]() {
+      ghist.reserve(sort_ghist_len(nl));
+      out_cost.reserve(std::max<uint64_t>(1, nl));
+    });
     SortBufs sb{{skey[0].p, skey[1].p}, {sval[0].p, sval[1].p}, ghist.p, nl};
     const int bytes[7] = {0, 1, 2, 3, 4, 5, 6};  // slot < 256: bits 48..55
     const int res = radix_sort_pairs(sb, nl, bytes, 7, stream);
-    out_cost.reserve(std::max<uint64_t>(1, nl));
     launch_mq_gather_costs(sval[res].p, st[cur].cost.p, nl, out_cost.p, stream);
     std::vector<float> all(nl);
     d2h(all.data(), out_cost.p, nl, stream);
@@ -2733,8 +2778,10 @@ struct cpg_server {
     for (int i = nslots - 1; i >= 0; --i)
       if (!slot_reserved[i]) free_slots.push_back(i);
     const uint64_t c = std::min<uint64_t>(2 * st[cur].cap, 0x7fffffffull);
-    st[cur].reserve(c);
-    batch.reserve(c);
+    room([&]() {
+      st[cur].reserve(c);
+      batch.reserve(c);
+    });
     node_n = 0;
     const MqCtl z{};
     nonmono_base = stats.nonmonotone;

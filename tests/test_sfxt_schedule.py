@@ -187,6 +187,30 @@ def test_emulated_full_device_in_a_batch(emu, nth):  # noqa: F811
             assert bits_equal(want[q], b.get_slacks(q, k))
 
 
+@pytest.mark.parametrize("nth", range(0, 102, 6))
+def test_emulated_full_device_in_a_server(emu, nth):  # noqa: F811
+    """An allocation fails while a server with two resident graphs adds the
+    second, starts or serves its queries (six numbers apart: a first query's
+    buffers are reserved in groups): every query is answered."""
+    graphs = [SHAPES["mean3"](), SHAPES["mean6"]()]
+    jobs = []
+    with emu.Server(max_in_flight=4, initial_nodes=4000) as s:
+        s.add_graph(*graphs[0])
+        emu._lib.simt_fail_malloc(nth)
+        try:
+            s.add_graph(*graphs[1])
+            for i in range(3):
+                jobs.append((i % 2, s.submit(i % 2, 4 + i)))
+            while s.step() > 0:
+                pass
+        finally:
+            emu._lib.simt_fail_malloc(-1)
+        for gi, q in jobs:
+            og = pyoracle.OracleGraph.from_edges(*graphs[gi])
+            dist, succ, _, _ = og.sfxt()
+            assert bits_equal(og.topk(dist, succ, 3 + q)[0], s.get_slacks(q, 3 + q))
+
+
 def test_emulated_layout_is_not_tried_again(emu):  # noqa: F811
     """A device with no room for the schedule: the level loop stays until the
     graph is loaded again, without another attempt at each query."""

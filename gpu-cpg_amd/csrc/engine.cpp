@@ -208,6 +208,20 @@ unsigned long long first_target(unsigned long long target) {
   return std::max<unsigned long long>(256, target / 16);
 }
 
+// Whether a multi-query slot's first round is a trial under a bound: where its
+// roots' whole walks hold many edges (chain vertices times the mean
+// out-degree).  Below the line the roots are expanded without a bound at
+// once, as a trial that falls short costs a round.  24 designs alike, 24K edges
+// of root walks each: unbounded 0.75 / 1.29 / 2.4 ms for K = 10 / 1,000 /
+// 10,000, by trials 0.71 / 1.27 / 5.3; 55K: 1.23 / 1.74 / 2.7 and 1.07 / 1.79 /
+// 2.7; 120K: 1.48 / 1.87 / 2.6 and 1.27 / 1.80 / 2.6; 800K: 3.3 / 3.9 / 4.7 and
+// 1.5 / 2.2 / 2.9; 21 edges, K = 10: 0.48 and 1.39 (six served queries 1.3 and
+// 3.4).
+bool worth_trial(int64_t roots, int levels, int64_t n, int64_t m) {
+  return static_cast<double>(roots) * (levels + 1.0) * static_cast<double>(m) >
+         static_cast<double>(1 << 16) * static_cast<double>(std::max<int64_t>(1, n));
+}
+
 // A multi-query slot's first trial bound (see mq.hip).
 void start_trial(MqQuery& m, const std::vector<float>& rc, float cmin, float max_abs_distf) {
   m.trial = 1;
@@ -1717,11 +1731,13 @@ struct cpg_batch {
       m = MqQuery{};
       m.ukey = kKeyInf;
       m.klo = cnt ? float_key(minc) : 0u;
-      if (cnt) {
+      if (cnt && worth_trial(cnt, uh.diameter, designs[q].n, static_cast<int64_t>(designs[q].u.size()))) {
         std::vector<float> rc;
         for (size_t i = 0; i < nr; ++i)
           if (keep[i]) rc.push_back(rcost[q][i]);
         start_trial(m, rc, minc, uh.max_abs_distf);
+      } else {
+        m.all = 1;
       }
       m.shift = window_shift_bins(m.klo, m.ukey, kMqBins);
       m.k = static_cast<unsigned long long>(std::max<int64_t>(0, designs[q].k));
@@ -2110,7 +2126,7 @@ struct cpg_server {
   // Seeds query q, whose SFXT columns and index are in place: its roots
   // (unexpanded) in the graph handle's own node store, from which admission
   // copies them into the shared store, and its first bound: the k-th root's
-  // cost or a trial bound that the shared rounds widen or confirm.
+  // cost, a trial bound that the shared rounds widen or confirm, or none yet.
   void seed_query(Query& q, cpg_handle& h, const SfxtArgs& aq, float max_abs_distf) {
     const int nsrc = static_cast<int>(h.g.srcs.size());
     std::vector<int> sd(nsrc);
@@ -2140,7 +2156,7 @@ struct cpg_server {
     // where the roots' chains are short; otherwise a trial finds a tighter
     // bound.
     const bool short_chains = nkept * (static_cast<int64_t>(h.diameter) + 1) <= (int64_t(1) << 20);
-    bool trial = false;
+    bool trial = false, all = false;
     // the roots in the graph handle's node store, for admission to copy
     auto seed_roots = [&]() {
       const uint64_t cap = std::max<uint64_t>(uint64_t(1) << 16, static_cast<uint64_t>(nkept));
@@ -2164,8 +2180,10 @@ struct cpg_server {
       std::lock_guard<std::mutex> lk(stats_mu);
       stats.root_bounds++;
     } else if (nkept > 0 && q.k > 0) {
-      // roots alone, with a trial bound: the shared rounds find the first one
-      trial = true;
+      // roots alone: the shared rounds find the first bound, from a trial or
+      // from the roots' whole walks
+      trial = worth_trial(nkept, h.diameter, h.g.n, h.g.m);
+      all = !trial;
       seed_roots();
     }
     MqQuery m{};
@@ -2183,6 +2201,7 @@ struct cpg_server {
     m.batch_target = first_target(m.target_max);
     m.done = (nkept == 0 || q.k == 0) ? 1 : 0;
     m.rebuild = 1;
+    m.all = all ? 1 : 0;
     m.vrec = aq.vrec;
     m.devinfo = aq.devinfo;
     m.devs = aq.devs;

@@ -22,8 +22,9 @@
 //      at memory),
 //   5. a fill pass storing its children <= U_q (inclusive: the counted
 //      children at U_q are needed).
-// A query starts with its roots and a trial bound a little above the
-// cheapest (the single query's probe, without its host round trips): a round
+// A query whose roots' walks are long starts with its roots and a trial bound
+// a little above the cheapest (the single query's probe, without its host
+// round trips; the others start unbounded, all roots at once): a round
 // counts the children of the roots under the trial bound, and if the roots
 // and they are fewer than K_q it stores nothing, puts the roots back and
 // widens the bound for the next round.  Without a first bound round 0 walks

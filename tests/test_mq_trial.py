@@ -69,6 +69,73 @@ def check_server(lib, ks, big=False):
         s.close()
 
 
+def tiny():
+    """Fewer paths than any K asked of it; root walks of a few dozen edges."""
+    return layered((2, 4, 4, 4, 4, 2), 2, 60)
+
+
+def check_tiny_rounds(lib):
+    """A query with few paths takes a round per prefix-tree level, not one per
+    trial bound on top."""
+    levels = 6
+    with lib.Server() as s:
+        gid = s.add_graph(*tiny())
+        q = s.submit(gid, 1000)
+        while s.step() > 0:
+            pass
+        assert bits_equal(want_costs(tiny(), 1000), s.get_slacks(q, 1000))
+        assert s.stats()["rounds"] <= levels + 1
+    with lib.Batch() as b:
+        b.add(*tiny(), 1000)
+        b.set_tuning(group=1)
+        b.run()
+        assert bits_equal(want_costs(tiny(), 1000), b.get_slacks(0, 1000))
+        assert b.timings()["rounds"] <= levels + 1
+
+
+def wide(roots):
+    """Root walks of more than 65,536 edges, or of somewhat fewer."""
+    return layered((roots, 15, 15, 9), 9, 61)
+
+
+def check_wide(lib, ks):
+    for roots in (1000, 3000):
+        d = wide(roots)
+        edges = roots * 5 * len(d[1]) / d[0]
+        assert (edges > 65536) == (roots == 3000)
+        with lib.Batch() as b:
+            for k in ks:
+                b.add(*d, k)
+            b.run()
+            for q, k in enumerate(ks):
+                assert bits_equal(want_costs(d, k), b.get_slacks(q, k)), (roots, k)
+        with lib.Server() as s:
+            gid = s.add_graph(*d)
+            qs = [s.submit(gid, k) for k in ks]
+            while s.step() > 0:
+                pass
+            for q, k in zip(qs, ks):
+                assert bits_equal(want_costs(d, k), s.get_slacks(q, k)), (roots, k)
+
+
+def test_emulated_tiny_queries_take_no_trials(emu):  # noqa: F811
+    check_tiny_rounds(emu)
+
+
+def test_emulated_bounds_on_either_side_of_the_line(emu):  # noqa: F811
+    check_wide(emu, [1, 5000])
+
+
+@pytest.mark.gpu
+def test_gpu_tiny_queries_take_no_trials():
+    check_tiny_rounds(cpgamd)
+
+
+@pytest.mark.gpu
+def test_gpu_bounds_on_either_side_of_the_line():
+    check_wide(cpgamd, [1, 7, 300, 5000, 30000, 1000000])
+
+
 def test_emulated_batch_first_bounds(emu):  # noqa: F811
     check_batch(emu, [1, 7, 300])
 

@@ -210,16 +210,17 @@ unsigned long long first_target(unsigned long long target) {
 
 // Whether a multi-query slot's first round is a trial under a bound: where its
 // roots' whole walks hold many edges (chain vertices times the mean
-// out-degree).  Below the line the roots are expanded without a bound at
-// once, as a trial that falls short costs a round.  24 designs alike, 24K edges
-// of root walks each: unbounded 0.75 / 1.29 / 2.4 ms for K = 10 / 1,000 /
-// 10,000, by trials 0.71 / 1.27 / 5.3; 55K: 1.23 / 1.74 / 2.7 and 1.07 / 1.79 /
-// 2.7; 120K: 1.48 / 1.87 / 2.6 and 1.27 / 1.80 / 2.6; 800K: 3.3 / 3.9 / 4.7 and
-// 1.5 / 2.2 / 2.9; 21 edges, K = 10: 0.48 and 1.39 (six served queries 1.3 and
-// 3.4).
-bool worth_trial(int64_t roots, int levels, int64_t n, int64_t m) {
-  return static_cast<double>(roots) * (levels + 1.0) * static_cast<double>(m) >
-         static_cast<double>(1 << 16) * static_cast<double>(std::max<int64_t>(1, n));
+// out-degree) for the paths it asks for, which count up to 32.  Below the line
+// the roots are expanded without a bound at once, as a trial that falls short
+// costs a round.  24 designs alike, unbounded and by trials (ms): 21 edges of
+// root walks each, K = 10: 0.48 and 1.39 (six served queries 1.3 and 3.4); 24K
+// edges, K = 10 / 1,000 / 10,000: 0.75 / 1.29 / 2.4 and 0.71 / 1.27 / 5.3; 55K:
+// 1.22 / 1.82 / 2.7 and 1.09 / 1.89 / 2.8; 120K: 1.47 / 1.88 / 2.6 and 1.26 /
+// 1.80 / 2.5; 800K: 3.2 / 3.9 / 4.8 and 1.5 / 2.2 / 2.8.
+bool worth_trial(int64_t roots, int levels, int64_t n, int64_t m, int64_t k) {
+  const double edges = static_cast<double>(roots) * (levels + 1.0) * static_cast<double>(m) /
+                       static_cast<double>(std::max<int64_t>(1, n));
+  return edges > 2048.0 * static_cast<double>(std::min<int64_t>(k, 32));
 }
 
 // A multi-query slot's first trial bound (see mq.hip).
@@ -1731,7 +1732,8 @@ struct cpg_batch {
       m = MqQuery{};
       m.ukey = kKeyInf;
       m.klo = cnt ? float_key(minc) : 0u;
-      if (cnt && worth_trial(cnt, uh.diameter, designs[q].n, static_cast<int64_t>(designs[q].u.size()))) {
+      if (cnt && worth_trial(cnt, uh.diameter, designs[q].n, static_cast<int64_t>(designs[q].u.size()),
+                             designs[q].k)) {
         std::vector<float> rc;
         for (size_t i = 0; i < nr; ++i)
           if (keep[i]) rc.push_back(rcost[q][i]);
@@ -2182,7 +2184,7 @@ struct cpg_server {
     } else if (nkept > 0 && q.k > 0) {
       // roots alone: the shared rounds find the first bound, from a trial or
       // from the roots' whole walks
-      trial = worth_trial(nkept, h.diameter, h.g.n, h.g.m);
+      trial = worth_trial(nkept, h.diameter, h.g.n, h.g.m, q.k);
       all = !trial;
       seed_roots();
     }

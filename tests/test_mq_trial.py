@@ -94,7 +94,8 @@ def check_tiny_rounds(lib):
 
 
 def wide(roots):
-    """Root walks of more than 65,536 edges, or of somewhat fewer."""
+    """Root walks of more than 65,536 edges, or of somewhat fewer (but many
+    for one path)."""
     return layered((roots, 15, 15, 9), 9, 61)
 
 

@@ -24,6 +24,11 @@ struct SfxtCtl {
   // edge-parallel level loop: one counter per level parity, arrivals << 40 |
   // vertices pushed (both running totals, never reset)
   unsigned long long lvl_bar[2];
+  // edge-parallel level loop that left before the last level (SfxtArgs::leave):
+  // the level to go on with (0: the loop is done) and its queue entries
+  int cont_d;
+  unsigned cont_lb, cont_le;
+  int pad2;
 };
 
 struct SfxtArgs {
@@ -61,6 +66,13 @@ struct SfxtArgs {
   // (the XCD count) every working block lands on one XCD under round-robin
   // dispatch
   int place_stride;
+  // Edge-parallel level loop in parts: leave != 0 ends a launch once two levels
+  // in a row (level 0 aside) hold more than leave vertices together, or fewer
+  // than -leave; a launch that goes on with level d0 > 0, queue entries [lb0,
+  // le0), has its barrier counters cleared before it.
+  int leave;
+  int d0;
+  unsigned lb0, le0;
   int64_t m;  // edges (the fence-free loop picks its records per step by m / n)
   // 1: succ[] is not set yet; the deviation pass finds each successor among
   // the fanouts (largest original id at the smallest candidate)

@@ -460,7 +460,10 @@ __device__ __forceinline__ int queue_entry(const SfxtArgs& a, unsigned i) {
 // last record in its final step issue no-ops (on the pad slots).  Records of
 // one vertex sit in consecutive lanes, so their loads coalesce.  Each level
 // ends at the counter barrier.
-template <int kS>
+//
+// kParts: the launch may go on where another left and leave before the last
+// level (SfxtArgs::leave, d0).
+template <int kS, bool kParts = false>
 __device__ void levels_edges_loop(const SfxtArgs& a) {
   __shared__ int s_q[kLdsQueue];
   __shared__ int s_qn;
@@ -476,12 +479,19 @@ __device__ void levels_edges_loop(const SfxtArgs& a) {
   __syncthreads();
 
   unsigned lb = 0, le = static_cast<unsigned>(a.nsinks);
-  int d = 0;
+  int d = 0, bar_d = 0;  // the level, and its number in this launch's barrier
+  bool left = false;
+  if (kParts && a.d0 > 0) {
+    d = a.d0;
+    lb = a.lb0;
+    le = a.le0;
+  }
+  const int leave = kParts ? __builtin_amdgcn_readfirstlane(a.leave) : 0;  // kept in a register
   LevelCounts lc;
   auto push = [&](int x) {
     const int p = atomicAdd(&s_qn, 1);
     if (p < kLdsQueue) s_q[p] = x;
-    else st_dev32(a.queue + counter_reserve(ctl, d, le, lc), x);  // past the LDS queue
+    else st_dev32(a.queue + counter_reserve(ctl, kParts ? bar_d : d, le, lc), x);  // past the LDS queue
   };
 
   float local_max = 0.0f;
@@ -564,25 +574,40 @@ __device__ void levels_edges_loop(const SfxtArgs& a) {
       }
     }
     unsigned ne = 0;
-    if (!counter_barrier(ctl, a.queue, s_q, &s_qn, nblocks, d, le, lc, &ne)) return;
+    if (!counter_barrier(ctl, a.queue, s_q, &s_qn, nblocks, kParts ? bar_d : d, le, lc, &ne)) return;
     if (ne == le) break;
+    if (kParts) {  // the same decision in every block: d, lb and ne are the same
+      // the level just settled, and the next
+      const int two = static_cast<int>(ne - lb);
+      left = d > 0 && (leave > 0 ? two > leave : two < -leave);
+      ++bar_d;
+    }
     lb = le;
     le = ne;
     ++d;
+    if (kParts && left) break;
   }
   const float m = wave_max(local_max);
   if (__lane_id() == 0) atomicMax(&ctl->max_abs_distf_bits, __float_as_uint(m));
   if (gtid == 0) {
-    a.lvlp[d + 1] = static_cast<int>(le);
-    ctl->num_levels = le > 0 ? d + 1 : 0;
-    ctl->levelized = le;
+    if (kParts && left) {
+      ctl->cont_d = d;
+      ctl->cont_lb = lb;
+      ctl->cont_le = le;
+    } else {
+      a.lvlp[d + 1] = static_cast<int>(le);
+      ctl->num_levels = le > 0 ? d + 1 : 0;
+      ctl->levelized = le;
+    }
   }
 }
 
 // One list position per lane step where the blocks share an XCD, two over all
-// XCDs (launch_sfxt_levels_edges).
+// XCDs (launch_sfxt_levels_edges); each also for a loop in parts.
 __global__ void __launch_bounds__(kSfxtBlock) sfxt_levels_e1_kernel(SfxtArgs a) { levels_edges_loop<1>(a); }
 __global__ void __launch_bounds__(kSfxtBlock) sfxt_levels_e2_kernel(SfxtArgs a) { levels_edges_loop<2>(a); }
+__global__ void __launch_bounds__(kSfxtBlock) sfxt_levels_e1p_kernel(SfxtArgs a) { levels_edges_loop<1, true>(a); }
+__global__ void __launch_bounds__(kSfxtBlock) sfxt_levels_e2p_kernel(SfxtArgs a) { levels_edges_loop<2, true>(a); }
 
 // ---------------------------------------------------------------------------
 // Dataflow loop: the same levelize / relax / successor results as the level
@@ -2101,7 +2126,9 @@ int launch_sfxt_levels_edges(const SfxtArgs& args, int blocks, hipStream_t strea
   // 1 / 2 / 3 / 8 positions take 1.52 / 1.55 / 1.67 / 2.65 ms on a 120K-vertex
   // graph of 346 levels (one XCD), 2.23 / 2.09 / 2.19 / 3.09 on 1.5M vertices of
   // 300 levels (all XCDs)
-  auto k = args.place_stride > 1 ? sfxt_levels_e1_kernel : sfxt_levels_e2_kernel;
+  const bool parts = args.leave != 0 || args.d0 > 0;
+  auto k = args.place_stride > 1 ? (parts ? sfxt_levels_e1p_kernel : sfxt_levels_e1_kernel)
+                                 : (parts ? sfxt_levels_e2p_kernel : sfxt_levels_e2_kernel);
   // place_stride launch blocks per working block (the others return at once)
   const int stride = std::max(1, args.place_stride);
   const int working = loop_grid(blocks, resident_blocks(k, kSfxtBlock) / stride);

@@ -166,6 +166,7 @@ inline int __builtin_amdgcn_update_dpp(int, int v, int ctrl, int, int, bool) {
   return __shfl(v, from);
 }
 inline int __builtin_amdgcn_readlane(int v, int src) { return __shfl(v, src); }
+inline int __builtin_amdgcn_readfirstlane(int v) { return __shfl(v, 0); }  // with every lane of the wave live
 inline void __builtin_amdgcn_wave_barrier() { (void)simt::wave_sync(0); }
 
 template <class T>

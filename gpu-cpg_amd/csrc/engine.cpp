@@ -48,6 +48,12 @@ double now_ms() {
       .count();
 }
 
+// Bits of a BVSS triple's sort key (a test build sets few, to split a call's
+// frontiers into parts).
+#ifndef CPG_BVSS_KEY_BITS
+#define CPG_BVSS_KEY_BITS 64
+#endif
+
 // The device has no memory left for a buffer.
 struct DeviceFull : std::runtime_error {
   using std::runtime_error::runtime_error;
@@ -1437,7 +1443,7 @@ struct cpg_handle {
     // frontiers beyond 2^(64 - 2 vbits) are taken in calls of their own.
     int vbits = 1;
     while ((1ll << vbits) < g.n) ++vbits;
-    const int fbits = 64 - 2 * vbits;
+    const int fbits = CPG_BVSS_KEY_BITS - 2 * vbits;
     if (fbits < 31 && nfront > (1 << fbits)) return bvss_in_parts(nfront, 1 << fbits, fptr, fsrc, mode, dense_min, of, ou, ov, cap);
     const size_t room = std::max<int64_t>(1, cap);
     skey[0].reserve(room); skey[1].reserve(room);

@@ -5,12 +5,14 @@ set definition (u in the frontier, an edge u -> v with v != succ[u]), in
 all three modes, from no triple to many per wave step, over frontier counts
 around a tile's 16, with exact, short and zero capacity."""
 import ctypes
+import os
+import subprocess
 
 import numpy as np
 import pytest
 
 import cpgamd
-from test_simt_emulator import emu  # noqa: F401  (fixture)
+from test_simt_emulator import SIMT, emu  # noqa: F401  (fixture)
 
 
 def bipartite(a, b, fan, seed):
@@ -62,3 +64,38 @@ def test_emulated_triples_sorted(emu, case):  # noqa: F811
 @pytest.mark.parametrize("case", CASES + [(4096, 3000, 25, 8, 3000)])
 def test_gpu_triples_sorted(case):
     check(cpgamd, *case)
+
+
+@pytest.fixture
+def parts(emu):  # noqa: F811
+    """The emulator with keys of 18 bits, in place of the other one."""
+    subprocess.run(["make", "-s", "-C", SIMT, "libcpgamd_simt_parts.so"], check=True)
+    saved, cpgamd._lib = cpgamd._lib, cpgamd.load_library(os.path.join(SIMT, "libcpgamd_simt_parts.so"))
+    yield cpgamd
+    cpgamd._lib = saved
+
+
+@pytest.mark.parametrize("case", [(64, 70, 60, 5, 400), (130, 20, 3, 17, 40), (65, 9, 1, 33, 10), (30, 100, 2, 8, 6)])
+def test_emulated_triples_in_parts(parts, case):
+    """More frontiers than one key holds."""
+    check(parts, *case)
+
+
+def test_emulated_parts_and_capacity(parts):
+    """Parts that fill the caller's arrays, overrun them, or find nothing."""
+    n, u, v, w = bipartite(80, 60, 3, 5)
+    fronts = [np.arange(f, 80, 17, dtype=np.int32) if f % 3 else np.zeros(0, np.int32) for f in range(14)]
+    with parts.CpGen() as g:
+        g.load_edges(n, u, v, w)
+        total, full = discover(g, fronts, 0, 4096)
+        assert total > 60
+        for cap in sorted({0, 1, 7, total // 2, total // 2 + 1, total - 1, total, total + 2}):
+            got, out = discover(g, fronts, 0, cap)
+            assert got == (total if cap >= total else -total - 1000)
+            if cap >= total:
+                for a, b in zip(full, out):
+                    np.testing.assert_array_equal(a[:total], b[:total])
+                    assert (b[total:] == -7).all()
+        one = [x.ctypes.data_as(ctypes.POINTER(ctypes.c_int)) for x in
+               (np.array([0, 5] + [10] * 8, np.int32), np.arange(10, dtype=np.int32))]
+        assert g.L.cpg_bvss_discover(g.h, 9, one[0], one[1], 0, 4, None, None, None, 4096) > 0  # counts only

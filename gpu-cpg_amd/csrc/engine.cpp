@@ -1935,7 +1935,6 @@ struct cpg_server {
     int slot = -1;
     int state = 0;              // 0 queued, 1 in flight, 2 done
     std::unique_ptr<IndexSet> index;
-    std::vector<int> roots;     // kept roots (vertex ids, ascending)
     uint64_t seed_n = 0;        // roots left in the graph handle's store until admission
     int64_t node_est = 0;       // node-store estimate held while admitted (0 = not held)
     MqQuery init{};             // slot state at admission
@@ -2751,15 +2750,15 @@ struct cpg_server {
       const uint64_t take = std::min<uint64_t>(pq[sl], static_cast<uint64_t>(q.k));
       {
         Graph& Gq = *graphs[q.graph];
-        const double used = static_cast<double>(hq[sl].stored + q.seed_n + q.roots.size());
+        const double used = static_cast<double>(hq[sl].stored + q.seed_n);
         const double r = used / static_cast<double>(std::max<int64_t>(q.k, 1));
         Gq.nodes_per_k = 0.5 * Gq.nodes_per_k + 0.5 * std::max(1.0, r);
         dead_nodes += static_cast<uint64_t>(used);
         if (trace_on())
-          std::fprintf(stderr, "served t %.2f query %lld graph %d k %lld stored %llu seed %llu roots %zu ratio %.1f\n",
+          std::fprintf(stderr, "served t %.2f query %lld graph %d k %lld stored %llu roots %llu ratio %.1f\n",
                        now_ms(), static_cast<long long>(q.id), q.graph, static_cast<long long>(q.k),
                        static_cast<unsigned long long>(hq[sl].stored),
-                       static_cast<unsigned long long>(q.seed_n), q.roots.size(), r);
+                       static_cast<unsigned long long>(q.seed_n), r);
       }
       q.result.assign(all.begin() + off, all.begin() + off + take);
       off += pq[sl];

@@ -41,8 +41,6 @@ constexpr int kBlock = 256;
 constexpr int kSelBlock = 1024;
 constexpr int kHistBlock = 1024;
 
-__device__ inline unsigned long long ld_u64(const unsigned long long* p) { return *p; }
-
 // Block-wide search for the first bin at which the running sum of h (words
 // other blocks of the launch wrote) reaches target (1-based count).  Returns
 // kHistBins if the total is smaller; *total receives the sum.  Must be called

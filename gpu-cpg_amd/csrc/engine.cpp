@@ -25,6 +25,7 @@
 #include "common.hpp"
 #include "graph.hpp"
 #include "kernels.hpp"
+#include "slots.hpp"
 
 namespace cpg {
 void launch_gather_int(const int* src, const int* idx, int n, int* out, hipStream_t s);
@@ -298,6 +299,7 @@ struct cpg_handle {
   bool sched_ready = false;
   bool order_ready = false;    // queue, level and lvlp hold a finished level loop of the resident graph
   bool order_pending = false;  // the queued SFXT will leave them so
+  LoopLease loop_lease;        // of the SFXT's loop, from its launch to the stream's next synchronisation
   bool budgeted = false;       // the query has a device-byte budget: no schedule
   bool schedule_off = false;   // the device had no room beside one: the level loop until the graph changes
   bool sfxt_valid = false;
@@ -559,8 +561,8 @@ struct cpg_handle {
   // a CU's scattered-load rate bounds wide levels: on the 1.5M-vertex DAG 0.87
   // ms with 128 blocks (0.74 with 256), 1.6 with 32; narrow levels measure the
   // same from 16 up (50K-vertex DAG 0.14 ms).  128 blocks are a sixteenth of
-  // what the device holds, so the loops of 16 handles on streams of their own
-  // are resident together; a wave may wait for any other wave of its loop.
+  // what the device holds; a wave may wait for any other wave of its loop, so
+  // beside many other loops it gets fewer (LoopSlots).
   // Keeping the blocks on one XCD was slower on every graph wider than that
   // one (1.6 ms and 0.74; 3.4 and 1.9 at 1.1M vertices).
   int sched_blocks(int lanes) const {
@@ -782,12 +784,18 @@ struct cpg_handle {
       else launch_sfxt_init(a, stream);
       if (kernel_timing) CPG_HIP(hipEventRecord(ev_levels.a, stream));
       a.find_succ = scheduled ? 1 : 0;
-      timing.sfxt_blocks = scheduled     ? launch_sfxt_scheduled(a, sched, sched_blocks(sched.lanes), stream)
-                           : dataflow    ? launch_sfxt_dataflow(a, df_grid, stream)
-                           : method == 3 ? launch_sfxt_local(a, level_loop_blocks(), stream)
-                           : method == 4 ? launch_sfxt_levels_nf(a, level_loop_blocks(), stream)
-                           : method == 5 ? launch_sfxt_levels_edges(a, edge_loop_blocks(), stream)
-                                         : launch_sfxt_levels(a, level_loop_blocks(), stream);
+      // the dataflow loop's blocks wait for no others; loops 1, 3 and 4 keep
+      // fewer blocks resident than the slots are counted for
+      int blocks = df_grid;
+      if (scheduled) blocks = loop_lease.take(sched_blocks(sched.lanes));
+      else if (method == 5) blocks = loop_lease.take(edge_loop_blocks(), a.place_stride);
+      else if (!dataflow) blocks = loop_lease.take(level_loop_blocks(), 2);
+      timing.sfxt_blocks = scheduled     ? launch_sfxt_scheduled(a, sched, blocks, stream)
+                           : dataflow    ? launch_sfxt_dataflow(a, blocks, stream)
+                           : method == 3 ? launch_sfxt_local(a, blocks, stream)
+                           : method == 4 ? launch_sfxt_levels_nf(a, blocks, stream)
+                           : method == 5 ? launch_sfxt_levels_edges(a, blocks, stream)
+                                         : launch_sfxt_levels(a, blocks, stream);
       if (kernel_timing) CPG_HIP(hipEventRecord(ev_levels.b, stream));
       if (relabelled && !scheduled) launch_sfxt_succ_relabel(succ.p, perm_d.p, g.n, stream);
       // The lifting table needs the level count.  Levels depend on the
@@ -813,6 +821,7 @@ struct cpg_handle {
   }
 
   void sfxt_finish(const SfxtCtl& c, bool count_cache, const uint8_t* mask) {
+    loop_lease.release();
     if (kernel_timing && g.n > 0) {
       timing.sfxt_kernel_ms = ev_sfxt.ms();
       timing.sfxt_levels_ms = ev_levels.ms();
@@ -2013,6 +2022,8 @@ struct cpg_server {
   std::mutex stats_mu;  // statistics the seedings of several graphs update
   std::mutex room_mu;   // likewise the giving back of schedules
   int parts_cap = 1;              // blocks one partitioned level-loop launch keeps resident
+  LoopLease loop_lease;           // of the groups' loops, one launch after another on sstream,
+  int loop_blocks = 0;            // until no group is in progress
 
   uint64_t first_cap = uint64_t(1) << 24;
 
@@ -2042,6 +2053,13 @@ struct cpg_server {
       for (auto& G : graphs) G->h->give_back_schedule();
     }
     f();
+  }
+
+  // Blocks for the next of sstream's loop launches, of up to `total` (at least
+  // `least`): the lease covers the largest launch that may be in flight.
+  int lease_blocks(int total, int least) {
+    loop_blocks = loop_lease.take(std::max(total, loop_blocks), 1, least);
+    return std::min(total, loop_blocks);
   }
 
   void init() {
@@ -2355,6 +2373,12 @@ struct cpg_server {
       int total = 0;
       for (int i = 0; i < sparts.n; ++i) {
         sparts.p[i].nb = std::max(1, std::min(sparts.p[i].nb, parts_cap / sparts.n));
+        total += sparts.p[i].nb;
+      }
+      const int got = lease_blocks(total, sparts.n), want = total;
+      total = 0;
+      for (int i = 0; i < sparts.n; ++i) {
+        if (got < want) sparts.p[i].nb = std::max(1, sparts.p[i].nb * got / want);
         sparts.p[i].b0 = total;
         total += sparts.p[i].nb;
       }
@@ -2364,9 +2388,9 @@ struct cpg_server {
     if (parts.n > 0) {
       // fit every partition into one resident launch (admission forms at
       // most parts_cap groups, so one block each always fits)
-      const int cap = parts_cap;
       int total = 0;
       for (int i = 0; i < parts.n; ++i) total += parts.p[i].nb;
+      const int cap = lease_blocks(std::min(total, parts_cap), parts.n);
       if (total > cap) {
         for (int i = 0; i < parts.n; ++i)
           parts.p[i].nb = std::max(1, static_cast<int>(static_cast<int64_t>(parts.p[i].nb) * cap / total));
@@ -2682,6 +2706,10 @@ struct cpg_server {
       }
       stats.group_wait_ms += now_ms() - tw;
       finish_groups(r);
+    }
+    if (!any_busy()) {
+      loop_lease.release();
+      loop_blocks = 0;
     }
   }
 
@@ -3457,5 +3485,15 @@ int cpg_write_text(const cpg_edge_list* el, const char* path) {
     return 0;
   });
 }
+
+#ifdef CPG_TEST_HOOKS
+// Takes loop slots, as a loop in flight elsewhere would hold (test builds; 0
+// gives them back).
+void cpg_test_hold_slots(int slots) {
+  static LoopLease held;
+  if (slots > 0) held.take(slots);
+  else held.release();
+}
+#endif
 
 }  // extern "C"

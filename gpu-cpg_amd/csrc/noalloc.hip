@@ -16,6 +16,7 @@
 
 #include "common.hpp"
 #include "kernels.hpp"
+#include "slots.hpp"
 
 namespace cpg {
 
@@ -120,7 +121,8 @@ int sfxt_noalloc(int n, const int* oadjp, const int* iadjp, const int2* iedge, c
   for (int changes = 0;; ++changes) {
     a.place_stride = wide ? 1 : kNarrowStride;
     a.leave = n < kNoallocParts || changes >= kNoallocChanges ? 0 : wide ? -kNarrowLevels : kWideLevels;
-    launch_sfxt_levels_edges(a, wide ? kWideBlocks : kNarrowBlocks, stream);
+    LoopLease lease;
+    launch_sfxt_levels_edges(a, lease.take(wide ? kWideBlocks : kNarrowBlocks, a.place_stride), stream);
     CPG_HIP(hipMemcpyAsync(&c, a.ctl, sizeof(SfxtCtl), hipMemcpyDeviceToHost, stream));
     CPG_HIP(hipStreamSynchronize(stream));
     if (c.err) throw std::runtime_error("SFXT grid barrier did not complete");

@@ -37,9 +37,12 @@
 // u}; a greedy descent from the top level finds the first chain vertex
 // whose smallest delta is below u's with one dependent load per level.
 #include <algorithm>
+#include <memory>
+#include <mutex>
 
 #include "common.hpp"
 #include "kernels.hpp"
+#include "slots.hpp"
 
 namespace cpg {
 
@@ -2281,6 +2284,22 @@ void launch_sfxt_init_multi(const SfxtArgs& args, const SfxtMulti& m, hipStream_
 int sfxt_parts_capacity() {
   return std::min(resident_blocks(sfxt_levels_parts_kernel, kSfxtBlock),
                   resident_blocks(sfxt_sched_multi_kernel, kSchedBlock));
+}
+
+LoopSlots& LoopSlots::current() {
+  constexpr int kMaxDevices = 64;
+  static std::mutex mu;
+  static std::unique_ptr<LoopSlots> all[kMaxDevices];
+  int dev = 0;
+  CPG_HIP(hipGetDevice(&dev));
+  if (dev < 0 || dev >= kMaxDevices) throw std::runtime_error("device index out of range");
+  std::lock_guard<std::mutex> lk(mu);
+  if (!all[dev]) {
+    auto s = std::make_unique<LoopSlots>();
+    s->set_capacity(2 * sfxt_parts_capacity());  // which is half of what the device holds
+    all[dev] = std::move(s);
+  }
+  return *all[dev];
 }
 
 void launch_sfxt_levels_parts(const SfxtParts& parts, int total_blocks, hipStream_t stream) {

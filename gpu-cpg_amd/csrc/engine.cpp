@@ -1102,6 +1102,12 @@ struct cpg_handle {
       wa.max_abs_distf = max_abs_distf; wa.max_abs_wgt = g.max_abs_wgt;
       wa.collect_stats = o.collect_stats;
       wa.step_limit = step_limit();
+      // Lanes per parent in the walks (see launch_walk).  The line lies between
+      // the graphs first measured, at mean out-degrees 2.7 and 5.3; what decides
+      // is the parents a round has, more than the mean.  With 2 / 4 lanes at K =
+      // 1M, 1.5M vertices: mean 2.1 3.55 / 3.75 ms, 2.7 3.57 / 3.76, 3.5 3.65 /
+      // 3.74, 4.1 3.81 / 3.95; at K = 20K 2.04 / 2.00, 1.99 / 1.95, 1.95 / 1.91,
+      // 2.26 / 2.23; 200K vertices, K = 1M: mean 2.1 5.28 / 5.01, 3.1 4.32 / 4.11.
       wa.lanes = g.m < 3 * static_cast<int64_t>(g.n) ? 2 : 4;
       const int64_t nkept = nroots - dropped;
       // Without a probe the first round walks every root's whole chain and all
@@ -1150,7 +1156,9 @@ struct cpg_handle {
       // 900K a first round of 131K parents walked 51M children (the query 473
       // ms, through a store overflow; 4.8 ms growing); on 189K / 14.5 49.8 ms
       // and 4.4; on 1.5M / 2.7, K = 1M, 3.99 and 3.82.  Up to one batch the
-      // rounds start whole: there the loose round is bounded by k parents.
+      // rounds start whole, so a loose first round can still fill the store and
+      // start the query over in a larger one: growing there gave 2% (400K
+      // vertices, K = 100K, 2.54 -> 2.46 ms) and changes which designs retry.
       const bool grow = o.batch == 0 && static_cast<uint64_t>(k) > batch_target;
       auto round_batch = [&](int round) {
         return !grow || round >= 16 ? batch_target
@@ -2263,7 +2271,7 @@ struct cpg_server {
 
   // Starts admission groups on several idle graphs (at most kMaxParts):
   // reserves their queries' slots and budget, then on the server's SFXT
-  // stream one cooperative launch runs every group's multi-subset level
+  // stream one launch, all of it resident, runs every group's multi-subset
   // loop, each graph on its own partition of blocks with its own barrier
   // (the launch takes as long as the slowest graph, not the sum).  Each
   // graph's stream then builds its queries' deviation indexes after the

@@ -133,7 +133,7 @@ struct SfxtParts {
 int sfxt_parts_capacity();
 // parts.p[0..n) cover the blocks [0, total_blocks) in ascending b0.
 void launch_sfxt_levels_parts(const SfxtParts& parts, int total_blocks, hipStream_t stream);
-// Per-vertex init, then the cooperative level loop (returns the grid used).
+// Per-vertex init, then the level loop, all of it resident (returns the grid used).
 void launch_sfxt_init(const SfxtArgs& args, hipStream_t stream);
 int launch_sfxt_levels(const SfxtArgs& args, int blocks, hipStream_t stream);
 // The same loop without cache fences (device-scope queue and best[] access);

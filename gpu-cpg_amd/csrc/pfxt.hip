@@ -51,7 +51,9 @@ __device__ uint32_t find_crossing(const unsigned* h, unsigned long long target,
   __shared__ unsigned s_wave[kW];
   __shared__ unsigned s_bin;
   const int t = threadIdx.x, lane = __lane_id(), wave = t >> 6;
-  unsigned v[kPer], mine = 0;  // a node store holds fewer than 2^31 paths
+  // 32-bit sums: a node store holds fewer than 2^31 paths (ensure_pfxt_buffers
+  // refuses more), and a count pass adds at most as many keys (ckeys_cap)
+  unsigned v[kPer], mine = 0;
 #pragma unroll
   for (int i = 0; i < kPer; ++i) {
     v[i] = dev_load(h + t * kPer + i);

@@ -1164,8 +1164,10 @@ __global__ void __launch_bounds__(kLocBlock) sfxt_local_kernel(SfxtArgs a) {
 // (SfxtSched), and later runs settle the vertices in that order pull-style,
 // as relax_bu_step (gpucpg/gpucpg.cu:1167-1187) reads the fanouts: dist =
 // min over reachable fanouts of dist[w] + (int)(w_e * 10000.0f), level = 1 +
-// max level[w] (the peel depth of bfs_td_step_privatized, :2215-2283).  Only
-// the order is kept; both values are computed from the edges on every run.
+// max level[w] (the peel depth of bfs_td_step_privatized, :2215-2283).  The
+// schedule keeps the vertices' positions and, in place of the CSR, the edges
+// as {head's position, int-scaled weight}; both values are computed from them
+// on every run.
 //
 // There is no barrier, queue or atomic.  Each position has a write-once
 // 64-bit state word, level << 32 | dist (all ones until settled), stored and

@@ -50,7 +50,9 @@ typedef struct {
   int64_t mem_budget_bytes; /* device bytes a query may hold (0 = no limit): the
                                prefix-tree node store and the final sort get
                                what the graph and its SFXT leave; a query whose
-                               store would have to grow past it fails          */
+                               store would have to grow past it fails.  A
+                               budgeted query lays out no level-order schedule
+                               and gives an existing one back (see cpg_sfxt)   */
   const uint8_t* endpoint_mask; /* optional n-byte sink subset (NULL = all sinks) */
   int collect_stats;        /* 1: count hops / deviations / emitted children  */
   int kernel_timing;        /* 1: time the SFXT and walk kernels with HIP events
@@ -177,6 +179,10 @@ int64_t cpg_step_times(cpg_handle* h, double* ms, int64_t* paths, int64_t cap);
  * time.  The BVSS entry points need 0. */
 int cpg_set_csr_reorder(cpg_handle* h, int method);
 double cpg_reorder_ms(cpg_handle* h);
+/* The SFXT alone.  A handle's memory grows on a graph's second SFXT, which
+ * lays out the graph's level-order schedule (8 bytes an edge, about 8 to 20 a
+ * vertex) that later ones run in.  It goes with the graph, and is given back
+ * to a query with mem_budget_bytes and where the device has no room left. */
 int cpg_sfxt(cpg_handle* h);
 /* No counterpart in the reference.  For callers that cannot allocate device
  * memory (serving loops or harnesses that forbid hipMalloc): the SFXT level
@@ -281,7 +287,8 @@ typedef struct {
   double probe_ms;           /* 0 (first bounds are found in the rounds)       */
   double round_ms, extract_ms, compact_ms;  /* host wall time                */
 } cpg_server_stats;
-/* budget_bytes: device bytes for in-flight indexes (0 = 64 GiB);
+/* budget_bytes: device bytes for in-flight indexes (0 = 64 GiB; the resident
+ * graphs, their level-order schedules and the node store are not counted);
  * max_in_flight: query slots, at most 256 (0 = 64); initial_nodes: first
  * capacity of the shared node store (0 = 2^24; it grows as needed). */
 cpg_server* cpg_server_create(int64_t budget_bytes, int max_in_flight, int64_t initial_nodes);

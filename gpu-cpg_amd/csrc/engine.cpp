@@ -1484,6 +1484,19 @@ struct cpg_handle {
     if (c.mismatch) throw std::runtime_error("BVSS MFMA count disagrees with the decoded words");
     const uint64_t cnt = c.count;
     if (cnt > static_cast<uint64_t>(cap)) return -static_cast<int64_t>(cnt) - 1000;
+    if (cnt <= kBvssHostSort) {
+      std::vector<uint64_t> key(cnt);
+      d2h(key.data(), skey[0].p, cnt, stream);
+      CPG_HIP(hipStreamSynchronize(stream));
+      std::sort(key.begin(), key.end());
+      const uint64_t id = (uint64_t(1) << vbits) - 1;
+      for (uint64_t i = 0; i < cnt; ++i) {
+        if (of) of[i] = static_cast<int>(key[i] >> (2 * vbits));
+        if (ou) ou[i] = static_cast<int>((key[i] >> vbits) & id);
+        if (ov) ov[i] = static_cast<int>(key[i] & id);
+      }
+      return static_cast<int64_t>(cnt);
+    }
     // ordered by (f, u, v): the keys' used bytes
     int used = 2 * vbits;
     while (used < 64 && (1ll << (used - 2 * vbits)) < nfront) ++used;
@@ -1501,6 +1514,12 @@ struct cpg_handle {
     CPG_HIP(hipStreamSynchronize(stream));
     return static_cast<int64_t>(cnt);
   }
+
+  // Triples up to which the host sorts their keys, after one copy in place of
+  // two launches and three copies.  A call on the host / on the device: 34
+  // triples 0.112 / 0.146 ms, 624 0.126 / 0.144, 1,265 0.142 / 0.152, 3,076 0.187
+  // / 0.165, 12,300 0.420 / 0.239.
+  static constexpr uint64_t kBvssHostSort = 1536;
 
   // Discovery for more frontiers than one key holds: parts of `per`
   // frontiers, each part's triples after the last's (f ascends over parts).

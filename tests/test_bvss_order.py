@@ -66,6 +66,31 @@ def test_gpu_triples_sorted(case):
     check(cpgamd, *case)
 
 
+def check_sort_line(lib):
+    """Numbers of triples around the line between the host's sort and the
+    device's (each source leaves all its edges but one)."""
+    for a in (511, 512, 513):
+        n, u, v, w = bipartite(a, 40, 4, a)
+        with lib.CpGen() as g:
+            g.load_edges(n, u, v, w)
+            g.bvss_build()
+            dev = v != g.sfxt()[1][u]
+            got, out = discover(g, [np.arange(a)], 0, 4 * a)
+            assert got == 3 * a == dev.sum()
+            want = sorted(zip(u[dev].tolist(), v[dev].tolist()))
+            assert list(zip(out[1][:got].tolist(), out[2][:got].tolist())) == want
+            assert not out[0][:got].any()
+
+
+def test_emulated_triples_at_the_sort_line(emu):  # noqa: F811
+    check_sort_line(emu)
+
+
+@pytest.mark.gpu
+def test_gpu_triples_at_the_sort_line():
+    check_sort_line(cpgamd)
+
+
 @pytest.fixture
 def parts(emu):  # noqa: F811
     """The emulator with keys of 18 bits, in place of the other one."""

@@ -8,6 +8,7 @@ import pytest
 
 import cpgamd
 import pyoracle
+from test_sfxt_schedule import layered
 from test_simt_emulator import bits_equal, emu  # noqa: F401  (fixture)
 from test_walk_lanes import rows
 
@@ -55,3 +56,11 @@ def test_gpu_histogram_parts(probe):
     """Stores of one histogram block (8,192 paths) and just past it, of a few,
     and of more than there are partials for."""
     check(cpgamd, rows(6, 30, 300, 11, False), [2, 2000, 4000, 8000, 16000, 33000, 700000], bound_probe=probe)
+
+
+@pytest.mark.gpu
+def test_gpu_shallow_graph_takes_whole_batches():
+    """Few children per parent: a round per level of the prefix tree, none of
+    them small."""
+    graph = layered([4000, 3000, 3000, 2000], 5, 90)
+    assert check(cpgamd, graph, [131073, 200000, 300000])["rounds"] <= 4
